@@ -1036,12 +1036,14 @@ void launch_pack_span(const PackArgs& pa, hipStream_t stream, hipEvent_t ea, hip
 // the gpu ids and, `split` entries later, the cpu ids (device memory), and
 // `host` is null.  `grid_cap` is compute units x occupancy of the kernel the
 // launch takes; staging launches that take the whole-group variant use
-// `whole_grid_cap` instead when it is given.
+// `whole_grid_cap` instead when it is given.  `done` (zero-copy launches
+// with profiling off): an event the launch completes, carried by the kernel's
+// own packet instead of a marker behind it.
 template <bool kH2D, bool kIota>
 int launch_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int64_t cks, int64_t cls,
                 int64_t cbs, int b0, int nb, int l0, int nl, int grid_cap,
                 hipStream_t stream, ProfRecorder& prof, int32_t split = 0,
-                int whole_grid_cap = 0) {
+                int whole_grid_cap = 0, hipEvent_t done = nullptr) {
   if (nl < 1 || static_cast<int64_t>(nl) * g.ptrs_per_layer > kMaxLayersPerLaunch)
     return fail(kInval, "internal: a launch of %d layers exceeds the %d layer pointers of the "
                 "kernel arguments", nl, kMaxLayersPerLaunch / g.ptrs_per_layer);
@@ -1142,6 +1144,7 @@ int launch_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int64_t cks
   int rc = prof.kernel_events(&ea, &eb);
   if (rc) return rc;
   prof.kernel_span(ea, eb, static_cast<int64_t>(nb) * nl * g.kv * g.chunk);
+  if (!eb) eb = done;
   (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
   const unsigned lds = kIota ? FKV_HBM_LDS_PAD : 0;
   if (whole)
@@ -1765,7 +1768,12 @@ int transfer_ce_per_chunk(const Geometry& g, hipStream_t stream, bool h2d) {
 struct fkv_transfer_handle_s {
   int dev = 0;
   hipStream_t stream = nullptr;
-  std::vector<hipEvent_t> done;   // one per layer group, in order
+  std::vector<hipEvent_t> done;   // per layer group, in order; groups of one launch share one
+  std::vector<hipEvent_t> events; // the distinct events of `done`
+  // Kernel path: one past the last group whose transfer group i's event also
+  // covers on the legacy null stream (see fkv_handle_stream_wait).
+  std::vector<int> null_covers;
+  int null_upto = 0;              // groups the device's legacy null stream waits for (mu)
   IdBuf ids;
   ProfRecorder prof;
   bool enqueued = false;          // every group was enqueued
@@ -1812,6 +1820,40 @@ bool handle_live(fkv_transfer_handle_s* h) {
   return std::find(g_handles.begin(), g_handles.end(), h) != g_handles.end();
 }
 
+// Whether `stream` is under HIP graph capture (or cannot tell).
+bool stream_captured(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (stream && hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return cap != hipStreamCaptureStatusNone;
+}
+
+// Whether the legacy null stream waits for work queued on `stream` by itself.
+bool stream_blocks_null(hipStream_t stream) {
+  unsigned flags = 0;
+  if (stream && hipStreamGetFlags(stream, &flags) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return !(flags & hipStreamNonBlocking);
+}
+
+// Bytes a layer-wise launch of the zero-copy kernel aims for: groups smaller
+// than this share launches, whose one event serves all of them.  Every launch
+// costs about 8 us beyond its bytes' link time on the device (ramp, drain and
+// the gap to the next) and 3-6 us on the host, so a 2 MiB handle of 32
+// one-layer groups takes 349 us with a launch per group and 85 us in two.
+// Launches grow from the minimum to the maximum and shrink towards the end
+// (at most half of what is left), so the first groups arrive early and little
+// compute is left when the last ones land.  Measured on MI355X, 80 MiB in 32
+// groups of 2.5 MiB: 1877 us with a launch and a recorded event per group,
+// 1771 us with the event on the kernel's packet, 1642 us with 4 MiB
+// launches.
+constexpr int64_t kLayerwiseMinLaunchBytes = int64_t(1) << 20;
+constexpr int64_t kLayerwiseMaxLaunchBytes = int64_t(4) << 20;
+
 int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transfer_cus, bool h2d,
                       int granularity, fkv_transfer_handle_s* h) {
   DeviceState& d = g_dev[dev];
@@ -1823,21 +1865,46 @@ int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transf
                                     : std::min(transfer_cus, d.num_cus);
   const int grid_cap = cus * (h2d ? d.occ_zero_copy[1] : d.occ_zero_copy[0]);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
-  for (int g0 = 0; g0 < g.num_layers; g0 += granularity) {
-    const int gend = std::min(g.num_layers, g0 + granularity);
-    for (int l0 = g0; l0 < gend; l0 += g.layers_per_launch()) {
-      const int nl = std::min(g.layers_per_launch(), gend - l0);
-      char* base = cpu_dev + static_cast<int64_t>(l0) * g.cls;
-      rc = h2d ? launch_copy<true, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0,
-                                          g.num_blocks, l0, nl, grid_cap, stream, h->prof)
-               : launch_copy<false, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0,
-                                           g.num_blocks, l0, nl, grid_cap, stream, h->prof);
-      if (rc) return rc;
-    }
+  // Under capture the launches record plain events, as graph nodes.
+  const bool captured = stream_captured(stream);
+  // A launch's event rides on its kernel's packet, host-to-device only: a
+  // device-to-host group's event has to release to the host.
+  const bool on_kernel = h2d && !h->prof.on && !captured;
+  const bool null_ordered = !captured && stream_blocks_null(stream);
+  const int ngroups = (g.num_layers + granularity - 1) / granularity;
+  const int64_t group_bytes = static_cast<int64_t>(g.num_blocks) *
+                              std::min(granularity, g.num_layers) * g.kv * g.chunk;
+  const int64_t max_groups = std::max(1, g.layers_per_launch() / granularity);
+  int64_t ramp = kLayerwiseMinLaunchBytes;
+  for (int grp = 0; grp < ngroups;) {
+    const int64_t left = static_cast<int64_t>(ngroups - grp) * group_bytes;
+    const int64_t want = std::min({ramp, kLayerwiseMaxLaunchBytes,
+                                   std::max(kLayerwiseMinLaunchBytes, left / 2)});
+    ramp = std::min(2 * ramp, kLayerwiseMaxLaunchBytes);
+    const int64_t take = std::min({std::max<int64_t>(1, (want + group_bytes / 2) / group_bytes),
+                                   max_groups, static_cast<int64_t>(ngroups - grp)});
+    const int gend = grp + static_cast<int>(take);
+    const int lend = static_cast<int>(
+        std::min<int64_t>(g.num_layers, static_cast<int64_t>(gend) * granularity));
     hipEvent_t ev = nullptr;
     FKV_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    h->done.push_back(ev);
-    FKV_HIP(hipEventRecord(ev, stream));
+    h->events.push_back(ev);
+    for (int l0 = grp * granularity; l0 < lend;) {
+      const int nl = std::min(g.layers_per_launch(), lend - l0);
+      char* base = cpu_dev + static_cast<int64_t>(l0) * g.cls;
+      hipEvent_t done = on_kernel && l0 + nl == lend ? ev : nullptr;
+      rc = h2d ? launch_copy<true, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
+                                          l0, nl, grid_cap, stream, h->prof, 0, 0, done)
+               : launch_copy<false, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
+                                           l0, nl, grid_cap, stream, h->prof);
+      if (rc) return rc;
+      l0 += nl;
+    }
+    if (!on_kernel) FKV_HIP(hipEventRecord(ev, stream));
+    h->done.insert(h->done.end(), static_cast<size_t>(take), ev);
+    h->null_covers.insert(h->null_covers.end(), static_cast<size_t>(take),
+                          null_ordered ? ngroups : gend);
+    grp = gend;
   }
   h->enqueued = true;
   return 0;
@@ -1857,7 +1924,7 @@ int handle_destroy(fkv_transfer_handle_s* h) {
     if (e != hipSuccess) rc = fail(static_cast<int>(e), "hipStreamSynchronize: %s", hipGetErrorString(e));
   }
   h->prof.flush();
-  for (hipEvent_t ev : h->done) (void)hipEventDestroy(ev);
+  for (hipEvent_t ev : h->events) (void)hipEventDestroy(ev);
   if (h->start) (void)hipEventDestroy(h->start);
   if (h->ids.host) ids_release(h->ids);
   delete h;
@@ -2155,6 +2222,7 @@ int layerwise_ce_start(const Geometry& g, hipStream_t stream, int dev, int granu
     hipEvent_t ev = nullptr;
     FKV_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     h->done.push_back(ev);
+    h->events.push_back(ev);
   }
   FKV_HIP(hipEventCreateWithFlags(&h->start, hipEventDisableTiming));
   FKV_HIP(hipEventRecord(h->start, stream));
@@ -2473,7 +2541,26 @@ int fkv_handle_stream_wait(fkv_transfer_handle h, int group, fkv_stream_t other)
     const int rc = ce_group_recorded(h, group);
     if (rc) return rc;
   }
-  FKV_HIP(hipStreamWaitEvent(static_cast<hipStream_t>(other), h->done[group], 0));
+  // The legacy null stream waits by itself for all work already queued on the
+  // device's blocking streams, and every operation on it pays for that (about
+  // 14 us of host time and 11 us of the stream's while a transfer runs).  So
+  // one wait on it covers every group already queued on a blocking stream,
+  // and later waits of the handle for those groups add nothing: 32 of them
+  // beside an 80 MiB transfer made its pass 2.2 ms instead of 1.8 ms.
+  hipStream_t st = static_cast<hipStream_t>(other);
+  int cur = -1;
+  if (!st) FKV_HIP(hipGetDevice(&cur));
+  if (!st && cur == h->dev) {
+    std::lock_guard<std::mutex> lk(h->mu);
+    if (group < h->null_upto) return 0;
+    // the pipeline stream, which records a copy-engine handle's events, is a
+    // blocking one
+    const int covers = h->ce ? h->recorded : h->null_covers[group];
+    FKV_HIP(hipStreamWaitEvent(st, h->done[group], 0));
+    h->null_upto = std::max(h->null_upto, covers);
+    return 0;
+  }
+  FKV_HIP(hipStreamWaitEvent(st, h->done[group], 0));
   return 0;
 }
 

@@ -195,6 +195,7 @@ int fkv_scatter_kv_blocks(int num_blocks, int num_layers, const int64_t* gpu_blo
  * use_ce_transfer = FKV_XFER_KERNEL: the zero-copy kernel, every group
  * enqueued on `stream` before the call returns; fkv_handle_stream_wait makes
  * the other stream wait on the device, without a host round trip.
+ * Small groups share launches of 1-4 MiB, and the event of the launch.
  * transfer_cus = -1 selects 2 compute units for host-to-device transfers
  * (enough for the link; the rest of the chip stays with the compute the
  * transfer overlaps) and 8 for device-to-host.

@@ -441,3 +441,102 @@ def test_ce_handle_without_engines():
     assert res.returncode == 0, res.stderr[-2000:]
     assert "match the oracle" in res.stdout
     assert res.stderr.count("copy engines unavailable") == 1
+
+
+def _kernel_launches(L, G, layer_bytes, lpl=128, lo=1 << 20, hi=4 << 20):
+    """Launches of a zero-copy layer-wise handle: groups share launches that
+    grow from `lo` to `hi` bytes and hold at most half of what is left (but
+    `lo`); a group of more layers than one launch's pointers takes several."""
+    ngroups, gb = -(-L // G), min(G, L) * layer_bytes
+    ramp, grp, launches = lo, 0, 0
+    while grp < ngroups:
+        want = min(ramp, hi, max(lo, (ngroups - grp) * gb // 2))
+        ramp = min(2 * ramp, hi)
+        take = min(max(1, (want + gb // 2) // gb), max(1, lpl // G), ngroups - grp)
+        layers = min(L, (grp + take) * G) - grp * G
+        launches += -(-layers // lpl)
+        grp += take
+    return launches
+
+
+@pytest.mark.parametrize("h2d", [True, False], ids=["h2d", "d2h"])
+@pytest.mark.parametrize("L,heads,n,gran", [(16, 8, 1, 1), (16, 8, 40, 1), (19, 8, 9, 2),
+                                            (16, 1, 3, 1), (130, 1, 4, 130), (140, 1, 2, 1)])
+def test_kernel_handle_launches(L, heads, n, gran, h2d):
+    """Groups that share a launch, groups of one launch each and a group of
+    two launches: the planned launches, and every group's bytes once its event
+    has fired."""
+    from flexkv_amd import _lib
+    from gpu_util import DeviceCase
+    case = KVCase(layers_total=L, num_layers=L, start_layer=0, kv=2, ng=48, nh=64, tokens=16,
+                  heads=heads, dim=128).fill(seed=L + n)
+    gids, cids = inputs.distinct_ids(110, n, 48), inputs.distinct_ids(111, n, 64)
+    dc = DeviceCase(case)
+    fresh = case.host ^ np.uint16(0x55AA)
+    if h2d:
+        dc.set_host(fresh)
+    for profiled in (True, False):
+        if h2d:
+            dc.set_gpu([np.zeros_like(g) for g in case.gpu])
+        else:
+            dc.set_host(case.host)
+        torch.cuda.synchronize()
+        if profiled:
+            _lib.profile_enable(True)
+        try:
+            with _abi_layerwise(dc, gids.copy(), cids.copy(), h2d, gran) as hnd:
+                assert hnd.num_groups == -(-L // gran)
+                for g in range(hnd.num_groups):
+                    hnd.wait(g)
+                    for l in range(g * gran, min(L, (g + 1) * gran)):
+                        if h2d:
+                            want = np.stack([case.host_view(fresh)[c, l, :, 0] for c in cids], axis=1)
+                            assert np.array_equal(dc.gpu_np()[l][:, gids], want), (g, l)
+                        else:
+                            got = case.host_view(dc.host_np())[cids, l, :, 0]
+                            want = np.stack([case.gpu[l][:, b] for b in gids])
+                            assert np.array_equal(got, want), (g, l)
+            if profiled:
+                launches = _lib.profile_read()["kernel_launches"]
+        finally:
+            if profiled:
+                _lib.profile_enable(False)
+    assert launches == _kernel_launches(L, gran, 2 * n * case.strides()["chunk"])
+
+
+@pytest.mark.parametrize("ce", [False, True], ids=["kernel", "ce"])
+@pytest.mark.parametrize("own_queue", [False, True], ids=["torch-stream", "transfer-stream"])
+@pytest.mark.parametrize("n", [1, 40])
+def test_null_stream_consumer(n, own_queue, ce):
+    """A consumer on the legacy null stream, which waits for blocking streams
+    by itself: with the transfer on a stream it does not wait for (torch's)
+    and on one it does (fkv_stream_create's), it sees every group's bytes."""
+    from flexkv_amd import c_ext
+    from gpu_util import DeviceCase
+    L = 12
+    case = KVCase(layers_total=L, num_layers=L, start_layer=0, kv=2, ng=64, nh=96, tokens=16,
+                  heads=8, dim=128).fill(seed=120 + n)
+    gids, cids = inputs.distinct_ids(121, n, 64), inputs.distinct_ids(122, n, 96)
+    dc = DeviceCase(case)
+    xfer = c_ext.transfer_stream() if own_queue else torch.cuda.Stream()
+    g_dev = torch.from_numpy(gids).to("cuda")
+    hv = None
+    for rnd in range(3):
+        fresh = case.host ^ np.uint16(0x1111 * (rnd + 1))
+        dc.set_host(fresh)
+        dc.set_gpu([np.zeros_like(g) for g in case.gpu])
+        torch.cuda.synchronize()
+        with torch.cuda.stream(xfer):
+            hnd = _abi_layerwise(dc, gids.copy(), cids.copy(), True, 1, stream=xfer, ce=ce)
+        null = torch.cuda.default_stream()
+        outs = []
+        with torch.cuda.stream(null):
+            for l in (0, 5, 2, 5, *range(L)):
+                hnd.stream_wait(l, null)
+                outs.append((l, dc.gpu[l][:, g_dev].clone()))
+        null.synchronize()
+        hnd.release()
+        hv = case.host_view(fresh)
+        for l, out in outs:
+            want = np.stack([hv[c, l, :, 0] for c in cids], axis=1)
+            assert np.array_equal(out.cpu().numpy().view(np.uint16), want), (rnd, l)
