@@ -1,24 +1,26 @@
 // kv_transfer.hip - GPU<->CPU KV-block transfer for MI355X (gfx950).
 //
-// One kernel template moves "chunks": the (layer, K|V, block) pieces of the
-// KV cache, each `chunk_size` contiguous bytes on both sides
-// (csrc/transfer.cu:39-53 gives the reference addressing).  It is used twice:
-//   * zero-copy mode: the "CPU side" is the pinned host cache itself and the
-//     kernel's 16-byte loads/stores travel over PCIe;
-//   * copy-engine mode: the "CPU side" is a contiguous HBM staging buffer laid
-//     out [block][layer][K|V][chunk]; the SDMA engines (queued through HSA)
-//     then move maximal contiguous host runs between staging and the host
-//     cache.
+// The unit is the "chunk": a (layer, K|V, block) piece of the KV cache,
+// `chunk_size` contiguous bytes on both sides (csrc/transfer.cu:39-53 gives
+// the reference addressing).
+//   * Zero-copy transfers: kv_zero_copy_kernel (kv_small_copy_kernel for the
+//     smallest calls) moves chunks between the GPU cache and the pinned host
+//     cache itself; its 16-byte loads or stores travel over PCIe.
+//   * Copy-engine transfers and device gathers / scatters: a staging kernel
+//     moves chunks between the GPU cache and a contiguous HBM buffer laid out
+//     [block][layer][K|V][chunk]; for copy-engine transfers the SDMA engines
+//     (queued through HSA) then move maximal contiguous host runs between
+//     that buffer and the host cache.
 //
-// Work decomposition: a workgroup (4 wavefronts) owns a tile of consecutive
-// blocks; it stages the tile's (gpu_id, cpu_id) pairs in LDS, then its
-// wavefronts stream the tile's rows (64 lanes x 16 B = 1 KiB) in groups of
-// kUnroll rows, issuing all loads of a group before any store.  Rows are
-// ordered block -> layer -> K|V -> offset, which is host-address order for the
-// block-wise host layout.  Layer base pointers travel in the kernel argument
-// block (scalar loads, no PCIe round trip per chunk).  Staging gathers whose
-// chunks are whole groups of 32 rows address each group from one buffer
-// resource per side instead of a 64-bit base per row.
+// Staging work decomposition (kv_chunk_copy_kernel): a workgroup (4
+// wavefronts) owns a tile of consecutive blocks; it stages the tile's ids in
+// LDS, then its wavefronts stream the tile's rows (64 lanes x 16 B = 1 KiB)
+// in groups of kUnroll rows, issuing all loads of a group before any store.
+// Rows are ordered block -> layer -> K|V -> offset.  Layer base pointers
+// travel in the kernel argument block.  Gathers whose chunks are whole groups
+// of 32 rows address each group from one buffer resource per side instead of
+// a 64-bit base per row; kv_pack_kernel and kv_pack_span_kernel take the other
+// shapes of whole rows.
 //
 // This file holds the kernels, the transfer paths that launch them and the
 // transfer entry points of the C ABI; kv_host.cpp holds validation, id staging
@@ -46,32 +48,17 @@ using namespace fkv_detail;
 
 namespace {
 
-// Rows (64 lanes x 16 B) each wavefront keeps in flight: the zero-copy
-// kernel is PCIe bound, the staging gather/scatter HBM bound.  Measured on
-// MI355X at the Llama-3-8B shape with 8 CUs: D2H best at 8 rows, H2D at 4.
-#ifndef FKV_UNROLL_ZC_D2H
-#define FKV_UNROLL_ZC_D2H 8
-#endif
-#ifndef FKV_UNROLL_ZC_H2D
-#define FKV_UNROLL_ZC_H2D 4
-#endif
+// Rows (64 lanes x 16 B) each wavefront of the staging kernels keeps in
+// flight.
 #ifndef FKV_UNROLL_HBM
 #define FKV_UNROLL_HBM 32
-#endif
-// Wave issue priority (s_setprio, 0-3) of the zero-copy kernel, which shares
-// compute units with the caller's kernels when transfers overlap compute.
-#ifndef FKV_ZC_PRIO
-#define FKV_ZC_PRIO 0
 #endif
 // Staging gather/scatter launch shape: 1 = one workgroup per tile (grid =
 // tiles), 0 = an occupancy-sized grid looping over tiles.
 #ifndef FKV_HBM_ONEPASS
 #define FKV_HBM_ONEPASS 1
 #endif
-// Tiles per occupancy slot the tiling aims for (zero-copy / staging).
-#ifndef FKV_TILE_FACTOR
-#define FKV_TILE_FACTOR 4
-#endif
+// Tiles per occupancy slot the staging tiling aims for.
 #ifndef FKV_TILE_FACTOR_HBM
 #define FKV_TILE_FACTOR_HBM 16
 #endif
@@ -91,23 +78,13 @@ namespace {
 #ifndef FKV_WHOLE_SCATTER
 #define FKV_WHOLE_SCATTER 1
 #endif
-// Zero-copy launches whose chunks are whole sub-groups (4 rows D2H, whose
-// group of 8 rows in flight is addressed as two halves; 4 rows H2D) take the
-// whole-group variant, which keeps one base per sub-group instead of one
-// address per row (no spills).
-#ifndef FKV_WHOLE_ZERO_COPY
-#define FKV_WHOLE_ZERO_COPY 1
-#endif
-// Cache hints: loads are non-temporal everywhere; stores are non-temporal
-// into HBM but plain into pinned host memory (about 2% faster D2H over PCIe).
+// Cache hints: loads are non-temporal everywhere, and so are stores into HBM
+// (stores into host memory: store_system).
 #ifndef FKV_NT_LOAD
 #define FKV_NT_LOAD 1
 #endif
 #ifndef FKV_NT_STORE_HBM
 #define FKV_NT_STORE_HBM 1
-#endif
-#ifndef FKV_NT_STORE_HOST
-#define FKV_NT_STORE_HOST 0
 #endif
 // The staging scatter (packed HBM -> scattered chunks) has its own knobs.
 #ifndef FKV_UNROLL_SCATTER
@@ -146,17 +123,12 @@ constexpr int kThreads = 256;               // 4 wavefronts of 64 lanes
 constexpr int64_t kWholeScatterMaxBytes = int64_t(512) << 20;
 constexpr int kWaves = kThreads / 64;
 constexpr int kUnrollHbm = FKV_UNROLL_HBM;
-// Sub-groups per group of the whole-group variant: the zero-copy D2H group of
-// 8 rows in flight is two sub-groups of 4 rows, so chunks of 4 KiB (the
-// Llama-3-70B TP-8 shard) take it; every other instantiation addresses its
-// group as one.  Each sub-group lies inside one chunk.
-template <bool kH2D, bool kIotaCpu>
-constexpr int whole_sub_groups() { return (!kIotaCpu && !kH2D && FKV_UNROLL_ZC_D2H % 2 == 0) ? 2 : 1; }
 constexpr int kMaxTileBlocks = 64;
-// Transfers of at most this many blocks carry their (gpu_id, cpu_id) pairs in
+// Launches of at most this many blocks carry their (gpu_id, cpu_id) pairs in
 // the kernel arguments, so no workgroup reads them over PCIe first (one host
-// round trip less per call; a one-block zero-copy call is latency-bound).
+// round trip less per launch).
 constexpr int kInlineIds = 32;
+constexpr int kInlineIdsZeroCopy = 96;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -204,27 +176,19 @@ __device__ inline int64_t wave_uniform(int64_t x) {
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-// kH2D: copy CPU side -> GPU side.  kIotaCpu: the CPU side is staging and
-// block i of the launch sits at CPU-side block index i (ids[2i+1] unused).
+// Staging gather (kH2D false: GPU cache -> packed buffer, the "CPU side") or
+// scatter (kH2D true).  Block i of the launch sits at CPU-side block index i.
 // Row addresses are wave-uniform (scalar registers); each lane adds its own
 // 16-byte slot, so one 32-bit lane offset serves every access.
-// kWhole: the launch's chunks are whole sub-groups of kUnroll / kSub full
-// rows (kSub = whole_sub_groups(); the host checks rows_per_chunk % (kUnroll /
-// kSub) == 0 and no partial row), so each sub-group lies inside one chunk and
-// is addressed from one base per side.
-template <bool kH2D, bool kIotaCpu, bool kWhole = false>
+// kWhole: the launch's chunks are whole groups of kUnroll full rows, so each
+// group lies inside one chunk and is addressed from one base per side.
+template <bool kH2D, bool kWhole = false>
 __global__ __launch_bounds__(kThreads) void kv_chunk_copy_kernel(CopyArgs a) {
-  constexpr bool kScatter = kIotaCpu && kH2D;
-  constexpr int kUnroll = kIotaCpu ? (kScatter ? FKV_UNROLL_SCATTER : kUnrollHbm)
-                                   : (kH2D ? FKV_UNROLL_ZC_H2D : FKV_UNROLL_ZC_D2H);
-  // only the zero-copy D2H instantiation stores into host memory
-  constexpr bool kNtStore = kScatter ? FKV_NT_STORE_SCATTER
-                                     : ((kIotaCpu || kH2D) ? FKV_NT_STORE_HBM : FKV_NT_STORE_HOST);
-  constexpr bool kNtLoad = kScatter ? FKV_NT_LOAD_SCATTER : FKV_NT_LOAD;
+  constexpr int kUnroll = kH2D ? FKV_UNROLL_SCATTER : kUnrollHbm;
+  constexpr bool kNtStore = kH2D ? FKV_NT_STORE_SCATTER : FKV_NT_STORE_HBM;
+  constexpr bool kNtLoad = kH2D ? FKV_NT_LOAD_SCATTER : FKV_NT_LOAD;
   __shared__ int64_t s_gid[kMaxTileBlocks];
-  __shared__ int64_t s_cid[kMaxTileBlocks];
 
-  if (!kIotaCpu && FKV_ZC_PRIO > 0) __builtin_amdgcn_s_setprio(FKV_ZC_PRIO);
   const int lane = threadIdx.x & 63;
   const uint32_t lane_off = static_cast<uint32_t>(lane) * 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -235,7 +199,7 @@ __global__ __launch_bounds__(kThreads) void kv_chunk_copy_kernel(CopyArgs a) {
   const bool full_rows = (a.chunk_vec & 63) == 0;
 
   int first = blockIdx.x;
-  if (kIotaCpu && FKV_XCD_REMAP && (gridDim.x & 7) == 0) {
+  if (FKV_XCD_REMAP && (gridDim.x & 7) == 0) {
     const int per = gridDim.x >> 3;
     first = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   }
@@ -252,19 +216,9 @@ __global__ __launch_bounds__(kThreads) void kv_chunk_copy_kernel(CopyArgs a) {
     __syncthreads();  // previous tile's readers are done with the LDS ids
     if (threadIdx.x < nb) {
       const int j = b0 + threadIdx.x;
-      int64_t gid, cid;
-      if (a.inline_n) {
-        gid = a.inline_ids[2 * j];
-        cid = a.inline_ids[2 * j + 1];
-      } else if (a.ids_split) {
-        gid = a.ids[j];
-        cid = a.ids[static_cast<int64_t>(a.ids_split) + j];
-      } else {
-        gid = a.ids[2 * static_cast<int64_t>(j)];
-        cid = a.ids[2 * static_cast<int64_t>(j) + 1];
-      }
-      s_gid[threadIdx.x] = gid;
-      s_cid[threadIdx.x] = kIotaCpu ? static_cast<int64_t>(j) : cid;
+      s_gid[threadIdx.x] = a.inline_n    ? a.inline_ids[2 * j]
+                           : a.ids_split ? a.ids[j]
+                                         : a.ids[2 * static_cast<int64_t>(j)];
     }
     __syncthreads();
 
@@ -273,154 +227,84 @@ __global__ __launch_bounds__(kThreads) void kv_chunk_copy_kernel(CopyArgs a) {
     const uint32_t g_begin = static_cast<uint32_t>(tr) * a.split_rows;
     const uint32_t g_end = min(rows, g_begin + a.split_rows);
     if constexpr (kWhole) {
-      // Groups start at multiples of kUnroll and sub-groups at multiples of
-      // kR, so each sub-group lies inside one chunk: consecutive 1 KiB rows
-      // on both sides.  A tile's rows are a multiple of kR, not always of
-      // kUnroll, so a group's later sub-groups may lie past g_end.
-      constexpr int kSub = whole_sub_groups<kH2D, kIotaCpu>();
-      constexpr int kR = kUnroll / kSub;
-      static_assert(kR * kSub == kUnroll, "a group is kSub sub-groups of kR rows");
       for (uint32_t g = g_begin + static_cast<uint32_t>(wave) * kUnroll; g < g_end;
            g += kWaves * kUnroll) {
-        // Raw buffer accesses: the sub-group's base in a buffer resource
-        // (scalar registers), the lane's 16-byte slot as the vector offset
-        // and the row as a scalar offset, so no per-row 64-bit address is
-        // kept.
-        __amdgpu_buffer_rsrc_t rs[kSub], rd[kSub];
-        bool live[kSub];
-#pragma unroll
-        for (int s = 0; s < kSub; ++s) {
-          const uint32_t gs = g + static_cast<uint32_t>(s * kR);
-          live[s] = s == 0 || gs < g_end;
-          // a sub-group past g_end takes the first one's row (never accessed)
-          const uint32_t row = live[s] ? gs : g;
-          const uint32_t item = row / rpc;
-          const uint32_t rr = row - item * rpc;
-          const uint32_t bi = item / items_per_block;
-          const uint32_t rem = item - bi * items_per_block;
-          const uint32_t l = rem / kv;
-          const uint32_t k = rem - l * kv;
-          const uint32_t layer = static_cast<uint32_t>(l0) + l;
-          const int64_t gid = wave_uniform(s_gid[bi]);
-          const int64_t cid = wave_uniform(s_cid[bi]);
-          const int64_t row_off = static_cast<int64_t>(rr) * (64 * 16);
-          char* gpu = reinterpret_cast<char*>(a.layer_ptr[layer * ppl + k * (ppl - 1)]) +
-                      static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride +
-                      row_off;
-          char* cpu = a.cpu_base + static_cast<int64_t>(layer) * a.cpu_layer_stride +
-                      static_cast<int64_t>(k) * a.cpu_kv_stride + cid * a.cpu_block_stride +
-                      row_off;
-          rs[s] = __builtin_amdgcn_make_buffer_rsrc(kH2D ? cpu : gpu, 0, -1, kBufferRsrcWord3);
-          rd[s] = __builtin_amdgcn_make_buffer_rsrc(kH2D ? gpu : cpu, 0, -1, kBufferRsrcWord3);
-        }
+        // Raw buffer accesses: the group's base in a buffer resource (scalar
+        // registers), the lane's 16-byte slot as the vector offset and the
+        // row as a scalar offset, so no per-row 64-bit address is kept.
+        const uint32_t item = g / rpc;
+        const uint32_t rr = g - item * rpc;
+        const uint32_t bi = item / items_per_block;
+        const uint32_t rem = item - bi * items_per_block;
+        const uint32_t l = rem / kv;
+        const uint32_t k = rem - l * kv;
+        const uint32_t layer = static_cast<uint32_t>(l0) + l;
+        const int64_t gid = wave_uniform(s_gid[bi]);
+        const int64_t row_off = static_cast<int64_t>(rr) * (64 * 16);
+        char* gpu = reinterpret_cast<char*>(a.layer_ptr[layer * ppl + k * (ppl - 1)]) +
+                    static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride + row_off;
+        char* cpu = a.cpu_base + static_cast<int64_t>(layer) * a.cpu_layer_stride +
+                    static_cast<int64_t>(k) * a.cpu_kv_stride +
+                    static_cast<int64_t>(b0 + static_cast<int>(bi)) * a.cpu_block_stride + row_off;
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc(kH2D ? cpu : gpu, 0, -1, kBufferRsrcWord3);
+        const __amdgpu_buffer_rsrc_t rd =
+            __builtin_amdgcn_make_buffer_rsrc(kH2D ? gpu : cpu, 0, -1, kBufferRsrcWord3);
         i32x4 v[kUnroll];
 #pragma unroll
-        for (int s = 0; s < kSub; ++s)
-          if (live[s]) {
+        for (int u = 0; u < kUnroll; ++u)
+          v[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, u * (64 * 16),
+                                                       kNtLoad ? kCachePolicyNt : 0);
 #pragma unroll
-            for (int u = 0; u < kR; ++u)
-              v[s * kR + u] = __builtin_amdgcn_raw_buffer_load_b128(
-                  rs[s], lane_off, u * (64 * 16), kNtLoad ? kCachePolicyNt : 0);
-          }
-#pragma unroll
-        for (int s = 0; s < kSub; ++s)
-          if (live[s]) {
-#pragma unroll
-            for (int u = 0; u < kR; ++u)
-              __builtin_amdgcn_raw_buffer_store_b128(v[s * kR + u], rd[s], lane_off,
-                                                     u * (64 * 16),
-                                                     kNtStore ? kCachePolicyNt : 0);
-          }
+        for (int u = 0; u < kUnroll; ++u)
+          __builtin_amdgcn_raw_buffer_store_b128(v[u], rd, lane_off, u * (64 * 16),
+                                                 kNtStore ? kCachePolicyNt : 0);
       }
     } else {
       for (uint32_t g = g_begin + static_cast<uint32_t>(wave) * kUnroll; g < g_end;
            g += kWaves * kUnroll) {
-        if constexpr (kIotaCpu) {
-          // Staging: the group's rows are walked twice from the same cursor
-          // over (block, layer, K|V, row), once to issue the loads and once to
-          // issue the stores.  No row address is held between the two walks,
-          // so only the loaded data stays live: holding 2 x U 64-bit row
-          // addresses spilled 358-387 scalar registers at U = 32.
-          const uint32_t item0 = g / rpc;
-          const uint32_t rr0 = g - item0 * rpc;
-          const uint32_t bi0 = item0 / items_per_block;
-          const uint32_t rem0 = item0 - bi0 * items_per_block;
-          const uint32_t lw0 = rem0 / kv;
-          const uint32_t kw0 = rem0 - lw0 * kv;
-          u32x4 v[kUnroll];
+        // The group's rows are walked twice from the same cursor
+        // over (block, layer, K|V, row), once to issue the loads and once to
+        // issue the stores.  No row address is held between the two walks,
+        // so only the loaded data stays live: holding 2 x U 64-bit row
+        // addresses spilled 358-387 scalar registers at U = 32.
+        const uint32_t item0 = g / rpc;
+        const uint32_t rr0 = g - item0 * rpc;
+        const uint32_t bi0 = item0 / items_per_block;
+        const uint32_t rem0 = item0 - bi0 * items_per_block;
+        const uint32_t lw0 = rem0 / kv;
+        const uint32_t kw0 = rem0 - lw0 * kv;
+        u32x4 v[kUnroll];
 #pragma unroll
-          for (int pass = 0; pass < 2; ++pass) {
-            uint32_t rr = rr0, bi = bi0, l = lw0, k = kw0;
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-              const uint32_t bsafe = min(bi, static_cast<uint32_t>(nb - 1));
-              const uint32_t layer = static_cast<uint32_t>(l0) + min(l, nl - 1);
-              const int64_t gid = wave_uniform(s_gid[bsafe]);
-              const int64_t cid = wave_uniform(s_cid[bsafe]);
-              const int64_t row_off = static_cast<int64_t>(rr) * (64 * 16);
-              char* gpu = reinterpret_cast<char*>(a.layer_ptr[layer * ppl + k * (ppl - 1)]) +
-                          static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride +
-                          row_off;
-              char* cpu = a.cpu_base + static_cast<int64_t>(layer) * a.cpu_layer_stride +
-                          static_cast<int64_t>(k) * a.cpu_kv_stride + cid * a.cpu_block_stride +
-                          row_off;
-              const bool live = (g + u < g_end) &&
-                                (full_rows || static_cast<int64_t>(rr) * 64 + lane < a.chunk_vec);
-              if (live) {
-                if (pass == 0) {
-                  const gvec* p = (const gvec*)((kH2D ? cpu : gpu) + lane_off);
-                  v[u] = kNtLoad ? __builtin_nontemporal_load(p) : *p;
-                } else {
-                  gvec* p = (gvec*)((kH2D ? gpu : cpu) + lane_off);
-                  if (kNtStore)
-                    __builtin_nontemporal_store(v[u], p);
-                  else
-                    *p = v[u];
-                }
-              }
-              // advance the cursor by one row
-              if (++rr == rpc) {
-                rr = 0;
-                if (++k == kv) {
-                  k = 0;
-                  if (++l == nl) {
-                    l = 0;
-                    ++bi;
-                  }
-                }
-              }
-            }
-          }
-        } else {
-          // Zero-copy: U is 4-8, so the group's row addresses are computed
-          // once and held.  Walking twice made the host-to-device kernel on 2
-          // compute units 35% slower (36.7 against 56.7 GB/s).
-          uint32_t item = g / rpc;
-          uint32_t rr = g - item * rpc;
-          uint32_t bi = item / items_per_block;
-          uint32_t rem = item - bi * items_per_block;
-          uint32_t l = rem / kv;
-          uint32_t k = rem - l * kv;
-          const char* src[kUnroll];
-          char* dst[kUnroll];
-          bool live[kUnroll];
+        for (int pass = 0; pass < 2; ++pass) {
+          uint32_t rr = rr0, bi = bi0, l = lw0, k = kw0;
 #pragma unroll
           for (int u = 0; u < kUnroll; ++u) {
             const uint32_t bsafe = min(bi, static_cast<uint32_t>(nb - 1));
             const uint32_t layer = static_cast<uint32_t>(l0) + min(l, nl - 1);
             const int64_t gid = wave_uniform(s_gid[bsafe]);
-            const int64_t cid = wave_uniform(s_cid[bsafe]);
             const int64_t row_off = static_cast<int64_t>(rr) * (64 * 16);
             char* gpu = reinterpret_cast<char*>(a.layer_ptr[layer * ppl + k * (ppl - 1)]) +
                         static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride +
                         row_off;
             char* cpu = a.cpu_base + static_cast<int64_t>(layer) * a.cpu_layer_stride +
-                        static_cast<int64_t>(k) * a.cpu_kv_stride + cid * a.cpu_block_stride +
+                        static_cast<int64_t>(k) * a.cpu_kv_stride +
+                        static_cast<int64_t>(b0 + static_cast<int>(bsafe)) * a.cpu_block_stride +
                         row_off;
-            live[u] = (g + u < g_end) &&
-                      (full_rows || static_cast<int64_t>(rr) * 64 + lane < a.chunk_vec);
-            src[u] = kH2D ? cpu : gpu;
-            dst[u] = kH2D ? gpu : cpu;
+            const bool live = (g + u < g_end) &&
+                              (full_rows || static_cast<int64_t>(rr) * 64 + lane < a.chunk_vec);
+            if (live) {
+              if (pass == 0) {
+                const gvec* p = (const gvec*)((kH2D ? cpu : gpu) + lane_off);
+                v[u] = kNtLoad ? __builtin_nontemporal_load(p) : *p;
+              } else {
+                gvec* p = (gvec*)((kH2D ? gpu : cpu) + lane_off);
+                if (kNtStore)
+                  __builtin_nontemporal_store(v[u], p);
+                else
+                  *p = v[u];
+              }
+            }
             // advance the cursor by one row
             if (++rr == rpc) {
               rr = 0;
@@ -431,24 +315,6 @@ __global__ __launch_bounds__(kThreads) void kv_chunk_copy_kernel(CopyArgs a) {
                   ++bi;
                 }
               }
-            }
-          }
-          u32x4 v[kUnroll];
-#pragma unroll
-          for (int u = 0; u < kUnroll; ++u) {
-            if (live[u]) {
-              const gvec* p = (const gvec*)(src[u] + lane_off);
-              v[u] = kNtLoad ? __builtin_nontemporal_load(p) : *p;
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < kUnroll; ++u) {
-            if (live[u]) {
-              gvec* p = (gvec*)(dst[u] + lane_off);
-              if (kNtStore)
-                __builtin_nontemporal_store(v[u], p);
-              else
-                *p = v[u];
             }
           }
         }
@@ -629,6 +495,158 @@ __global__ __launch_bounds__(kThreads) void kv_pack_span_kernel(PackArgs a) {
   }
 }
 
+// The zero-copy kernel: the launch's bytes as one sequence of 16-byte
+// vectors, block -> layer -> K|V -> offset (host-address order for the
+// block-wise host layout), cut into groups of kU rows of 64 vectors.  Each
+// workgroup takes a run of consecutive groups, its wavefronts in turn, and
+// each lane finds the two addresses of its vector by itself, so rows that
+// cross chunks (sizes that are not whole KiB, or under one) leave no lane
+// idle and every shape takes the same code.  Two divisions by multiplication
+// and three LDS reads a row are nothing beside the link, which gives a
+// wavefront a row every 2000 cycles.
+//
+// The link bounds it, and few loads or stores in flight fill the link.
+// Measured on MI355X, us a call (host to device 32 MiB and 1 GiB, device to
+// host 16 MiB and 320 MiB):
+//   workgroups        8      12      14      16      20      24      32
+//   H2D 32 MiB      603.9   603.6   603.1   603.5   616.6   636.1   641
+//   H2D 1 GiB       18781   18755   18673   18721   19112   19778
+//   D2H 16 MiB      315.6   311.1   312.6   317.3   315.0   312.7   310.1
+//   D2H 320 MiB      6083    5921    5954            6079    5967    5910
+// so 14 workgroups read (groups of 4 rows) and 12 write (8 rows).  A tiled
+// kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
+// 1 MiB host-to-device call of one layer (here 33.5).
+template <bool kH2D>
+constexpr int zero_copy_workgroups() { return kH2D ? 14 : 12; }
+template <bool kH2D>
+constexpr int zero_copy_rows() { return kH2D ? 4 : 8; }
+constexpr int kMaxItems = 2 * kMaxLayersPerLaunch;   // (layer, K|V) pairs of a launch
+// LDS for block offsets: with the item table, within the 64 KiB of a launch
+constexpr int kZeroCopyMaxLds = 56 << 10;
+// vectors of a launch: Divider divides numbers below 2^31
+constexpr int64_t kZeroCopyMaxVec = (int64_t(1) << 31) - 1;
+constexpr int64_t kZeroCopyMaxChunkVec = int64_t(1) << 29;
+
+// n / d for n < 2^31 as a multiplication (Granlund and Montgomery, "Division
+// by Invariant Integers using Multiplication", 1994): with 2^(l-1) < d <= 2^l,
+// mul = ceil(2^(31+l) / d) < 2^32 and n / d = floor(n * mul / 2^(31+l)).
+struct Divider {
+  uint32_t d = 1, mul = 0, shift = 0;
+  explicit Divider(uint32_t by = 1) : d(by) {
+    int l = 0;
+    while ((uint64_t(1) << l) < by) ++l;
+    shift = static_cast<uint32_t>(31 + l);
+    mul = static_cast<uint32_t>(((static_cast<unsigned __int128>(1) << shift) + by - 1) / by);
+  }
+  __device__ uint32_t div(uint32_t n) const {
+    return static_cast<uint32_t>((static_cast<uint64_t>(n) * mul) >> shift);
+  }
+};
+
+struct ZeroCopyArgs {
+  const int64_t* ids;        // device-visible (gpu_id, cpu_id) pairs (inline_n == 0)
+  char* cpu_base;            // host side of launch layer 0, block id 0
+  int64_t gpu_kv_stride;
+  int64_t gpu_block_stride;
+  int64_t cpu_kv_stride;
+  int64_t cpu_layer_stride;
+  int64_t cpu_block_stride;
+  Divider chunk;             // by the vectors of a chunk
+  Divider items;             // by the chunks of a block, layers x K|V
+  uint32_t kv_dim;
+  uint32_t num_vec;          // vectors of the launch
+  uint32_t num_groups;
+  uint32_t groups_per_wg;
+  int32_t ptrs_per_layer;    // 1: layer_ptr[l] + k*gpu_kv_stride; kv: layer_ptr[l*kv + k]
+  int32_t inline_n;          // > 0: the launch's pairs are inline_ids, not ids
+  int32_t ids_split;         // > 0: ids holds gpu ids, and cpu ids ids_split entries later
+  uint64_t layer_ptr[kMaxLayersPerLaunch];
+  int64_t inline_ids[2 * kInlineIdsZeroCopy];
+};
+
+// 16 bytes written through every cache (system scope).  Stores into pinned
+// host memory go this way: left to the caches they arrive in the order of
+// evictions, and a 16 MiB device-to-host call took 360 us instead of 317 (16
+// workgroups).  In assembly, as no builtin stores 16 bytes at system scope;
+// the s_nop keeps the two wait states a wide store needs before its data
+// registers are written again, which the compiler cannot see it needs.
+__device__ inline void store_system(char* p, u32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+}
+
+template <bool kH2D>
+__global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) {
+  constexpr int kU = zero_copy_rows<kH2D>();
+  constexpr uint32_t kGroupVec = kU * 64;
+  extern __shared__ int64_t s_block[];      // byte offsets (gpu, cpu) of the run's blocks
+  __shared__ int64_t s_item[2 * kMaxItems]; // address (gpu), byte offset (cpu) of (layer, K|V)
+  const uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t g0 = blockIdx.x * a.groups_per_wg;
+  const uint32_t g1 = min(g0 + a.groups_per_wg, a.num_groups);
+  // the blocks of the run
+  const uint32_t b0 = a.items.div(a.chunk.div(g0 * kGroupVec));
+  const uint32_t b1 = a.items.div(a.chunk.div(min(g1 * kGroupVec, a.num_vec) - 1));
+  const uint32_t kv = a.kv_dim;
+  const uint32_t ppl = static_cast<uint32_t>(a.ptrs_per_layer);
+  for (uint32_t i = tid; i < a.items.d; i += kThreads) {
+    const uint32_t l = kv == 1 ? i : i >> 1;
+    const uint32_t k = i - l * kv;
+    s_item[2 * i] = static_cast<int64_t>(a.layer_ptr[l * ppl + k * (ppl - 1)]) +
+                    static_cast<int64_t>(k) * a.gpu_kv_stride;
+    s_item[2 * i + 1] = static_cast<int64_t>(l) * a.cpu_layer_stride +
+                        static_cast<int64_t>(k) * a.cpu_kv_stride;
+  }
+  for (uint32_t j = tid; j <= b1 - b0; j += kThreads) {
+    const uint32_t b = b0 + j;
+    int64_t gid, cid;
+    if (a.inline_n) {
+      gid = a.inline_ids[2 * b];
+      cid = a.inline_ids[2 * b + 1];
+    } else if (a.ids_split) {
+      gid = a.ids[b];
+      cid = a.ids[static_cast<uint32_t>(a.ids_split) + b];
+    } else {
+      gid = a.ids[2 * static_cast<int64_t>(b)];
+      cid = a.ids[2 * static_cast<int64_t>(b) + 1];
+    }
+    s_block[2 * j] = gid * a.gpu_block_stride;
+    s_block[2 * j + 1] = cid * a.cpu_block_stride;
+  }
+  __syncthreads();
+  for (uint32_t g = g0 + wave; g < g1; g += kWaves) {
+    const uint32_t v0 = g * kGroupVec + lane;
+    const char* src[kU];
+    char* dst[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      // past the end a lane reloads the last vector and stores nothing
+      const uint32_t v = min(v0 + u * 64, a.num_vec - 1);
+      const uint32_t c = a.chunk.div(v);
+      const uint32_t b = a.items.div(c);
+      const uint32_t item = c - b * a.items.d;
+      const int64_t off = static_cast<int64_t>(v - c * a.chunk.d) * 16;
+      char* gpu = reinterpret_cast<char*>(s_item[2 * item] + s_block[2 * (b - b0)] + off);
+      char* cpu = a.cpu_base + s_item[2 * item + 1] + s_block[2 * (b - b0) + 1] + off;
+      src[u] = kH2D ? cpu : gpu;
+      dst[u] = kH2D ? gpu : cpu;
+    }
+    u32x4 v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) v[u] = __builtin_nontemporal_load((const gvec*)src[u]);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (v0 + u * 64 < a.num_vec) {
+        if (kH2D)
+          __builtin_nontemporal_store(v[u], (gvec*)dst[u]);
+        else
+          store_system(dst[u], v[u]);
+      }
+    }
+  }
+}
+
 // Copies a transfer's (gpu_id, cpu_id) pairs from the pinned buffer into a
 // device buffer laid out [gpu ids | cpu ids], n entries each, which the
 // staging kernels then read with ids_split = n.
@@ -688,7 +706,6 @@ struct SmallArgs {
 // both addresses arrive in one round.
 template <bool kH2D>
 __global__ __launch_bounds__(kThreads) void kv_small_copy_kernel(SmallArgs a) {
-  constexpr bool kNtStore = kH2D ? FKV_NT_STORE_HBM : FKV_NT_STORE_HOST;
   constexpr int kU = small_rows_per_wave<kH2D>();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -708,10 +725,10 @@ __global__ __launch_bounds__(kThreads) void kv_small_copy_kernel(SmallArgs a) {
   for (int u = 0; u < kU; ++u) {
     const int vi = (u * kWaves + wave) * 64 + lane;
     if (vi < n) {
-      if (kNtStore)
+      if (kH2D)
         __builtin_nontemporal_store(v[u], dst + vi);
       else
-        dst[vi] = v[u];
+        store_system(reinterpret_cast<char*>(a.dst[w]) + static_cast<int64_t>(vi) * 16, v[u]);
     }
   }
 }
@@ -721,22 +738,9 @@ std::mutex g_init_mu;
 // ---------------------------------------------------------------------------
 // Host-side policy of the transfer paths
 
-// Compute units of the zero-copy kernel when the caller passes -1: enough
-// loads/stores in flight to saturate the PCIe Gen5 x16 link (measured on
-// MI355X: 8 CUs reach the link's copy rate; more add contention).
-constexpr int kAutoZeroCopyCus = 8;
-// The whole-group variant of the device-to-host zero-copy kernel fills the
-// link with fewer compute units and loses rate with more (MI355X, Llama-3-8B
-// shape, 2 GiB: 56.4 / 56.7 / 56.2 / 55.8 GB/s on 3 / 4 / 6 / 8 CUs, against
-// 56.6 GB/s for the row-by-row variant on 8), for calls of at least
-// kZeroCopyFewCusMinBytes.
-constexpr int kAutoZeroCopyCusWholeD2H = 4;
-// Layer-wise host-to-device transfers run beside the caller's compute.  Two
-// CUs still fill the link for reads from host memory (56.9 vs 57.2 GB/s with
-// 8) and leave the rest of the chip to the compute kernels: a 32-layer
-// Llama-3-8B load overlapped with per-layer GEMMs finishes in 42.8 ms on 2
-// CUs against 46.1 ms on 8.
-constexpr int kAutoLayerwiseH2DCus = 2;
+// Compute units whose workgroups the small-transfer kernel may fill when the
+// caller passes -1.
+constexpr int kAutoSmallCus = 8;
 // Copy-engine size policy: smallest transfer, and smallest bytes per engine
 // copy, worth handing to the SDMA engines (ce_pays_off).  Measured on MI355X
 // (block-wise host caches, random ids, GB/s zero-copy kernel / engines): the
@@ -798,9 +802,9 @@ int64_t layer_run_bytes(bool h2d) {
 // was queued); not a hipError_t value
 constexpr int kSdmaUnavailable = -1000;
 
-template <bool H, bool I, bool W = false>
-void* kernel_ptr() {
-  return reinterpret_cast<void*>(&kv_chunk_copy_kernel<H, I, W>);
+template <bool H, bool W = false>
+void* staging_kernel_ptr() {
+  return reinterpret_cast<void*>(&kv_chunk_copy_kernel<H, W>);
 }
 
 int ensure_device_basics(int dev) {
@@ -815,18 +819,20 @@ int ensure_device_basics(int dev) {
   FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
       &o, reinterpret_cast<void*>(&kv_small_copy_kernel<true>), kThreads, 0));
   d.occ_small[1] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel_ptr<false, false>(), kThreads, 0));
+  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      &o, reinterpret_cast<void*>(&kv_zero_copy_kernel<false>), kThreads, 0));
   d.occ_zero_copy[0] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel_ptr<true, false>(), kThreads, 0));
+  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      &o, reinterpret_cast<void*>(&kv_zero_copy_kernel<true>), kThreads, 0));
   d.occ_zero_copy[1] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel_ptr<false, true>(), kThreads, 0));
+  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<false>(), kThreads, 0));
   d.occ_staged[0] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel_ptr<true, true>(), kThreads, 0));
+  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<true>(), kThreads, 0));
   d.occ_staged[1] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel_ptr<false, true, true>(),
+  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<false, true>(),
                                                        kThreads, 0));
   d.occ_whole[0] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, kernel_ptr<true, true, true>(),
+  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<true, true>(),
                                                        kThreads, 0));
   d.occ_whole[1] = std::max(1, o);
   d.init = true;
@@ -879,8 +885,7 @@ int stage_ids_on_device(const IdBuf& ids, int n, int dev, hipStream_t stream, De
 // per slot is the best shape (6.0 TB/s with whole-group addressing; 4 and 8
 // tiles per slot 5.93 / 6.00, 32 tiles 5.44).
 //
-// `balanced` (the HBM-bound staging kernels): a workgroup's wavefronts take
-// the tile's unrolled row groups in turn, so a tile whose rows are not a
+// A workgroup's wavefronts take the tile's unrolled row groups in turn, so a tile whose rows are not a
 // multiple of kWaves * unroll leaves some wavefronts idle while the others
 // finish (a one-layer Llama-3-8B tile, 64 rows, keeps two of four busy; a
 // one-layer MLA tile, 72 rows, fills 56% of the group slots).  The layer
@@ -891,11 +896,9 @@ int stage_ids_on_device(const IdBuf& ids, int n, int dev, hipStream_t stream, De
 //
 // A transfer too small for that many tiles even one (block, layer) per tile
 // splits each tile's rows into up to `factor`-filling ranges of at least one
-// `unroll`-row group per wavefront, so more wavefronts share its few chunks:
-// one block of one layer moves in one round of loads instead of several
-// (zero-copy latency is bound by PCIe round trips).
+// `unroll`-row group per wavefront, so more wavefronts share its few chunks.
 void choose_tiles(int nb, int nl, int kv, int rpc, int grid_cap, int factor, int unroll,
-                  bool balanced, CopyArgs* a) {
+                  CopyArgs* a) {
   const int64_t target = factor * static_cast<int64_t>(std::max(1, grid_cap));
   auto tiles = [&](int tb, int tl) {
     return static_cast<int64_t>((nb + tb - 1) / tb) * ((nl + tl - 1) / tl);
@@ -911,7 +914,7 @@ void choose_tiles(int nb, int nl, int kv, int rpc, int grid_cap, int factor, int
   int tb = 1, tl = nl;
   while (tl > 1 && tiles(tb, tl) < target) {
     const int half = (tl + 1) / 2;
-    if (balanced && fill_below(rows_of(tb, half), rows_of(tb, tl))) break;
+    if (fill_below(rows_of(tb, half), rows_of(tb, tl))) break;
     tl = half;
   }
   while (tb < kMaxTileBlocks && tiles(tb * 2, tl) >= target) tb *= 2;
@@ -921,10 +924,8 @@ void choose_tiles(int nb, int nl, int kv, int rpc, int grid_cap, int factor, int
   const int64_t tile_rows = static_cast<int64_t>(tb) * tl * kv * rpc;
   int64_t tr = 1, split = tile_rows;
   if (t < target) {
-    const int64_t min_split = wave_groups;
-    const int64_t quantum = balanced ? wave_groups : unroll;
-    tr = std::min<int64_t>(std::max<int64_t>(1, tile_rows / min_split), (target + t - 1) / t);
-    split = ((tile_rows + tr - 1) / tr + quantum - 1) / quantum * quantum;
+    tr = std::min<int64_t>(std::max<int64_t>(1, tile_rows / wave_groups), (target + t - 1) / t);
+    split = ((tile_rows + tr - 1) / tr + wave_groups - 1) / wave_groups * wave_groups;
     tr = (tile_rows + split - 1) / split;
   }
   a->tile_blocks = tb;
@@ -940,33 +941,13 @@ int64_t op_bytes(const Geometry& g) {
   return static_cast<int64_t>(g.num_blocks) * g.num_layers * g.kv * g.chunk;
 }
 
-// Whether the zero-copy launches of a transfer take the whole-group kernel
-// variant (launch_copy: full 1 KiB rows, chunks of whole sub-groups).
-// Host-to-device calls under kZeroCopyWholeH2DMinBytes keep the row-by-row
-// variant, which measured faster on short calls and slower on long ones
-// (MI355X, Llama-3-8B chunks, kernel mode, whole-group against row by row:
-// 1 block, 2 MiB, 34.4-34.6 against 35.6-36.1 GB/s; 16 blocks x 1 layer,
-// 36.2-36.7 against 34.5-34.7 us per call; 16 MiB equal; 64 MiB 56.33
-// against 56.21-56.22 GB/s; 2 GiB 57.34-57.35 against 57.19-57.20).
-constexpr int64_t kZeroCopyWholeH2DMinBytes = int64_t(32) << 20;
-bool zero_copy_whole(const Geometry& g, bool h2d) {
-  const int64_t sub_rows = h2d ? FKV_UNROLL_ZC_H2D / whole_sub_groups<true, false>()
-                               : FKV_UNROLL_ZC_D2H / whole_sub_groups<false, false>();
-  return FKV_WHOLE_ZERO_COPY && g.chunk % (64 * 16) == 0 &&
-         (g.chunk / (64 * 16)) % sub_rows == 0 &&
-         (!h2d || op_bytes(g) >= kZeroCopyWholeH2DMinBytes);
-}
-
-// Compute units of a zero-copy transfer when the caller passes -1.
-// The whole-group device-to-host kernel's fewer compute units pay from this
-// many bytes per call; below it the ramp of a short call wants more (MI355X,
-// 4 / 8 / 16 CUs: 16 MiB ops 51.3 / 52.1 / 52.8 GB/s, 32 MiB 53.6 / 53.9 /
-// 53.9, 2 GiB 56.7 / 55.6 / 55.2).
-constexpr int64_t kZeroCopyFewCusMinBytes = int64_t(64) << 20;
-int auto_zero_copy_cus(const Geometry& g, bool h2d) {
-  return !h2d && zero_copy_whole(g, h2d) && op_bytes(g) >= kZeroCopyFewCusMinBytes
-             ? kAutoZeroCopyCusWholeD2H
-             : kAutoZeroCopyCus;
+// Workgroups of a zero-copy transfer on device `d`: the fastest count, within
+// `transfer_cus` compute units when the caller bounds them.
+int zero_copy_grid(const DeviceState& d, int transfer_cus, bool h2d) {
+  const int best = h2d ? zero_copy_workgroups<true>() : zero_copy_workgroups<false>();
+  return transfer_cus <= 0 ? best
+                           : std::min(best, std::min(transfer_cus, d.num_cus) *
+                                                d.occ_zero_copy[h2d ? 1 : 0]);
 }
 
 // The packed-row kernel for a staging launch of chunks of `rpc` full rows:
@@ -1028,29 +1009,27 @@ void launch_pack_span(const PackArgs& pa, hipStream_t stream, hipEvent_t ea, hip
                         kPackLdsOneGroup, stream, ea, eb, 0, pa);
 }
 
-// Fill the per-launch part of CopyArgs and launch over `nb` blocks starting at
+// Launch the staging gather / scatter over `nb` blocks starting at
 // block `b0` of the (already packed) id list, for GPU layers [l0, l0 + nl).
 // `cpu_base` is the CPU-side address of launch layer 0 of block index 0.
 // `ids` holds the packed pairs: `host` for the host's view, `dev` for the
 // device's (the same pinned buffer).  With `split` > 0, `dev` instead holds
 // the gpu ids and, `split` entries later, the cpu ids (device memory), and
 // `host` is null.  `grid_cap` is compute units x occupancy of the kernel the
-// launch takes; staging launches that take the whole-group variant use
-// `whole_grid_cap` instead when it is given.  `done` (zero-copy launches
-// with profiling off): an event the launch completes, carried by the kernel's
-// own packet instead of a marker behind it.
-template <bool kH2D, bool kIota>
-int launch_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int64_t cks, int64_t cls,
+// launch takes; launches that take the whole-group variant use
+// `whole_grid_cap` instead when it is given.
+template <bool kH2D>
+int launch_staging(const Geometry& g, const IdBuf& ids, char* cpu_base, int64_t cks, int64_t cls,
                 int64_t cbs, int b0, int nb, int l0, int nl, int grid_cap,
                 hipStream_t stream, ProfRecorder& prof, int32_t split = 0,
-                int whole_grid_cap = 0, hipEvent_t done = nullptr) {
+                int whole_grid_cap = 0) {
   if (nl < 1 || static_cast<int64_t>(nl) * g.ptrs_per_layer > kMaxLayersPerLaunch)
     return fail(kInval, "internal: a launch of %d layers exceeds the %d layer pointers of the "
                 "kernel arguments", nl, kMaxLayersPerLaunch / g.ptrs_per_layer);
   // Staging launches whose packed side is contiguous in row order, with full
   // rows and ids in device memory, take kv_pack_kernel or kv_pack_span_kernel
   // where pack_shape says so.
-  if constexpr (kIota) {
+  {
     const int64_t rpc = g.chunk / (64 * 16);
     const bool packed_rows = FKV_PACK_KERNEL && split > 0 && g.chunk % (64 * 16) == 0 &&
                              (g.kv == 1 || cks == g.chunk) && cls == g.kv * g.chunk &&
@@ -1118,42 +1097,106 @@ int launch_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int64_t cks
   a.ptrs_per_layer = g.ptrs_per_layer;
   for (int i = 0; i < nl * g.ptrs_per_layer; ++i)
     a.layer_ptr[i] = reinterpret_cast<uint64_t>(g.layer_ptrs[l0 * g.ptrs_per_layer + i]);
-  constexpr int kLaunchUnroll = kIota ? (kH2D ? FKV_UNROLL_SCATTER : kUnrollHbm)
-                                     : (kH2D ? FKV_UNROLL_ZC_H2D : FKV_UNROLL_ZC_D2H);
-  // staging launches whose chunks are whole groups of full rows take the
-  // kernel variant that addresses each group from one base; its occupancy
-  // sizes the tiling
-  constexpr int kStagedUnroll = kH2D ? FKV_UNROLL_SCATTER : kUnrollHbm;
+  // launches whose chunks are whole groups of full rows take the kernel
+  // variant that addresses each group from one base; its occupancy sizes the
+  // tiling
+  constexpr int kUnroll = kH2D ? FKV_UNROLL_SCATTER : kUnrollHbm;
   const bool whole_variant =
       kH2D ? (FKV_WHOLE_SCATTER &&
               static_cast<int64_t>(nb) * nl * g.kv * g.chunk <= kWholeScatterMaxBytes)
            : FKV_WHOLE_GATHER;
-  // zero-copy launches whose chunks are whole groups of the launch's unroll
-  // take it too (FKV_WHOLE_ZERO_COPY)
-  const bool whole = kIota ? a.chunk_vec % 64 == 0 && whole_variant &&
-                                 a.rows_per_chunk % kStagedUnroll == 0
-                           : zero_copy_whole(g, kH2D);
+  const bool whole = a.chunk_vec % 64 == 0 && whole_variant && a.rows_per_chunk % kUnroll == 0;
   if (whole && whole_grid_cap > 0) grid_cap = whole_grid_cap;
   choose_tiles(nb, nl, g.kv, a.rows_per_chunk, grid_cap,
-               kIota ? (kH2D ? FKV_TILE_FACTOR_SCATTER : FKV_TILE_FACTOR_HBM) : FKV_TILE_FACTOR,
-               kLaunchUnroll, /*balanced=*/kIota, &a);
-  a.block_major = kIota && (kH2D ? FKV_BLOCK_MAJOR_SCATTER : FKV_BLOCK_MAJOR_GATHER);
-  int grid = std::max(1, std::min(grid_cap, a.num_tiles));
-  if (kIota && FKV_HBM_ONEPASS) grid = a.num_tiles;
+               kH2D ? FKV_TILE_FACTOR_SCATTER : FKV_TILE_FACTOR_HBM, kUnroll, &a);
+  a.block_major = kH2D ? FKV_BLOCK_MAJOR_SCATTER : FKV_BLOCK_MAJOR_GATHER;
+  const int grid = FKV_HBM_ONEPASS ? a.num_tiles : std::max(1, std::min(grid_cap, a.num_tiles));
   hipEvent_t ea = nullptr, eb = nullptr;
   int rc = prof.kernel_events(&ea, &eb);
   if (rc) return rc;
   prof.kernel_span(ea, eb, static_cast<int64_t>(nb) * nl * g.kv * g.chunk);
-  if (!eb) eb = done;
   (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-  const unsigned lds = kIota ? FKV_HBM_LDS_PAD : 0;
+  const unsigned lds = FKV_HBM_LDS_PAD;
   if (whole)
-    hipExtLaunchKernelGGL((kv_chunk_copy_kernel<kH2D, kIota, true>), dim3(grid), dim3(kThreads),
-                          lds, stream, ea, eb, 0, a);
-  else
-    hipExtLaunchKernelGGL((kv_chunk_copy_kernel<kH2D, kIota>), dim3(grid), dim3(kThreads), lds,
+    hipExtLaunchKernelGGL((kv_chunk_copy_kernel<kH2D, true>), dim3(grid), dim3(kThreads), lds,
                           stream, ea, eb, 0, a);
+  else
+    hipExtLaunchKernelGGL((kv_chunk_copy_kernel<kH2D>), dim3(grid), dim3(kThreads), lds, stream,
+                          ea, eb, 0, a);
   FKV_HIP(hipGetLastError());
+  return 0;
+}
+
+// Launch kv_zero_copy_kernel over call layers [l0, l0 + nl) of every block of
+// the call.  `cpu_base` is the host-side address of call layer 0 of block id
+// 0; ids and `split` as in launch_staging; at most `grid_cap` workgroups a
+// launch.  One launch, but for layers beyond the pointers a launch carries
+// and for runs beyond what Divider or a workgroup's LDS takes.  `done` (null
+// while profiling): an event the last launch completes, carried by its own
+// packet instead of a marker behind it.
+template <bool kH2D>
+int launch_zero_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int l0, int nl,
+                     int grid_cap, hipStream_t stream, ProfRecorder& prof, int32_t split = 0,
+                     hipEvent_t done = nullptr) {
+  constexpr int64_t kGroupVec = zero_copy_rows<kH2D>() * 64;
+  const int64_t chunk_vec = g.chunk / 16;
+  const int64_t part_max = std::min(chunk_vec, kZeroCopyMaxChunkVec);
+  const int lw_max = static_cast<int>(std::min<int64_t>(
+      {nl, g.layers_per_launch(), std::max<int64_t>(1, kZeroCopyMaxVec / (g.kv * part_max))}));
+  ZeroCopyArgs a;
+  for (int lw = l0; lw < l0 + nl; lw += lw_max)
+    for (int64_t off = 0; off < chunk_vec; off += part_max) {
+      const int n_layers = std::min(lw_max, l0 + nl - lw);
+      const int64_t part = std::min(part_max, chunk_vec - off);
+      const int64_t block_vec = n_layers * g.kv * part;
+      for (int b0 = 0; b0 < g.num_blocks;) {
+        // blocks of the launch: as many as its vectors and a run's LDS allow
+        int64_t nb = std::min<int64_t>(g.num_blocks - b0, kZeroCopyMaxVec / block_vec);
+        int64_t groups, per_wg, span;
+        for (;; nb = (nb + 1) / 2) {
+          groups = (nb * block_vec + kGroupVec - 1) / kGroupVec;
+          const int64_t wgs = std::min<int64_t>(std::max(1, grid_cap), (groups + kWaves - 1) / kWaves);
+          per_wg = (groups + wgs - 1) / wgs;
+          span = std::min(nb, per_wg * kGroupVec / block_vec + 2);
+          if (span * 16 <= kZeroCopyMaxLds || nb == 1) break;
+        }
+        a.ids = reinterpret_cast<const int64_t*>(ids.dev) + (split ? 1 : 2) * static_cast<int64_t>(b0);
+        a.ids_split = split;
+        a.inline_n = 0;
+        if (nb <= kInlineIdsZeroCopy && ids.host) {
+          a.inline_n = static_cast<int32_t>(nb);
+          memcpy(a.inline_ids, ids.host + 2 * static_cast<int64_t>(b0), sizeof(int64_t) * 2 * nb);
+        }
+        a.cpu_base = cpu_base + static_cast<int64_t>(lw) * g.cls + off * 16;
+        a.gpu_kv_stride = g.gks;
+        a.gpu_block_stride = g.gbs;
+        a.cpu_kv_stride = g.cks;
+        a.cpu_layer_stride = g.cls;
+        a.cpu_block_stride = g.cbs;
+        a.chunk = Divider(static_cast<uint32_t>(part));
+        a.items = Divider(static_cast<uint32_t>(n_layers * g.kv));
+        a.kv_dim = static_cast<uint32_t>(g.kv);
+        a.num_vec = static_cast<uint32_t>(nb * block_vec);
+        a.num_groups = static_cast<uint32_t>(groups);
+        a.groups_per_wg = static_cast<uint32_t>(per_wg);
+        a.ptrs_per_layer = g.ptrs_per_layer;
+        for (int i = 0; i < n_layers * g.ptrs_per_layer; ++i)
+          a.layer_ptr[i] = reinterpret_cast<uint64_t>(g.layer_ptrs[lw * g.ptrs_per_layer + i]) +
+                           static_cast<uint64_t>(off) * 16;
+        b0 += static_cast<int>(nb);
+        hipEvent_t ea = nullptr, eb = nullptr;
+        int rc = prof.kernel_events(&ea, &eb);
+        if (rc) return rc;
+        prof.kernel_span(ea, eb, nb * block_vec * 16);
+        if (!eb && b0 == g.num_blocks && off + part == chunk_vec && lw + n_layers == l0 + nl)
+          eb = done;
+        (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
+        hipExtLaunchKernelGGL((kv_zero_copy_kernel<kH2D>),
+                              dim3(static_cast<uint32_t>((groups + per_wg - 1) / per_wg)),
+                              dim3(kThreads), static_cast<uint32_t>(span * 16), stream, ea, eb, 0, a);
+        FKV_HIP(hipGetLastError());
+      }
+    }
   return 0;
 }
 
@@ -1208,7 +1251,7 @@ int transfer_small(const Geometry& g, char* cpu_dev, int n_pieces, hipStream_t s
 int transfer_zero_copy(const Geometry& g, hipStream_t stream, int dev, int transfer_cus,
                        bool h2d) {
   DeviceState& d = g_dev[dev];
-  const int small_cus = transfer_cus <= 0 ? std::min(kAutoZeroCopyCus, d.num_cus)
+  const int small_cus = transfer_cus <= 0 ? std::min(kAutoSmallCus, d.num_cus)
                                           : std::min(transfer_cus, d.num_cus);
   if (const int n = small_pieces(g, small_cus * (h2d ? d.occ_small[1] : d.occ_small[0]), h2d)) {
     DrainOnError drain{stream};
@@ -1227,22 +1270,13 @@ int transfer_zero_copy(const Geometry& g, hipStream_t stream, int dev, int trans
   int rc = pack_ids(g, ids);
   if (rc) return rc;
   DrainOnError drain{stream};
-  int cus = transfer_cus <= 0 ? std::min(auto_zero_copy_cus(g, h2d), d.num_cus)
-                              : std::min(transfer_cus, d.num_cus);
-  const int grid_cap = cus * (h2d ? d.occ_zero_copy[1] : d.occ_zero_copy[0]);
+  const int grid_cap = zero_copy_grid(d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff +
                   static_cast<int64_t>(g.start_layer) * g.cls;
   ProfRecorder prof;
-  const int per_launch = g.layers_per_launch();
-  for (int l0 = 0; l0 < g.num_layers; l0 += per_launch) {
-    const int nl = std::min(per_launch, g.num_layers - l0);
-    char* base = cpu_dev + static_cast<int64_t>(l0) * g.cls;
-    rc = h2d ? launch_copy<true, false>(g, ids.buf, base, g.cks, g.cls, g.cbs, 0,
-                                        g.num_blocks, l0, nl, grid_cap, stream, prof)
-             : launch_copy<false, false>(g, ids.buf, base, g.cks, g.cls, g.cbs, 0,
-                                         g.num_blocks, l0, nl, grid_cap, stream, prof);
-    if (rc) return rc;
-  }
+  rc = h2d ? launch_zero_copy<true>(g, ids.buf, cpu_dev, 0, g.num_layers, grid_cap, stream, prof)
+           : launch_zero_copy<false>(g, ids.buf, cpu_dev, 0, g.num_layers, grid_cap, stream, prof);
+  if (rc) return rc;
   FKV_HIP(hipStreamSynchronize(stream));
   drain.armed = false;
   prof.flush();
@@ -1298,7 +1332,7 @@ int transfer_zero_copy_noalloc(const Geometry& g, hipStream_t stream, int dev, i
     return fail(kInval, "fkv_transfer_kv_blocks_noalloc moves at most %d blocks per call "
                 "(its id scratch is %zu bytes), got %d", kScratchMaxBlocks, kScratchBytes,
                 g.num_blocks);
-  const int small_cus = transfer_cus <= 0 ? std::min(kAutoZeroCopyCus, d.num_cus)
+  const int small_cus = transfer_cus <= 0 ? std::min(kAutoSmallCus, d.num_cus)
                                           : std::min(transfer_cus, d.num_cus);
   if (const int n = small_pieces(g, small_cus * (h2d ? d.occ_small[1] : d.occ_small[0]), h2d)) {
     DrainOnError drain{stream};
@@ -1312,13 +1346,13 @@ int transfer_zero_copy_noalloc(const Geometry& g, hipStream_t stream, int dev, i
     drain.armed = false;
     return 0;
   }
-  int64_t pairs[2 * kInlineIds];
+  int64_t pairs[2 * kInlineIdsZeroCopy];
   IdBuf ids;
   int32_t split = 0;
   // Declared before the DrainOnError below, so an error path drains the
   // stream before the next call may overwrite the scratch.
   std::unique_lock<std::mutex> scratch_use(g_scratch_use_mu[dev], std::defer_lock);
-  if (g.num_blocks <= kInlineIds) {
+  if (g.num_blocks <= kInlineIdsZeroCopy) {
     // the ids travel in the kernel arguments
     pack_ids_into(g, pairs);
     ids.host = pairs;
@@ -1336,24 +1370,15 @@ int transfer_zero_copy_noalloc(const Geometry& g, hipStream_t stream, int dev, i
     split = kScratchMaxBlocks;
   }
   DrainOnError drain{stream};
-  const int cus = transfer_cus <= 0 ? std::min(auto_zero_copy_cus(g, h2d), d.num_cus)
-                                    : std::min(transfer_cus, d.num_cus);
-  const int grid_cap = cus * (h2d ? d.occ_zero_copy[1] : d.occ_zero_copy[0]);
+  const int grid_cap = zero_copy_grid(d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
   ProfRecorder prof;
   prof.on = false;   // profiling events are allocations
-  const int per_launch = g.layers_per_launch();
-  for (int l0 = 0; l0 < g.num_layers; l0 += per_launch) {
-    const int nl = std::min(per_launch, g.num_layers - l0);
-    char* base = cpu_dev + static_cast<int64_t>(l0) * g.cls;
-    const int rc = h2d ? launch_copy<true, false>(g, ids, base, g.cks, g.cls, g.cbs, 0,
-                                                  g.num_blocks, l0, nl, grid_cap, stream, prof,
-                                                  split)
-                       : launch_copy<false, false>(g, ids, base, g.cks, g.cls, g.cbs, 0,
-                                                   g.num_blocks, l0, nl, grid_cap, stream, prof,
-                                                   split);
-    if (rc) return rc;
-  }
+  const int rc = h2d ? launch_zero_copy<true>(g, ids, cpu_dev, 0, g.num_layers, grid_cap, stream,
+                                              prof, split)
+                     : launch_zero_copy<false>(g, ids, cpu_dev, 0, g.num_layers, grid_cap, stream,
+                                               prof, split);
+  if (rc) return rc;
   FKV_HIP(hipStreamSynchronize(stream));
   drain.armed = false;
   return 0;
@@ -1592,9 +1617,9 @@ int transfer_staged(const Geometry& g, hipStream_t stream, int dev, bool h2d) {
       cbs = static_cast<int64_t>(p.nl) * cls;
     }
     char* stg = ln.staging + (pi & 1) * half;
-    return h2d ? launch_copy<true, true>(g, kids, stg, cks, cls, cbs, p.b0, p.nb, p.l0, p.nl,
+    return h2d ? launch_staging<true>(g, kids, stg, cks, cls, cbs, p.b0, p.nb, p.l0, p.nl,
                                          grid_cap, stream, prof, kids_split, whole_cap)
-               : launch_copy<false, true>(g, kids, stg, cks, cls, cbs, p.b0, p.nb, p.l0, p.nl,
+               : launch_staging<false>(g, kids, stg, cks, cls, cbs, p.b0, p.nb, p.l0, p.nl,
                                           grid_cap, stream, prof, kids_split, whole_cap);
   };
   if (!h2d) {
@@ -1667,9 +1692,9 @@ int transfer_contiguous(const Geometry& g, hipStream_t stream, int dev, bool to_
   for (int l0 = 0; l0 < g.num_layers; l0 += per_launch) {
     const int nl = std::min(per_launch, g.num_layers - l0);
     char* base = g.cpu_info.dev_ptr + static_cast<int64_t>(l0) * g.cls;
-    rc = to_gpu ? launch_copy<true, true>(g, kids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
+    rc = to_gpu ? launch_staging<true>(g, kids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
                                           l0, nl, grid_cap, stream, prof, kids_split, whole_cap)
-                : launch_copy<false, true>(g, kids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
+                : launch_staging<false>(g, kids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
                                            l0, nl, grid_cap, stream, prof, kids_split,
                                            whole_cap);
     if (rc) return rc;
@@ -1860,10 +1885,7 @@ int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transf
   int rc = ids_acquire(static_cast<size_t>(g.num_blocks) * 16, &h->ids);
   if (rc) return rc;
   pack_ids_into(g, h->ids.host);
-  const int automatic = h2d ? kAutoLayerwiseH2DCus : auto_zero_copy_cus(g, h2d);
-  const int cus = transfer_cus <= 0 ? std::min(automatic, d.num_cus)
-                                    : std::min(transfer_cus, d.num_cus);
-  const int grid_cap = cus * (h2d ? d.occ_zero_copy[1] : d.occ_zero_copy[0]);
+  const int grid_cap = zero_copy_grid(d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
   // Under capture the launches record plain events, as graph nodes.
   const bool captured = stream_captured(stream);
@@ -1889,17 +1911,13 @@ int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transf
     hipEvent_t ev = nullptr;
     FKV_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     h->events.push_back(ev);
-    for (int l0 = grp * granularity; l0 < lend;) {
-      const int nl = std::min(g.layers_per_launch(), lend - l0);
-      char* base = cpu_dev + static_cast<int64_t>(l0) * g.cls;
-      hipEvent_t done = on_kernel && l0 + nl == lend ? ev : nullptr;
-      rc = h2d ? launch_copy<true, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
-                                          l0, nl, grid_cap, stream, h->prof, 0, 0, done)
-               : launch_copy<false, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
-                                           l0, nl, grid_cap, stream, h->prof);
-      if (rc) return rc;
-      l0 += nl;
-    }
+    const int l0 = grp * granularity;
+    hipEvent_t done = on_kernel ? ev : nullptr;
+    rc = h2d ? launch_zero_copy<true>(g, h->ids, cpu_dev, l0, lend - l0, grid_cap, stream, h->prof,
+                                      0, done)
+             : launch_zero_copy<false>(g, h->ids, cpu_dev, l0, lend - l0, grid_cap, stream,
+                                       h->prof);
+    if (rc) return rc;
     if (!on_kernel) FKV_HIP(hipEventRecord(ev, stream));
     h->done.insert(h->done.end(), static_cast<size_t>(take), ev);
     h->null_covers.insert(h->null_covers.end(), static_cast<size_t>(take),
@@ -1998,21 +2016,15 @@ int layerwise_kernel_groups(fkv_transfer_handle_s* h, hipStream_t work, int firs
                             int end_group = -1) {
   const Geometry& g = h->geo;
   DeviceState& d = g_dev[h->dev];
-  const int cus = std::min(kAutoLayerwiseH2DCus, d.num_cus);
-  const int grid_cap = cus * d.occ_zero_copy[1];
+  const int grid_cap = zero_copy_grid(d, -1, true);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
   const int end_layer = end_group < 0 ? g.num_layers
                                       : std::min(g.num_layers, end_group * h->granularity);
   int group = first_group;
   for (int g0 = first_group * h->granularity; g0 < end_layer; g0 += h->granularity, ++group) {
     const int gend = std::min(g.num_layers, g0 + h->granularity);
-    for (int l0 = g0; l0 < gend; l0 += g.layers_per_launch()) {
-      const int nl = std::min(g.layers_per_launch(), gend - l0);
-      char* base = cpu_dev + static_cast<int64_t>(l0) * g.cls;
-      int rc = launch_copy<true, false>(g, h->ids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
-                                        l0, nl, grid_cap, work, h->prof);
-      if (rc) return rc;
-    }
+    int rc = launch_zero_copy<true>(g, h->ids, cpu_dev, g0, gend - g0, grid_cap, work, h->prof);
+    if (rc) return rc;
     FKV_HIP(hipEventRecord(h->done[group], work));
     std::lock_guard<std::mutex> lk(h->mu);
     h->recorded = group + 1;
@@ -2145,7 +2157,7 @@ int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
     const int64_t cls = static_cast<int64_t>(g.kv) * g.chunk;
     const int64_t cbs = static_cast<int64_t>(p.nl) * cls;
     // launch_copy reads the group's layer pointers from call layer p.l0 on
-    if ((rc = launch_copy<true, true>(g, h->ids, ln.staging + hf * half, cks, cls, cbs, p.b0,
+    if ((rc = launch_staging<true>(g, h->ids, ln.staging + hf * half, cks, cls, cbs, p.b0,
                                       p.nb, p.l0, p.nl, grid_cap, work, h->prof, 0,
                                       whole_cap)))
       return rc;

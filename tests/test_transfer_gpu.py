@@ -1206,3 +1206,22 @@ def test_copy_engine_mode_without_sdma(dev, env, fallback):
     assert "match the oracle" in res.stdout
     if fallback:
         assert res.stderr.count("copy engines unavailable") == 1
+
+
+@pytest.mark.parametrize("layout", ["BLOCKWISE", "LAYERWISE"])
+@pytest.mark.parametrize("chunk,n,nl,kv,cus", [
+    (16, 1, 1, 1, -1), (16, 95, 3, 2, -1), (1008, 96, 2, 1, -1), (1040, 97, 3, 2, -1),
+    (4608, 33, 5, 1, -1), (8192, 7, 2, 2, -1), (8208, 131, 1, 2, -1), (2304, 61, 61, 1, 1),
+    (512, 700, 40, 2, -1),
+    # more blocks than one workgroup run's LDS offsets: several launches
+    (16, 9000, 1, 1, 1), (16, 30000, 2, 2, 1)])
+def test_general_kernel_edges(dev, monkeypatch, layout, chunk, n, nl, kv, cus):
+    """The general zero-copy kernel where its rows meet chunk, block, group
+    and launch ends: chunks from one vector to more than a group, id counts
+    around those that travel in the kernel arguments, and more blocks than a
+    launch takes."""
+    monkeypatch.setenv("FLEXKV_SMALL_KERNEL", "0")
+    case = KVCase(layers_total=nl + 1, num_layers=nl, start_layer=1, kv=kv, ng=n + 3, nh=n + 5,
+                  tokens=1, heads=1, dim=chunk // 2, layout=layout).fill(seed=n + chunk)
+    check_case(case, inputs.distinct_ids(n, n, n + 3), inputs.distinct_ids(n + 1, n, n + 5), 0,
+               transfer_cus=cus)
