@@ -1369,9 +1369,8 @@ KERNEL_SECTION_END = b"// A system-scope acquire in every workgroup."
 
 def kernel_section_sha16(path: str = KERNEL_SOURCE) -> str:
     """sha256 prefix of the transfer kernels' source: kv_transfer.hip from its
-    start (build macros, CopyArgs, PackArgs) to the end of the data-moving
-    kernels (kv_chunk_copy_kernel, kv_pack_kernel, kv_pack_span_kernel,
-    stage_ids_kernel), the part that decides which bytes the kernels read and
+    start to the end of the data-moving kernels (kv_pack_kernel,
+    kv_zero_copy_kernel, stage_table_kernel, kv_small_copy_kernel), the part that decides which bytes the kernels read and
     write.  Comments,
     blank lines and indentation are left out, so a change to a comment keeps
     the key and any change to the code changes it."""
@@ -1758,7 +1757,7 @@ def main() -> int:
                 "median_ms": round(h2d_med * 1e3, 3), "best_ms": round(h2d_best * 1e3, 3)},
         "bit_exact": parity and gather_ok,
         "roofline": {"bound": "hbm",
-                     "kernel": "kv_chunk_copy_kernel<D2H, staging>: device-side gather of the "
+                     "kernel": "kv_pack_kernel<D2H, 32>: device-side gather of the "
                                "step's blocks into one packed HBM buffer",
                      "achieved": round(g_rate, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(g_rate / HBM_PEAK_GBS, 4),

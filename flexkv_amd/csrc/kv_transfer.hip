@@ -12,15 +12,9 @@
 //     (queued through HSA) then move maximal contiguous host runs between
 //     that buffer and the host cache.
 //
-// Staging work decomposition (kv_chunk_copy_kernel): a workgroup (4
-// wavefronts) owns a tile of consecutive blocks; it stages the tile's ids in
-// LDS, then its wavefronts stream the tile's rows (64 lanes x 16 B = 1 KiB)
-// in groups of kUnroll rows, issuing all loads of a group before any store.
-// Rows are ordered block -> layer -> K|V -> offset.  Layer base pointers
-// travel in the kernel argument block.  Gathers whose chunks are whole groups
-// of 32 rows address each group from one buffer resource per side instead of
-// a 64-bit base per row; kv_pack_kernel and kv_pack_span_kernel take the other
-// shapes of whole rows.
+// Staging work decomposition (kv_pack_kernel): the staging buffer's bytes are
+// one contiguous sequence, cut into groups of kU rows (64 lanes x 16 B = 1 KiB)
+// with a wavefront each, whatever the chunk size.
 //
 // This file holds the kernels, the transfer paths that launch them and the
 // transfer entry points of the C ABI; kv_host.cpp holds validation, id staging
@@ -48,449 +42,164 @@ using namespace fkv_detail;
 
 namespace {
 
-// Rows (64 lanes x 16 B) each wavefront of the staging kernels keeps in
-// flight.
-#ifndef FKV_UNROLL_HBM
-#define FKV_UNROLL_HBM 32
-#endif
-// Staging gather/scatter launch shape: 1 = one workgroup per tile (grid =
-// tiles), 0 = an occupancy-sized grid looping over tiles.
-#ifndef FKV_HBM_ONEPASS
-#define FKV_HBM_ONEPASS 1
-#endif
-// Tiles per occupancy slot the staging tiling aims for.
-#ifndef FKV_TILE_FACTOR_HBM
-#define FKV_TILE_FACTOR_HBM 16
-#endif
-// Staging gather / scatter: chunks of whole row groups take the kernel
-// variant that addresses each group from one base (1) or the row-by-row one
-// (0).  The whole-group variant keeps no per-row address and spills nothing.
-// Measured on MI355X at the Llama-3-8B shape (TB/s of HBM traffic by launch
-// size 128 MiB / 256 MiB / 512 MiB / 2 GiB): gather 5.41/5.71/5.89/6.07
-// against 5.46/5.67/5.89/6.05 row by row; scatter 4.67/4.97/5.08/5.26
-// against 4.01/4.67/5.10/5.42.  So the scatter takes the whole-group
-// variant up to kWholeScatterMaxBytes per launch and the row-by-row one
-// above, where kv_pack_span_kernel does not take it (a packed side that is
-// not contiguous in row order; pack_shape).
-#ifndef FKV_WHOLE_GATHER
-#define FKV_WHOLE_GATHER 1
-#endif
-#ifndef FKV_WHOLE_SCATTER
-#define FKV_WHOLE_SCATTER 1
-#endif
 // Cache hints: loads are non-temporal everywhere, and so are stores into HBM
 // (stores into host memory: store_system).
-#ifndef FKV_NT_LOAD
-#define FKV_NT_LOAD 1
-#endif
-#ifndef FKV_NT_STORE_HBM
-#define FKV_NT_STORE_HBM 1
-#endif
-// The staging scatter (packed HBM -> scattered chunks) has its own knobs.
-#ifndef FKV_UNROLL_SCATTER
-#define FKV_UNROLL_SCATTER FKV_UNROLL_HBM
-#endif
-#ifndef FKV_TILE_FACTOR_SCATTER
-#define FKV_TILE_FACTOR_SCATTER FKV_TILE_FACTOR_HBM
-#endif
-// Staging gather/scatter: hand each XCD a contiguous range of tiles instead
-// of every eighth tile (workgroups are dispatched to the 8 XCDs round robin).
-#ifndef FKV_XCD_REMAP
-#define FKV_XCD_REMAP 0
-#endif
-// Tile order of the staging gather / scatter: 1 = block-major (consecutive
-// workgroups take the layer windows of one block, so the packed side is
-// walked in address order), 0 = layer-window-major (consecutive workgroups
-// take one layer window of consecutive blocks).
-#ifndef FKV_BLOCK_MAJOR_GATHER
-#define FKV_BLOCK_MAJOR_GATHER 0
-#endif
-#ifndef FKV_BLOCK_MAJOR_SCATTER
-#define FKV_BLOCK_MAJOR_SCATTER 0
-#endif
-// Dynamic LDS per staging workgroup (bytes), to cap its occupancy.
-#ifndef FKV_HBM_LDS_PAD
-#define FKV_HBM_LDS_PAD 0
-#endif
-#ifndef FKV_NT_LOAD_SCATTER
-#define FKV_NT_LOAD_SCATTER FKV_NT_LOAD
-#endif
-#ifndef FKV_NT_STORE_SCATTER
-#define FKV_NT_STORE_SCATTER FKV_NT_STORE_HBM
-#endif
-
 constexpr int kThreads = 256;               // 4 wavefronts of 64 lanes
-constexpr int64_t kWholeScatterMaxBytes = int64_t(512) << 20;
 constexpr int kWaves = kThreads / 64;
-constexpr int kUnrollHbm = FKV_UNROLL_HBM;
-constexpr int kMaxTileBlocks = 64;
 // Launches of at most this many blocks carry their (gpu_id, cpu_id) pairs in
 // the kernel arguments, so no workgroup reads them over PCIe first (one host
 // round trip less per launch).
-constexpr int kInlineIds = 32;
 constexpr int kInlineIdsZeroCopy = 96;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-// Buffer resource word 3 for raw (unformatted, unswizzled) buffers on gfx9
-// parts, and the cache-policy bit of buffer instructions meaning
-// non-temporal on gfx94x/gfx950 (bit 1; bit 0 = sc0, bit 4 = sc1).
-constexpr int kBufferRsrcWord3 = 0x00020000;
-constexpr int kCachePolicyNt = 2;
 // Every address the kernel touches is global memory (HBM or mapped pinned
 // host memory); saying so lets the compiler emit global_* instead of flat_*.
 typedef __attribute__((address_space(1))) u32x4 gvec;
 
-struct CopyArgs {
-  const int64_t* ids;        // device-visible (gpu_id, cpu_id) pairs (inline_n == 0)
-  char* cpu_base;            // CPU side of launch layer 0, block index 0
-  int64_t gpu_kv_stride;
-  int64_t gpu_block_stride;
-  int64_t cpu_kv_stride;
-  int64_t cpu_layer_stride;
-  int64_t cpu_block_stride;
-  int64_t chunk_vec;         // 16-byte vectors per chunk
-  int32_t rows_per_chunk;    // ceil(chunk_vec / 64)
-  int32_t num_blocks;
-  int32_t num_layers;        // layers in this launch (<= kMaxLayersPerLaunch)
-  int32_t kv_dim;
-  int32_t tile_blocks;       // a tile is tile_blocks blocks x tile_layers layers
-  int32_t tile_layers;
-  int32_t tiles_b;           // tiles along the block axis
-  int32_t tiles_l;           // tiles along the layer axis
-  int32_t block_major;       // tile order: layer windows of a block are consecutive tiles
-  int32_t tiles_r;           // row ranges per tile (small transfers split a tile's rows)
-  uint32_t split_rows;       // rows per range: a whole tile, or a multiple of the unroll
-  int32_t num_tiles;
-  int32_t ptrs_per_layer;    // 1: layer_ptr[l] + k*gpu_kv_stride; kv: layer_ptr[l*kv + k]
-  int32_t inline_n;          // > 0: the launch's pairs are inline_ids, not ids
-  int32_t ids_split;         // > 0: ids holds gpu ids, and cpu ids ids_split entries later
-  uint64_t layer_ptr[kMaxLayersPerLaunch];
-  int64_t inline_ids[2 * kInlineIds];
+// n / d for n < 2^31 as a multiplication (Granlund and Montgomery, "Division
+// by Invariant Integers using Multiplication", 1994): with 2^(l-1) < d <= 2^l,
+// mul = ceil(2^(31+l) / d) < 2^32 and n / d = floor(n * mul / 2^(31+l)).
+struct Divider {
+  uint32_t d = 1, mul = 0, shift = 0;
+  explicit Divider(uint32_t by = 1) : d(by) {
+    int l = 0;
+    while ((uint64_t(1) << l) < by) ++l;
+    shift = static_cast<uint32_t>(31 + l);
+    mul = static_cast<uint32_t>(((static_cast<unsigned __int128>(1) << shift) + by - 1) / by);
+  }
+  __device__ uint32_t div(uint32_t n) const {
+    return static_cast<uint32_t>((static_cast<uint64_t>(n) * mul) >> shift);
+  }
 };
 
-// A value every lane of the wavefront holds, moved to a scalar register.
-__device__ inline int64_t wave_uniform(int64_t x) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(x));
-  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(x) >> 32));
-  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
-}
+// The staging gather / scatter.  The packed (staging) side is contiguous: the
+// launch's chunks in order, block -> layer -> K|V or layer -> K|V -> block.
+// Its 16-byte vectors are cut into groups of kU rows of 64 and wavefront w of
+// workgroup b moves group 4b + w (b in column order, launch_pack): no tile, no
+// LDS, no barrier, and every wavefront moves a full group.  Lane j first resolves the address of the
+// group's j-th chunk (a group touches at most 64, pack_fits), so ids and layer
+// pointers cost one round of loads a group whatever the chunk size; each row
+// then picks the chunk of each lane's vector out of those registers
+// (ds_bpermute), so rows that cross chunks (sizes that are not whole KiB, or
+// under one) leave no lane idle.  The scattered address is used in one of the
+// two walks only, so nothing but the loaded data is held between them.
+//
+// HBM bounds the large launches and the launch the small ones.  Measured on
+// MI355X, us a gather / scatter call, against a kernel per chunk shape (tiled
+// groups, 2-5 bases a group, a row-by-row one) with the ids staged by a launch
+// of their own: 2 GiB of 32 KiB chunks 727 / 808 -> 706 / 796, 1 GiB of 4 KiB
+// 383 / 440 -> 379 / 416, 1 GiB of 2 KiB 462 / 462 -> 381 / 413, 47 MiB of 2
+// KiB 57.2 / 57.0 -> 38.0 / 40.1, 64 MiB of 512 B 79.4 / 78.7 -> 47.2 / 46.3,
+// 1 MiB of 32 KiB 18.8 / 20.6 -> 15.2 / 14.6.
+constexpr int kPackInlineIds = 256;
+// vectors of a launch: Divider takes numbers below 2^31, the last group's
+// positions beyond the end included
+constexpr int64_t kPackMaxVec = int64_t(1) << 30;
 
-// Staging gather (kH2D false: GPU cache -> packed buffer, the "CPU side") or
-// scatter (kH2D true).  Block i of the launch sits at CPU-side block index i.
-// Row addresses are wave-uniform (scalar registers); each lane adds its own
-// 16-byte slot, so one 32-bit lane offset serves every access.
-// kWhole: the launch's chunks are whole groups of kUnroll full rows, so each
-// group lies inside one chunk and is addressed from one base per side.
-template <bool kH2D, bool kWhole = false>
-__global__ __launch_bounds__(kThreads) void kv_chunk_copy_kernel(CopyArgs a) {
-  constexpr int kUnroll = kH2D ? FKV_UNROLL_SCATTER : kUnrollHbm;
-  constexpr bool kNtStore = kH2D ? FKV_NT_STORE_SCATTER : FKV_NT_STORE_HBM;
-  constexpr bool kNtLoad = kH2D ? FKV_NT_LOAD_SCATTER : FKV_NT_LOAD;
-  __shared__ int64_t s_gid[kMaxTileBlocks];
-
-  const int lane = threadIdx.x & 63;
-  const uint32_t lane_off = static_cast<uint32_t>(lane) * 16;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t kv = static_cast<uint32_t>(a.kv_dim);
-  const uint32_t rpc = static_cast<uint32_t>(a.rows_per_chunk);
-  const uint32_t ppl = static_cast<uint32_t>(a.ptrs_per_layer);
-  // true when every row of a chunk is a full 64-lane row
-  const bool full_rows = (a.chunk_vec & 63) == 0;
-
-  int first = blockIdx.x;
-  if (FKV_XCD_REMAP && (gridDim.x & 7) == 0) {
-    const int per = gridDim.x >> 3;
-    first = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  }
-  for (int tile = first; tile < a.num_tiles; tile += gridDim.x) {
-    const int tr = tile % a.tiles_r;
-    const int tq = tile / a.tiles_r;
-    const int tb = a.block_major ? tq / a.tiles_l : tq % a.tiles_b;
-    const int tl = a.block_major ? tq % a.tiles_l : tq / a.tiles_b;
-    const int b0 = tb * a.tile_blocks;
-    const int nb = min(a.tile_blocks, a.num_blocks - b0);
-    const int l0 = tl * a.tile_layers;
-    const uint32_t nl = static_cast<uint32_t>(min(a.tile_layers, a.num_layers - l0));
-    const uint32_t items_per_block = nl * kv;
-    __syncthreads();  // previous tile's readers are done with the LDS ids
-    if (threadIdx.x < nb) {
-      const int j = b0 + threadIdx.x;
-      s_gid[threadIdx.x] = a.inline_n    ? a.inline_ids[2 * j]
-                           : a.ids_split ? a.ids[j]
-                                         : a.ids[2 * static_cast<int64_t>(j)];
-    }
-    __syncthreads();
-
-    // this workgroup's rows of the tile: [g_begin, g_end)
-    const uint32_t rows = static_cast<uint32_t>(nb) * items_per_block * rpc;
-    const uint32_t g_begin = static_cast<uint32_t>(tr) * a.split_rows;
-    const uint32_t g_end = min(rows, g_begin + a.split_rows);
-    if constexpr (kWhole) {
-      for (uint32_t g = g_begin + static_cast<uint32_t>(wave) * kUnroll; g < g_end;
-           g += kWaves * kUnroll) {
-        // Raw buffer accesses: the group's base in a buffer resource (scalar
-        // registers), the lane's 16-byte slot as the vector offset and the
-        // row as a scalar offset, so no per-row 64-bit address is kept.
-        const uint32_t item = g / rpc;
-        const uint32_t rr = g - item * rpc;
-        const uint32_t bi = item / items_per_block;
-        const uint32_t rem = item - bi * items_per_block;
-        const uint32_t l = rem / kv;
-        const uint32_t k = rem - l * kv;
-        const uint32_t layer = static_cast<uint32_t>(l0) + l;
-        const int64_t gid = wave_uniform(s_gid[bi]);
-        const int64_t row_off = static_cast<int64_t>(rr) * (64 * 16);
-        char* gpu = reinterpret_cast<char*>(a.layer_ptr[layer * ppl + k * (ppl - 1)]) +
-                    static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride + row_off;
-        char* cpu = a.cpu_base + static_cast<int64_t>(layer) * a.cpu_layer_stride +
-                    static_cast<int64_t>(k) * a.cpu_kv_stride +
-                    static_cast<int64_t>(b0 + static_cast<int>(bi)) * a.cpu_block_stride + row_off;
-        const __amdgpu_buffer_rsrc_t rs =
-            __builtin_amdgcn_make_buffer_rsrc(kH2D ? cpu : gpu, 0, -1, kBufferRsrcWord3);
-        const __amdgpu_buffer_rsrc_t rd =
-            __builtin_amdgcn_make_buffer_rsrc(kH2D ? gpu : cpu, 0, -1, kBufferRsrcWord3);
-        i32x4 v[kUnroll];
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
-          v[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane_off, u * (64 * 16),
-                                                       kNtLoad ? kCachePolicyNt : 0);
-#pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
-          __builtin_amdgcn_raw_buffer_store_b128(v[u], rd, lane_off, u * (64 * 16),
-                                                 kNtStore ? kCachePolicyNt : 0);
-      }
-    } else {
-      for (uint32_t g = g_begin + static_cast<uint32_t>(wave) * kUnroll; g < g_end;
-           g += kWaves * kUnroll) {
-        // The group's rows are walked twice from the same cursor
-        // over (block, layer, K|V, row), once to issue the loads and once to
-        // issue the stores.  No row address is held between the two walks,
-        // so only the loaded data stays live: holding 2 x U 64-bit row
-        // addresses spilled 358-387 scalar registers at U = 32.
-        const uint32_t item0 = g / rpc;
-        const uint32_t rr0 = g - item0 * rpc;
-        const uint32_t bi0 = item0 / items_per_block;
-        const uint32_t rem0 = item0 - bi0 * items_per_block;
-        const uint32_t lw0 = rem0 / kv;
-        const uint32_t kw0 = rem0 - lw0 * kv;
-        u32x4 v[kUnroll];
-#pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
-          uint32_t rr = rr0, bi = bi0, l = lw0, k = kw0;
-#pragma unroll
-          for (int u = 0; u < kUnroll; ++u) {
-            const uint32_t bsafe = min(bi, static_cast<uint32_t>(nb - 1));
-            const uint32_t layer = static_cast<uint32_t>(l0) + min(l, nl - 1);
-            const int64_t gid = wave_uniform(s_gid[bsafe]);
-            const int64_t row_off = static_cast<int64_t>(rr) * (64 * 16);
-            char* gpu = reinterpret_cast<char*>(a.layer_ptr[layer * ppl + k * (ppl - 1)]) +
-                        static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride +
-                        row_off;
-            char* cpu = a.cpu_base + static_cast<int64_t>(layer) * a.cpu_layer_stride +
-                        static_cast<int64_t>(k) * a.cpu_kv_stride +
-                        static_cast<int64_t>(b0 + static_cast<int>(bsafe)) * a.cpu_block_stride +
-                        row_off;
-            const bool live = (g + u < g_end) &&
-                              (full_rows || static_cast<int64_t>(rr) * 64 + lane < a.chunk_vec);
-            if (live) {
-              if (pass == 0) {
-                const gvec* p = (const gvec*)((kH2D ? cpu : gpu) + lane_off);
-                v[u] = kNtLoad ? __builtin_nontemporal_load(p) : *p;
-              } else {
-                gvec* p = (gvec*)((kH2D ? gpu : cpu) + lane_off);
-                if (kNtStore)
-                  __builtin_nontemporal_store(v[u], p);
-                else
-                  *p = v[u];
-              }
-            }
-            // advance the cursor by one row
-            if (++rr == rpc) {
-              rr = 0;
-              if (++k == kv) {
-                k = 0;
-                if (++l == nl) {
-                  l = 0;
-                  ++bi;
-                }
-              }
-            }
-          }
-        }
-      }
-    }
-  }
-}
-
-// The staging gather / scatter over packed rows.  The packed (staging)
-// side of a launch is contiguous in row order, block -> layer -> K|V ->
-// row, each row 1 KiB, so row r lies at packed + r KiB.  The launch's rows
-// are cut into groups of kU consecutive rows and wavefront w of workgroup b
-// moves group 4b + w: no tile, no LDS, no barrier, and every wavefront moves
-// a full group.  A group is kC whole chunks of kU / kC rows (kC > 1: chunks
-// of 4-16 KiB, e.g. the Llama-3-70B TP-8 shard's 4 KiB) or kU rows inside
-// one chunk (kC == 1: 24 KiB chunks at kU = 24).  The host checks the
-// shape: full 1 KiB
-// rows, whole groups, a contiguous packed side, ids in device memory.
 struct PackArgs {
-  const int64_t* gids;       // device memory: gpu id of launch block i at gids[i]
-  char* packed;              // staging address of launch row 0
+  const int64_t* gids;       // device memory: gpu ids by launch block; null: inline_ids
+  const uint64_t* ptrs;      // device memory: layer pointers; null: layer_ptr
+  char* packed;              // staging address of the launch's first vector
   int64_t gpu_kv_stride;
   int64_t gpu_block_stride;
-  uint32_t rows_per_chunk;
-  uint32_t items_per_block;  // layers x kv of the launch
+  Divider chunk;             // by the vectors of a chunk
+  Divider inner;             // by the chunks of a block, or of a (layer, K|V) when layer_major
+  uint32_t layer_major;
   uint32_t kv_dim;
-  uint32_t num_layers;       // layers of the launch
+  uint32_t num_vec;          // vectors of the launch
+  uint32_t num_chunks;
   uint32_t num_groups;
-  uint32_t num_rows;         // packed rows of the launch
+  Divider columns;           // runs of column_wgs workgroups' groups, taken in turn
+  uint32_t column_wgs;
   int32_t ptrs_per_layer;    // 1: layer_ptr[l] + k*gpu_kv_stride; kv: layer_ptr[l*kv + k]
   uint64_t layer_ptr[kMaxLayersPerLaunch];
+  int64_t inline_ids[kPackInlineIds];
 };
 
-template <bool kH2D, int kU, int kC>
-__global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
-  static_assert(kU % kC == 0, "a group is kC whole chunks");
-  constexpr int kR = kU / kC;                 // rows per chunk when kC > 1
-  constexpr int kRow = 64 * 16;               // bytes per row
-  const uint32_t lane_off = (threadIdx.x & 63) * 16;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t g = blockIdx.x * kWaves + wave;
-  if (g >= a.num_groups) return;
-  const uint32_t kv = a.kv_dim;
-  const uint32_t ppl = static_cast<uint32_t>(a.ptrs_per_layer);
-  // the group's first chunk and its first row inside that chunk
-  uint32_t c, rr;
-  if constexpr (kC > 1) {
-    c = g * kC;
-    rr = 0;
-  } else {
-    const uint32_t row0 = g * kU;
-    c = row0 / a.rows_per_chunk;
-    rr = row0 - c * a.rows_per_chunk;
-  }
-  uint32_t bi = c / a.items_per_block;
-  const uint32_t rem = c - bi * a.items_per_block;
-  uint32_t l = rem / kv;
-  uint32_t k = rem - l * kv;
-  // The ids do not change during the launch: read them through the constant
-  // address space, so the wave-uniform reads are scalar loads.
-  const __attribute__((address_space(4))) int64_t* gids =
-      (const __attribute__((address_space(4))) int64_t*)a.gids;
-  int64_t gid = gids[bi];
-  // scattered side: one base per chunk of the group
-  char* chunk_base[kC];
-#pragma unroll
-  for (int j = 0; j < kC; ++j) {
-    chunk_base[j] = reinterpret_cast<char*>(a.layer_ptr[l * ppl + k * (ppl - 1)]) +
-                    static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride +
-                    static_cast<int64_t>(rr) * kRow;
-    if (j + 1 < kC) {
-      if (++k == kv) {
-        k = 0;
-        if (++l == a.num_layers) {
-          l = 0;
-          gid = gids[++bi];
-        }
-      }
-    }
-  }
-  char* packed = a.packed + static_cast<int64_t>(g) * (kU * kRow);
-  u32x4 v[kU];
-#pragma unroll
-  for (int j = 0; j < kC; ++j)
-#pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      const char* src = kH2D ? packed + (j * kR + r) * kRow : chunk_base[j] + r * kRow;
-      v[j * kR + r] = __builtin_nontemporal_load((const gvec*)(src + lane_off));
-    }
-#pragma unroll
-  for (int j = 0; j < kC; ++j)
-#pragma unroll
-    for (int r = 0; r < kR; ++r) {
-      char* dst = kH2D ? chunk_base[j] + r * kRow : packed + (j * kR + r) * kRow;
-      __builtin_nontemporal_store(v[j * kR + r], (gvec*)(dst + lane_off));
-    }
+// Whether a group of `rows` rows touches at most 64 chunks of `chunk_vec`
+// vectors, wherever it starts.
+constexpr bool pack_fits(int rows, int64_t chunk_vec) {
+  const int64_t vec = int64_t(rows) * 64;
+  return (vec % chunk_vec == 0 ? vec / chunk_vec : (vec - 2) / chunk_vec + 2) <= 64;
 }
 
-// 32-row packed groups over chunks of 8 rows or more: group g moves packed
-// rows [32g, 32g + 32), fewer in the launch's last group.  They lie in chunk
-// c = 32g / rows_per_chunk and the chunks after it, at most kB = 2 + 30 /
-// rows_per_chunk chunks in all (2 from 31 rows per chunk, 3 from 16, 4 from
-// 11, 5 from 8; span_bases), so a wavefront
-// holds kB bases and picks one per row with wave-uniform compares (MLA's
-// 72-row chunks: a group reads 32 rows of one chunk, or the tail of one and
-// the head of the next).  Walk order, id reads and accesses as in
-// kv_pack_kernel.
-template <bool kH2D, int kB>
-__global__ __launch_bounds__(kThreads) void kv_pack_span_kernel(PackArgs a) {
-  constexpr int kU = 32;
-  constexpr int kRow = 64 * 16;
-  const uint32_t lane_off = (threadIdx.x & 63) * 16;
+// kRows: chunks are whole rows, so a row has one chunk and its address is
+// wave-uniform (scalar registers).  With per-lane addresses a 1 GiB scatter of
+// 72 KiB chunks took 404 us instead of 388.
+template <bool kH2D, int kU, bool kRows>
+__global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
+  const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t g = blockIdx.x * kWaves + wave;
+  const uint32_t q = a.columns.div(blockIdx.x);
+  const uint32_t wg = (blockIdx.x - q * a.columns.d) * a.column_wgs + q;
+  const uint32_t g = wg * kWaves + wave;
   if (g >= a.num_groups) return;
-  const uint32_t rpc = a.rows_per_chunk;
-  const uint32_t row0 = g * kU;
-  const uint32_t c = row0 / rpc;
-  const uint32_t rr = row0 - c * rpc;
-  const uint32_t rows = min(static_cast<uint32_t>(kU), a.num_rows - row0);
-  const uint32_t kv = a.kv_dim;
-  const uint32_t ppl = static_cast<uint32_t>(a.ptrs_per_layer);
-  uint32_t bi = c / a.items_per_block;
-  const uint32_t rem = c - bi * a.items_per_block;
-  uint32_t l = rem / kv;
-  uint32_t k = rem - l * kv;
-  const __attribute__((address_space(4))) int64_t* gids =
-      (const __attribute__((address_space(4))) int64_t*)a.gids;
-  int64_t gid = gids[bi];
-  // Row r of the group lies at base[j] + r * kRow for the last j with
-  // edge[j] <= r: chunk c + j starts at group row edge[j] (edge[0] = 0).
-  char* base[kB];
-  uint32_t edge[kB];
-  base[0] = reinterpret_cast<char*>(a.layer_ptr[l * ppl + k * (ppl - 1)]) +
-            static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride +
-            static_cast<int64_t>(rr) * kRow;
-  edge[0] = 0;
-#pragma unroll
-  for (int j = 1; j < kB; ++j) {
-    edge[j] = rpc - rr + (j - 1) * rpc;
-    base[j] = base[j - 1];
-    if (edge[j] < rows) {
-      if (++k == kv) {
-        k = 0;
-        if (++l == a.num_layers) {
-          l = 0;
-          gid = gids[++bi];
-        }
-      }
-      base[j] = reinterpret_cast<char*>(a.layer_ptr[l * ppl + k * (ppl - 1)]) +
-                static_cast<int64_t>(k) * a.gpu_kv_stride + gid * a.gpu_block_stride -
-                static_cast<int64_t>(edge[j]) * kRow;
-    }
+  const uint32_t v0 = g * (kU * 64);
+  const uint32_t c0 = a.chunk.div(v0);
+  const uint32_t r0 = v0 - c0 * a.chunk.d;    // the group's start within chunk c0
+  int64_t base;                               // lane j: the address chunk c0 + j gives position 0
+  {
+    const uint32_t c = min(c0 + lane, a.num_chunks - 1);
+    const uint32_t outer = a.inner.div(c);
+    const uint32_t rest = c - outer * a.inner.d;
+    const uint32_t b = a.layer_major ? rest : outer;
+    const uint32_t item = a.layer_major ? outer : rest;
+    const uint32_t l = a.kv_dim == 1 ? item : item >> 1;
+    const uint32_t k = item - l * a.kv_dim;
+    const uint32_t pi = a.ptrs_per_layer == 1 ? l : item;
+    const int64_t gid = a.gids ? a.gids[b] : a.inline_ids[b];
+    const uint64_t ptr = a.ptrs ? a.ptrs[pi] : a.layer_ptr[pi];
+    base = static_cast<int64_t>(ptr) + static_cast<int64_t>(k) * a.gpu_kv_stride +
+           gid * a.gpu_block_stride +
+           (static_cast<int64_t>(r0) - static_cast<int64_t>(lane) * a.chunk.d) * 16;
   }
-  char* packed = a.packed + static_cast<int64_t>(g) * (kU * kRow);
+  const int base_lo = static_cast<int>(base);
+  const int base_hi = static_cast<int>(base >> 32);
+  char* packed = a.packed + static_cast<int64_t>(v0) * 16;
+  const uint32_t n = a.num_vec - v0;          // vectors from the group's start to the end
   u32x4 v[kU];
+  if constexpr (kRows) {
+    const uint32_t lane_off = lane * 16;
+    // the scattered address of row u
+    auto scattered = [&](uint32_t u) {
+      const uint32_t j = a.chunk.div(r0 + u * 64);
+      const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(base_lo, j));
+      const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(base_hi, j));
+      return reinterpret_cast<char*>(((static_cast<uint64_t>(hi) << 32) | lo) + u * 1024);
+    };
 #pragma unroll
-  for (int r = 0; r < kU; ++r) {
-    if (r < rows) {
-      char* b = base[0];
+    for (uint32_t u = 0; u < kU; ++u)
+      if (u * 64 < n) {
+        const char* src = kH2D ? packed + u * 1024 : scattered(u);
+        v[u] = __builtin_nontemporal_load((const gvec*)(src + lane_off));
+      }
 #pragma unroll
-      for (int j = 1; j < kB; ++j)
-        if (r >= edge[j]) b = base[j];
-      const char* src = kH2D ? packed + r * kRow : b + r * kRow;
-      v[r] = __builtin_nontemporal_load((const gvec*)(src + lane_off));
+    for (uint32_t u = 0; u < kU; ++u)
+      if (u * 64 < n) {
+        char* dst = kH2D ? scattered(u) : packed + u * 1024;
+        __builtin_nontemporal_store(v[u], (gvec*)(dst + lane_off));
+      }
+  } else {
+    // the scattered address of the lane's vector at position i of the group
+    auto scattered = [&](uint32_t i) {
+      const int j = static_cast<int>(a.chunk.div(r0 + i)) * 4;
+      const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(j, base_lo));
+      const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(j, base_hi));
+      return reinterpret_cast<char*>(((static_cast<uint64_t>(hi) << 32) | lo) +
+                                     static_cast<uint64_t>(i) * 16);
+    };
+    // past the end a lane reloads the last vector and stores nothing
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t i = min(u * 64 + lane, n - 1);
+      const char* src = kH2D ? packed + i * 16 : scattered(i);
+      v[u] = __builtin_nontemporal_load((const gvec*)src);
     }
-  }
 #pragma unroll
-  for (int r = 0; r < kU; ++r) {
-    if (r < rows) {
-      char* b = base[0];
-#pragma unroll
-      for (int j = 1; j < kB; ++j)
-        if (r >= edge[j]) b = base[j];
-      char* dst = kH2D ? b + r * kRow : packed + r * kRow;
-      __builtin_nontemporal_store(v[r], (gvec*)(dst + lane_off));
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t i = u * 64 + lane;
+      char* dst = kH2D ? scattered(min(i, n - 1)) : packed + i * 16;
+      if (i < n) __builtin_nontemporal_store(v[u], (gvec*)dst);
     }
   }
 }
@@ -526,22 +235,6 @@ constexpr int kZeroCopyMaxLds = 56 << 10;
 // vectors of a launch: Divider divides numbers below 2^31
 constexpr int64_t kZeroCopyMaxVec = (int64_t(1) << 31) - 1;
 constexpr int64_t kZeroCopyMaxChunkVec = int64_t(1) << 29;
-
-// n / d for n < 2^31 as a multiplication (Granlund and Montgomery, "Division
-// by Invariant Integers using Multiplication", 1994): with 2^(l-1) < d <= 2^l,
-// mul = ceil(2^(31+l) / d) < 2^32 and n / d = floor(n * mul / 2^(31+l)).
-struct Divider {
-  uint32_t d = 1, mul = 0, shift = 0;
-  explicit Divider(uint32_t by = 1) : d(by) {
-    int l = 0;
-    while ((uint64_t(1) << l) < by) ++l;
-    shift = static_cast<uint32_t>(31 + l);
-    mul = static_cast<uint32_t>(((static_cast<unsigned __int128>(1) << shift) + by - 1) / by);
-  }
-  __device__ uint32_t div(uint32_t n) const {
-    return static_cast<uint32_t>((static_cast<uint64_t>(n) * mul) >> shift);
-  }
-};
 
 struct ZeroCopyArgs {
   const int64_t* ids;        // device-visible (gpu_id, cpu_id) pairs (inline_n == 0)
@@ -647,16 +340,12 @@ __global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) 
   }
 }
 
-// Copies a transfer's (gpu_id, cpu_id) pairs from the pinned buffer into a
-// device buffer laid out [gpu ids | cpu ids], n entries each, which the
-// staging kernels then read with ids_split = n.
-__global__ __launch_bounds__(256) void stage_ids_kernel(const int64_t* pairs, int64_t* out,
-                                                        int n) {
+// Copies n 64-bit values, `stride` apart in pinned memory, into a device table
+// (ids, layer pointers) that every workgroup of a staging launch then reads.
+__global__ __launch_bounds__(256) void stage_table_kernel(const int64_t* in, int stride,
+                                                          int64_t* out, int n) {
   const int i = blockIdx.x * 256 + static_cast<int>(threadIdx.x);
-  if (i < n) {
-    out[i] = pairs[2 * static_cast<int64_t>(i)];
-    out[static_cast<int64_t>(n) + i] = pairs[2 * static_cast<int64_t>(i) + 1];
-  }
+  if (i < n) out[i] = in[static_cast<int64_t>(i) * stride];
 }
 
 // A system-scope acquire in every workgroup.  Launched with a workgroup per
@@ -719,7 +408,7 @@ __global__ __launch_bounds__(kThreads) void kv_small_copy_kernel(SmallArgs a) {
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
     const int vi = min((u * kWaves + wave) * 64 + lane, n - 1);
-    v[u] = FKV_NT_LOAD ? __builtin_nontemporal_load(src + vi) : src[vi];
+    v[u] = __builtin_nontemporal_load(src + vi);
   }
 #pragma unroll
   for (int u = 0; u < kU; ++u) {
@@ -802,11 +491,6 @@ int64_t layer_run_bytes(bool h2d) {
 // was queued); not a hipError_t value
 constexpr int kSdmaUnavailable = -1000;
 
-template <bool H, bool W = false>
-void* staging_kernel_ptr() {
-  return reinterpret_cast<void*>(&kv_chunk_copy_kernel<H, W>);
-}
-
 int ensure_device_basics(int dev) {
   DeviceState& d = g_dev[dev];
   std::lock_guard<std::mutex> lk(g_init_mu);
@@ -825,116 +509,47 @@ int ensure_device_basics(int dev) {
   FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
       &o, reinterpret_cast<void*>(&kv_zero_copy_kernel<true>), kThreads, 0));
   d.occ_zero_copy[1] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<false>(), kThreads, 0));
-  d.occ_staged[0] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<true>(), kThreads, 0));
-  d.occ_staged[1] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<false, true>(),
-                                                       kThreads, 0));
-  d.occ_whole[0] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, staging_kernel_ptr<true, true>(),
-                                                       kThreads, 0));
-  d.occ_whole[1] = std::max(1, o);
   d.init = true;
   return 0;
 }
 
-// Staging launches take kv_pack_kernel / kv_pack_span_kernel where their
-// shape allows (1), or the row-by-row / whole-group kv_chunk_copy_kernel
-// throughout (0).
-#ifndef FKV_PACK_KERNEL
-#define FKV_PACK_KERNEL 1
-#endif
-
-// Staging kernels read their tile's ids from a device copy of the pairs
-// (stage_ids_on_device) rather than the pinned buffer: every workgroup of a
-// staging launch starts with that read, and over PCIe it costs a host round
-// trip per tile.
-#ifndef FKV_STAGE_IDS_ON_DEVICE
-#define FKV_STAGE_IDS_ON_DEVICE 1
-#endif
-
-// Queue a copy of the n pairs in `ids` (pinned) into a device buffer held by
-// `lease`, on `stream`, and describe it in `out` (the pinned pairs stay its
-// host side, for launches that take their ids inline) with `split` = n.
-// Without FKV_STAGE_IDS_ON_DEVICE, `out` is `ids` and `split` 0.
-int stage_ids_on_device(const IdBuf& ids, int n, int dev, hipStream_t stream, DevIdLease& lease,
-                        IdBuf* out, int32_t* split) {
-  *out = ids;
-  *split = 0;
-  if (!FKV_STAGE_IDS_ON_DEVICE || n <= 0) return 0;
+// Queue a copy of n values, `stride` apart in the pinned buffer `src`, into a
+// device buffer held by `lease`, on `stream`.
+int stage_table(const IdBuf& src, int stride, int n, int dev, hipStream_t stream,
+                DevIdLease& lease) {
   lease.dev = dev;
-  int rc = dev_ids_acquire(dev, static_cast<size_t>(n) * 16, &lease.buf);
+  int rc = dev_ids_acquire(dev, static_cast<size_t>(n) * 8, &lease.buf);
   if (rc) return rc;
   (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-  hipLaunchKernelGGL(stage_ids_kernel, dim3((n + 255) / 256), dim3(256), 0, stream,
-                     reinterpret_cast<const int64_t*>(ids.dev),
+  hipLaunchKernelGGL(stage_table_kernel, dim3((n + 255) / 256), dim3(256), 0, stream,
+                     reinterpret_cast<const int64_t*>(src.dev), stride,
                      reinterpret_cast<int64_t*>(lease.buf.dev), n);
   FKV_HIP(hipGetLastError());
-  out->dev = lease.buf.dev;
-  *split = n;
   return 0;
 }
 
-// Tiles are tb blocks x tl layers.  Start from whole block rows (one block,
-// every layer) and halve the layer window until there are about `factor`
-// tiles per occupancy slot of the grid; when blocks are plentiful, group
-// several per tile so one LDS id load serves more rows.  Rows per tile stay
-// below 2^31.  Measured on MI355X (2 GiB gather at the Llama-3-8B shape):
-// 32 rows in flight per wavefront with one workgroup per tile and 16 tiles
-// per slot is the best shape (6.0 TB/s with whole-group addressing; 4 and 8
-// tiles per slot 5.93 / 6.00, 32 tiles 5.44).
-//
-// A workgroup's wavefronts take the tile's unrolled row groups in turn, so a tile whose rows are not a
-// multiple of kWaves * unroll leaves some wavefronts idle while the others
-// finish (a one-layer Llama-3-8B tile, 64 rows, keeps two of four busy; a
-// one-layer MLA tile, 72 rows, fills 56% of the group slots).  The layer
-// window is then halved only while that fill does not drop, and row ranges
-// (below) are whole multiples of kWaves * unroll.  Measured on MI355X, 128 MiB
-// launches: Llama-3-8B gather 5.08 -> 5.40 TB/s, 70B-shard (4 KiB chunks)
-// gather 2.39 -> 3.66 TB/s.
-//
-// A transfer too small for that many tiles even one (block, layer) per tile
-// splits each tile's rows into up to `factor`-filling ranges of at least one
-// `unroll`-row group per wavefront, so more wavefronts share its few chunks.
-void choose_tiles(int nb, int nl, int kv, int rpc, int grid_cap, int factor, int unroll,
-                  CopyArgs* a) {
-  const int64_t target = factor * static_cast<int64_t>(std::max(1, grid_cap));
-  auto tiles = [&](int tb, int tl) {
-    return static_cast<int64_t>((nb + tb - 1) / tb) * ((nl + tl - 1) / tl);
-  };
-  auto rows_of = [&](int tb_, int tl_) { return static_cast<int64_t>(tb_) * tl_ * kv * rpc; };
-  const int64_t wave_groups = static_cast<int64_t>(unroll) * kWaves;   // rows of one round
-  // rows of a tile over the row slots its wavefronts' rounds provide
-  auto fill_below = [&](int64_t ra, int64_t rb) {   // fill(ra) < fill(rb)
-    const int64_t ca = (ra + wave_groups - 1) / wave_groups * wave_groups;
-    const int64_t cb = (rb + wave_groups - 1) / wave_groups * wave_groups;
-    return static_cast<__int128>(ra) * cb < static_cast<__int128>(rb) * ca;
-  };
-  int tb = 1, tl = nl;
-  while (tl > 1 && tiles(tb, tl) < target) {
-    const int half = (tl + 1) / 2;
-    if (fill_below(rows_of(tb, half), rows_of(tb, tl))) break;
-    tl = half;
-  }
-  while (tb < kMaxTileBlocks && tiles(tb * 2, tl) >= target) tb *= 2;
-  while (tb > 1 && static_cast<int64_t>(tb) * tl * kv * rpc >= (int64_t(1) << 31)) tb /= 2;
-  while (tl > 1 && static_cast<int64_t>(tb) * tl * kv * rpc >= (int64_t(1) << 31)) tl = (tl + 1) / 2;
-  const int64_t t = tiles(tb, tl);
-  const int64_t tile_rows = static_cast<int64_t>(tb) * tl * kv * rpc;
-  int64_t tr = 1, split = tile_rows;
-  if (t < target) {
-    tr = std::min<int64_t>(std::max<int64_t>(1, tile_rows / wave_groups), (target + t - 1) / t);
-    split = ((tile_rows + tr - 1) / tr + wave_groups - 1) / wave_groups * wave_groups;
-    tr = (tile_rows + split - 1) / split;
-  }
-  a->tile_blocks = tb;
-  a->tile_layers = tl;
-  a->tiles_b = (nb + tb - 1) / tb;
-  a->tiles_l = (nl + tl - 1) / tl;
-  a->tiles_r = static_cast<int32_t>(tr);
-  a->split_rows = static_cast<uint32_t>(split);
-  a->num_tiles = static_cast<int32_t>(t * tr);
+// The device tables of a transfer's staging launches: its gpu ids, and its
+// layer pointers when a launch covers more than the kernel arguments hold.
+struct StageTable {
+  const int64_t* gids = nullptr;    // null: launches carry their ids inline
+  const uint64_t* ptrs = nullptr;   // null: launches carry their layer pointers
+};
+
+// Queue the tables that launches of up to `nb` blocks and `nl` layers need.
+int stage_tables(const Geometry& g, int nb, int nl, int dev, hipStream_t stream, IdLease& host,
+                 DevIdLease& lease, StageTable* out) {
+  const int n_ids = nb > kPackInlineIds ? g.num_blocks : 0;
+  const int n_ptrs = nl > g.layers_per_launch() ? g.num_layers * g.ptrs_per_layer : 0;
+  if (n_ids + n_ptrs == 0) return 0;
+  int rc = ids_acquire(static_cast<size_t>(n_ids + n_ptrs) * 8, &host.buf);
+  if (rc) return rc;
+  memcpy(host.buf.host, g.gids, sizeof(int64_t) * n_ids);
+  memcpy(host.buf.host + n_ids, g.layer_ptrs, sizeof(int64_t) * n_ptrs);
+  if ((rc = stage_table(host.buf, 1, n_ids + n_ptrs, dev, stream, lease))) return rc;
+  int64_t* dev_table = reinterpret_cast<int64_t*>(lease.buf.dev);
+  if (n_ids) out->gids = dev_table;
+  if (n_ptrs) out->ptrs = reinterpret_cast<uint64_t*>(dev_table + n_ids);
+  return 0;
 }
 
 int64_t op_bytes(const Geometry& g) {
@@ -950,186 +565,130 @@ int zero_copy_grid(const DeviceState& d, int transfer_cus, bool h2d) {
                                                 d.occ_zero_copy[h2d ? 1 : 0]);
 }
 
-// The packed-row kernel for a staging launch of chunks of `rpc` full rows:
-// kv_pack_kernel<kU, kC>, kv_pack_span_kernel ({32, 0}), or {0, 0} when the
-// row-by-row or whole-group kv_chunk_copy_kernel takes it.
-struct PackShape {
-  int u = 0, c = 0;
-};
-// Measured on MI355X (HBM TB/s, interleaved A/B in one process):
-// - chunks of whole 32-row groups (32 KiB, 64 KiB, ...): gathers keep the
-//   tiled whole-group kernel (Llama-3-8B, 2 GiB: 6.07-6.10 against 6.01-6.08
-//   for 32-row span groups); scatters take the span kernel (5.53-5.54 against
-//   5.47-5.50; the copy-engine path's pieces 0.628 -> 0.650 of 8 TB/s);
-// - longer chunks that are not (MLA's 72 rows): 32-row span groups gather
-//   6.15-6.20 and scatter 5.70 against 5.60-5.62 and 5.48-5.49 for 36-row
-//   kv_pack_kernel groups (pieces: gather 0.695 -> 0.731, scatter 0.665 ->
-//   0.682);
-// - 4-16 KiB chunks: groups of 32 / rpc whole chunks;
-// - other chunks of 8-31 rows: span groups with 3-5 bases (DeepSeek MLA at
-//   16 tokens per block, 18 KiB chunks: gather 6.03-6.07 and scatter
-//   5.41-5.43 against 5.48-5.49 and 5.14-5.15 for the two-walk kernel;
-//   pieces 0.656 -> 0.712 and 0.614 -> 0.644).
-PackShape pack_shape(int64_t rpc, int64_t chunks, bool h2d) {
-  if (rpc % 32 == 0) return h2d ? PackShape{32, 0} : PackShape{};
-  if (rpc > 32) return {32, 0};
-  for (int c : {2, 4, 8})
-    if (rpc * c == 32 && chunks % c == 0) return {32, c};
-  if (rpc == 24) return {24, 1};
-  if (rpc >= 8) return {32, 0};
-  return {};
-}
+// Shape of a staging launch, by its size.  Measured on MI355X, us a gather /
+// scatter call (8 or 32 rows a wavefront; "columns": one workgroup per compute
+// unit, held there by unused LDS, each walking its own run of the buffer):
+//                                  8           32          32 columns
+//   1 MiB, 32 KiB chunks       15.2 / 14.6  19.1 / 16.1
+//   16 MiB, 32 KiB chunks      18.1 / 17.9  21.9 / 19.2
+//   21 MiB, 72 KiB chunks      26.9 / 28.0  29.3 / 27.3
+//   32 MiB, 32 KiB chunks      26.6 / 28.2  27.3 / 25.9
+//   47 MiB, 2 KiB chunks       37.2 / 39.7  38.0 / 40.1   42.1 / 39.9
+//   64 MiB, 4 KiB chunks       44.7 / 45.6  41.6 / 42.6   47.4 / 46.9
+//   256 MiB, 18 KiB chunks      114 / 119    113 / 118     114 / 117
+//   512 MiB, 32 KiB chunks      209 / 225    205 / 221     197 / 201
+//   1 GiB, 72 KiB chunks        398 / 419    376 / 406     363 / 382
+//   2 GiB, 32 KiB chunks        792 / 837    748 / 818     700 / 796
+// So 8 rows until 32-row groups give every compute unit a workgroup, and
+// columns from kPackColumnWgs workgroups a compute unit.
+constexpr uint32_t kPackColumnWgs = 12;
+constexpr unsigned kPackColumnLds = 84 << 10;
 
-// Chunks a 32-row span group can touch with chunks of `rpc` rows (rpc >= 8).
-int span_bases(int64_t rpc) { return 2 + static_cast<int>(30 / rpc); }
-
-// Dynamic LDS (unused by the kernels) that holds the span kernel and the
-// 24-row variant to one workgroup per compute unit.  Measured on MI355X,
-// capped / uncapped HBM TB/s: span groups gather 6.15-6.20 / 5.94-5.96 (MLA)
-// and 6.01-6.08 / 5.77-5.83 (Llama-3-8B), scatter 5.70-5.71 / 5.61-5.65 and
-// 5.53-5.54 / 5.37-5.43; two workgroups per CU (64 KiB) fall between; 24-row
-// groups gather 5.53 / 5.47.  The 4-16 KiB chunk groups gain nothing from it
-// (the Llama-3-70B TP-8 shard: gather 5.92-5.98 / 5.96-6.02, scatter 5.29 /
-// 5.24-5.28).
-constexpr unsigned kPackLdsOneGroup = 84 << 10;
-
-// Launch kv_pack_kernel<kH2D, kU, kC> over the launch's groups.
-template <bool kH2D, int kU, int kC>
-void launch_pack(const PackArgs& pa, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-  const uint32_t grid = (pa.num_groups + kWaves - 1) / kWaves;
-  hipExtLaunchKernelGGL((kv_pack_kernel<kH2D, kU, kC>), dim3(grid), dim3(kThreads),
-                        kU != 32 ? kPackLdsOneGroup : 0u, stream, ea, eb, 0, pa);
-}
-
-// Launch kv_pack_span_kernel<kH2D, kB> over the launch's groups.
-template <bool kH2D, int kB>
-void launch_pack_span(const PackArgs& pa, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-  const uint32_t grid = (pa.num_groups + kWaves - 1) / kWaves;
-  hipExtLaunchKernelGGL((kv_pack_span_kernel<kH2D, kB>), dim3(grid), dim3(kThreads),
-                        kPackLdsOneGroup, stream, ea, eb, 0, pa);
-}
-
-// Launch the staging gather / scatter over `nb` blocks starting at
-// block `b0` of the (already packed) id list, for GPU layers [l0, l0 + nl).
-// `cpu_base` is the CPU-side address of launch layer 0 of block index 0.
-// `ids` holds the packed pairs: `host` for the host's view, `dev` for the
-// device's (the same pinned buffer).  With `split` > 0, `dev` instead holds
-// the gpu ids and, `split` entries later, the cpu ids (device memory), and
-// `host` is null.  `grid_cap` is compute units x occupancy of the kernel the
-// launch takes; launches that take the whole-group variant use
-// `whole_grid_cap` instead when it is given.
-template <bool kH2D>
-int launch_staging(const Geometry& g, const IdBuf& ids, char* cpu_base, int64_t cks, int64_t cls,
-                int64_t cbs, int b0, int nb, int l0, int nl, int grid_cap,
-                hipStream_t stream, ProfRecorder& prof, int32_t split = 0,
-                int whole_grid_cap = 0) {
-  if (nl < 1 || static_cast<int64_t>(nl) * g.ptrs_per_layer > kMaxLayersPerLaunch)
-    return fail(kInval, "internal: a launch of %d layers exceeds the %d layer pointers of the "
-                "kernel arguments", nl, kMaxLayersPerLaunch / g.ptrs_per_layer);
-  // Staging launches whose packed side is contiguous in row order, with full
-  // rows and ids in device memory, take kv_pack_kernel or kv_pack_span_kernel
-  // where pack_shape says so.
-  {
-    const int64_t rpc = g.chunk / (64 * 16);
-    const bool packed_rows = FKV_PACK_KERNEL && split > 0 && g.chunk % (64 * 16) == 0 &&
-                             (g.kv == 1 || cks == g.chunk) && cls == g.kv * g.chunk &&
-                             cbs == static_cast<int64_t>(nl) * cls;
-    const int64_t chunks = static_cast<int64_t>(nb) * nl * g.kv;
-    const PackShape shape = packed_rows ? pack_shape(rpc, chunks, kH2D) : PackShape{};
-    if (shape.u > 0 && chunks * rpc + shape.u <= UINT32_MAX) {
-      PackArgs pa;
-      memset(&pa, 0, sizeof(pa));
-      pa.gids = reinterpret_cast<const int64_t*>(ids.dev) + b0;
-      pa.packed = cpu_base;
-      pa.gpu_kv_stride = g.gks;
-      pa.gpu_block_stride = g.gbs;
-      pa.rows_per_chunk = static_cast<uint32_t>(rpc);
-      pa.items_per_block = static_cast<uint32_t>(nl * g.kv);
-      pa.kv_dim = static_cast<uint32_t>(g.kv);
-      pa.num_layers = static_cast<uint32_t>(nl);
-      pa.num_rows = static_cast<uint32_t>(chunks * rpc);
-      pa.num_groups = (pa.num_rows + shape.u - 1) / shape.u;   // whole groups but for span launches
-      pa.ptrs_per_layer = g.ptrs_per_layer;
-      for (int i = 0; i < nl * g.ptrs_per_layer; ++i)
-        pa.layer_ptr[i] = reinterpret_cast<uint64_t>(g.layer_ptrs[l0 * g.ptrs_per_layer + i]);
-      hipEvent_t ea = nullptr, eb = nullptr;
-      int rc = prof.kernel_events(&ea, &eb);
-      if (rc) return rc;
-      prof.kernel_span(ea, eb, chunks * g.chunk);   // owns the events from here on
-      (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-      switch (shape.u * 16 + shape.c) {
-        case 32 * 16 + 2: launch_pack<kH2D, 32, 2>(pa, stream, ea, eb); break;
-        case 32 * 16 + 4: launch_pack<kH2D, 32, 4>(pa, stream, ea, eb); break;
-        case 32 * 16 + 8: launch_pack<kH2D, 32, 8>(pa, stream, ea, eb); break;
-        case 24 * 16 + 1: launch_pack<kH2D, 24, 1>(pa, stream, ea, eb); break;
-        default:
-          switch (span_bases(rpc)) {
-            case 2: launch_pack_span<kH2D, 2>(pa, stream, ea, eb); break;
-            case 3: launch_pack_span<kH2D, 3>(pa, stream, ea, eb); break;
-            case 4: launch_pack_span<kH2D, 4>(pa, stream, ea, eb); break;
-            default: launch_pack_span<kH2D, 5>(pa, stream, ea, eb); break;
-          }
-          break;
-      }
-      FKV_HIP(hipGetLastError());
-      return 0;
-    }
-  }
-  CopyArgs a;
-  memset(&a, 0, sizeof(a));
-  a.ids = reinterpret_cast<const int64_t*>(ids.dev) + (split ? 1 : 2) * static_cast<int64_t>(b0);
-  a.ids_split = split;
-  if (nb <= kInlineIds && ids.host) {
-    a.inline_n = nb;
-    memcpy(a.inline_ids, ids.host + 2 * static_cast<int64_t>(b0), sizeof(int64_t) * 2 * nb);
-  }
-  a.cpu_base = cpu_base;
-  a.gpu_kv_stride = g.gks;
-  a.gpu_block_stride = g.gbs;
-  a.cpu_kv_stride = cks;
-  a.cpu_layer_stride = cls;
-  a.cpu_block_stride = cbs;
-  a.chunk_vec = g.chunk / 16;
-  a.rows_per_chunk = static_cast<int32_t>((a.chunk_vec + 63) / 64);
-  a.num_blocks = nb;
-  a.num_layers = nl;
-  a.kv_dim = g.kv;
-  a.ptrs_per_layer = g.ptrs_per_layer;
-  for (int i = 0; i < nl * g.ptrs_per_layer; ++i)
-    a.layer_ptr[i] = reinterpret_cast<uint64_t>(g.layer_ptrs[l0 * g.ptrs_per_layer + i]);
-  // launches whose chunks are whole groups of full rows take the kernel
-  // variant that addresses each group from one base; its occupancy sizes the
-  // tiling
-  constexpr int kUnroll = kH2D ? FKV_UNROLL_SCATTER : kUnrollHbm;
-  const bool whole_variant =
-      kH2D ? (FKV_WHOLE_SCATTER &&
-              static_cast<int64_t>(nb) * nl * g.kv * g.chunk <= kWholeScatterMaxBytes)
-           : FKV_WHOLE_GATHER;
-  const bool whole = a.chunk_vec % 64 == 0 && whole_variant && a.rows_per_chunk % kUnroll == 0;
-  if (whole && whole_grid_cap > 0) grid_cap = whole_grid_cap;
-  choose_tiles(nb, nl, g.kv, a.rows_per_chunk, grid_cap,
-               kH2D ? FKV_TILE_FACTOR_SCATTER : FKV_TILE_FACTOR_HBM, kUnroll, &a);
-  a.block_major = kH2D ? FKV_BLOCK_MAJOR_SCATTER : FKV_BLOCK_MAJOR_GATHER;
-  const int grid = FKV_HBM_ONEPASS ? a.num_tiles : std::max(1, std::min(grid_cap, a.num_tiles));
-  hipEvent_t ea = nullptr, eb = nullptr;
-  int rc = prof.kernel_events(&ea, &eb);
-  if (rc) return rc;
-  prof.kernel_span(ea, eb, static_cast<int64_t>(nb) * nl * g.kv * g.chunk);
-  (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-  const unsigned lds = FKV_HBM_LDS_PAD;
-  if (whole)
-    hipExtLaunchKernelGGL((kv_chunk_copy_kernel<kH2D, true>), dim3(grid), dim3(kThreads), lds,
-                          stream, ea, eb, 0, a);
+template <bool kH2D, int kU>
+void launch_pack(PackArgs& pa, uint32_t num_cus, hipStream_t stream, hipEvent_t ea,
+                 hipEvent_t eb) {
+  pa.num_groups = (pa.num_vec + kU * 64 - 1) / (kU * 64);
+  uint32_t grid = (pa.num_groups + kWaves - 1) / kWaves;
+  const bool columns = kU == 32 && grid >= kPackColumnWgs * num_cus;
+  pa.columns = Divider(columns ? num_cus : 1);
+  pa.column_wgs = (grid + pa.columns.d - 1) / pa.columns.d;
+  grid = pa.column_wgs * pa.columns.d;
+  const unsigned lds = columns ? kPackColumnLds : 0;
+  if (pa.chunk.d % 64 == 0)
+    hipExtLaunchKernelGGL((kv_pack_kernel<kH2D, kU, true>), dim3(grid), dim3(kThreads), lds,
+                          stream, ea, eb, 0, pa);
   else
-    hipExtLaunchKernelGGL((kv_chunk_copy_kernel<kH2D>), dim3(grid), dim3(kThreads), lds, stream,
-                          ea, eb, 0, a);
-  FKV_HIP(hipGetLastError());
-  return 0;
+    hipExtLaunchKernelGGL((kv_pack_kernel<kH2D, kU, false>), dim3(grid), dim3(kThreads), lds,
+                          stream, ea, eb, 0, pa);
+}
+
+// Launch the staging gather / scatter over `nb` blocks of the call starting at
+// block `b0` and GPU layers [l0, l0 + nl).  `packed` holds their chunks back to
+// back, block -> layer -> K|V or, `layer_major`, layer -> K|V -> block.  More
+// than kPackInlineIds blocks need table.gids, and layers beyond
+// g.layers_per_launch() table.ptrs.
+template <bool kH2D>
+int launch_staging(const Geometry& g, const StageTable& table, char* packed, bool layer_major,
+                   int b0, int nb, int l0, int nl, int dev, hipStream_t stream,
+                   ProfRecorder& prof) {
+  const int64_t chunk_vec = g.chunk / 16;
+  // chunks of blocks [b, b + cb) and items (layer x K|V) [i, i + ci), all but
+  // `off` vectors of them
+  PackArgs pa;
+  auto launch = [&](int b, int cb, int64_t i, int64_t ci, int64_t off, int64_t part,
+                    char* at) -> int {
+    const int64_t chunks = cb * ci;
+    // one item: its pointer with K|V applied
+    const bool one = ci == 1;
+    const int64_t l = i / g.kv;
+    const int lp = static_cast<int>(one ? 1 : ci / g.kv);
+    const bool wide = !one && lp > g.layers_per_launch();
+    if ((cb > kPackInlineIds && !table.gids) || (wide && !table.ptrs))
+      return fail(kInval, "internal: a staging launch of %d blocks and %d layers without its "
+                  "tables", cb, lp);
+    pa.gids = table.gids ? table.gids + b : nullptr;
+    if (!pa.gids) memcpy(pa.inline_ids, g.gids + b, sizeof(int64_t) * cb);
+    pa.ptrs = nullptr;
+    if (one)
+      pa.layer_ptr[0] = reinterpret_cast<uint64_t>(
+          g.gpu_base(l0 + static_cast<int>(l), static_cast<int>(i % g.kv)) + off * 16);
+    else if (wide)
+      pa.ptrs = table.ptrs + (l0 + l) * g.ptrs_per_layer;
+    else
+      memcpy(pa.layer_ptr, g.layer_ptrs + (l0 + l) * g.ptrs_per_layer,
+             sizeof(uint64_t) * lp * g.ptrs_per_layer);
+    pa.packed = at;
+    pa.gpu_kv_stride = g.gks;
+    pa.gpu_block_stride = g.gbs;
+    pa.chunk = Divider(static_cast<uint32_t>(part));
+    pa.inner = Divider(static_cast<uint32_t>(layer_major ? cb : ci));
+    pa.layer_major = layer_major;
+    pa.kv_dim = one ? 1 : static_cast<uint32_t>(g.kv);
+    pa.ptrs_per_layer = one ? 1 : g.ptrs_per_layer;
+    pa.num_chunks = static_cast<uint32_t>(chunks);
+    pa.num_vec = static_cast<uint32_t>(chunks * part);
+    hipEvent_t ea = nullptr, eb = nullptr;
+    int rc = prof.kernel_events(&ea, &eb);
+    if (rc) return rc;
+    prof.kernel_span(ea, eb, chunks * part * 16);   // owns the events from here on
+    (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
+    const uint32_t num_cus = static_cast<uint32_t>(g_dev[dev].num_cus);
+    if (pack_fits(32, part) && pa.num_vec >= int64_t(num_cus) * kWaves * 32 * 64)
+      launch_pack<kH2D, 32>(pa, num_cus, stream, ea, eb);
+    else if (pack_fits(8, part))
+      launch_pack<kH2D, 8>(pa, num_cus, stream, ea, eb);
+    else
+      launch_pack<kH2D, 1>(pa, num_cus, stream, ea, eb);
+    FKV_HIP(hipGetLastError());
+    return 0;
+  };
+  const int64_t items = static_cast<int64_t>(nl) * g.kv;
+  const int64_t block_vec = items * chunk_vec;
+  int rc = 0;
+  if (nb * block_vec <= kPackMaxVec) return launch(b0, nb, 0, items, 0, chunk_vec, packed);
+  if (!layer_major && block_vec <= kPackMaxVec) {
+    const int step = static_cast<int>(kPackMaxVec / block_vec);
+    for (int b = 0; b < nb && !rc; b += step)
+      rc = launch(b0 + b, std::min(step, nb - b), 0, items, 0, chunk_vec,
+                  packed + b * block_vec * 16);
+    return rc;
+  }
+  // one (layer, K|V) at a time: runs of blocks where they are contiguous
+  const int64_t part_max = std::min(chunk_vec, kPackMaxVec);
+  const int step = layer_major ? static_cast<int>(std::min<int64_t>(nb, kPackMaxVec / part_max)) : 1;
+  for (int64_t i = 0; i < items && !rc; ++i)
+    for (int b = 0; b < nb && !rc; b += step)
+      for (int64_t off = 0; off < chunk_vec && !rc; off += part_max)
+        rc = launch(b0 + b, std::min(step, nb - b), i, 1, off, std::min(part_max, chunk_vec - off),
+                    packed + ((layer_major ? i * nb + b : b * items + i) * chunk_vec + off) * 16);
+  return rc;
 }
 
 // Launch kv_zero_copy_kernel over call layers [l0, l0 + nl) of every block of
 // the call.  `cpu_base` is the host-side address of call layer 0 of block id
-// 0; ids and `split` as in launch_staging; at most `grid_cap` workgroups a
+// 0; `ids` holds the packed pairs: `host` for the host's view, `dev` for the
+// device's (the same pinned buffer), or with `split` > 0 `dev` holds the gpu
+// ids and, `split` entries later, the cpu ids, and `host` is null; at most `grid_cap` workgroups a
 // launch.  One launch, but for layers beyond the pointers a launch carries
 // and for runs beyond what Divider or a workgroup's LDS takes.  `done` (null
 // while profiling): an event the last launch completes, carried by its own
@@ -1482,11 +1041,8 @@ int transfer_staged(const Geometry& g, hipStream_t stream, int dev, bool h2d) {
   int rc = guard.set(dev);
   if (rc) return rc;
   IdLease ids;
-  rc = pack_ids(g, ids);
-  if (rc) return rc;
   DevIdLease dev_ids;   // released after the drain below
-  IdBuf kids;           // the ids the staging kernels read
-  int32_t kids_split = 0;
+  StageTable table;
 
   // A piece is a run of whole blocks over a layer window; the window covers
   // all layers unless one block row would not fit a staging half.
@@ -1508,8 +1064,6 @@ int transfer_staged(const Geometry& g, hipStream_t stream, int dev, bool h2d) {
   }
   const size_t half = ln.staging_bytes / 2;
   const int blocks_per_piece = static_cast<int>(std::max<size_t>(1, half / row_bytes));
-  const int grid_cap = d.num_cus * (h2d ? d.occ_staged[1] : d.occ_staged[0]);
-  const int whole_cap = d.num_cus * (h2d ? d.occ_whole[1] : d.occ_whole[0]);
   const hsa_agent_t host_agent = d.cpu_agent;   // device-resident caches never get here
 
   struct Piece {
@@ -1560,7 +1114,8 @@ int transfer_staged(const Geometry& g, hipStream_t stream, int dev, bool h2d) {
     }
   } publish{ln};
   DrainOnError drain{stream, &d, &ln};
-  if ((rc = stage_ids_on_device(ids.buf, g.num_blocks, dev, stream, dev_ids, &kids, &kids_split)))
+  if ((rc = stage_tables(g, std::min(blocks_per_piece, g.num_blocks), nl_piece, dev, stream, ids,
+                         dev_ids, &table)))
     return rc;
   ProfRecorder prof;
   std::vector<Run> runs;
@@ -1605,22 +1160,11 @@ int transfer_staged(const Geometry& g, hipStream_t stream, int dev, bool h2d) {
   };
   auto launch = [&](int pi) -> int {
     const Piece& p = pieces[pi];
-    // staging strides (K|V, layer, block) of the piece
-    int64_t cks, cls, cbs;
-    if (layer_major) {
-      cbs = g.chunk;
-      cks = g.kv == 1 ? 0 : static_cast<int64_t>(p.nb) * g.chunk;
-      cls = static_cast<int64_t>(g.kv) * p.nb * g.chunk;
-    } else {
-      cks = g.kv == 1 ? 0 : g.chunk;
-      cls = static_cast<int64_t>(g.kv) * g.chunk;
-      cbs = static_cast<int64_t>(p.nl) * cls;
-    }
     char* stg = ln.staging + (pi & 1) * half;
-    return h2d ? launch_staging<true>(g, kids, stg, cks, cls, cbs, p.b0, p.nb, p.l0, p.nl,
-                                         grid_cap, stream, prof, kids_split, whole_cap)
-               : launch_staging<false>(g, kids, stg, cks, cls, cbs, p.b0, p.nb, p.l0, p.nl,
-                                          grid_cap, stream, prof, kids_split, whole_cap);
+    return h2d ? launch_staging<true>(g, table, stg, layer_major, p.b0, p.nb, p.l0, p.nl, dev,
+                                      stream, prof)
+               : launch_staging<false>(g, table, stg, layer_major, p.b0, p.nb, p.l0, p.nl, dev,
+                                       stream, prof);
   };
   if (!h2d) {
     for (int pi = 0; pi < np; ++pi) {
@@ -1675,30 +1219,19 @@ int transfer_staged(const Geometry& g, hipStream_t stream, int dev, bool h2d) {
 // buffer laid out [block][layer][K|V][chunk]; g.cpu_ptr is the buffer and
 // g.cids is 0..n-1.  Uses every compute unit: the copy is HBM-bound.
 int transfer_contiguous(const Geometry& g, hipStream_t stream, int dev, bool to_gpu) {
-  DeviceState& d = g_dev[dev];
   IdLease ids;
-  int rc = pack_ids(g, ids);
-  if (rc) return rc;
-  const int grid_cap = d.num_cus * (to_gpu ? d.occ_staged[1] : d.occ_staged[0]);
-  const int whole_cap = d.num_cus * (to_gpu ? d.occ_whole[1] : d.occ_whole[0]);
   DevIdLease dev_ids;
-  IdBuf kids;
-  int32_t kids_split = 0;
+  StageTable table;
   DrainOnError drain{stream};
-  if ((rc = stage_ids_on_device(ids.buf, g.num_blocks, dev, stream, dev_ids, &kids, &kids_split)))
-    return rc;
+  int rc = stage_tables(g, g.num_blocks, g.num_layers, dev, stream, ids, dev_ids, &table);
+  if (rc) return rc;
   ProfRecorder prof;
-  const int per_launch = g.layers_per_launch();
-  for (int l0 = 0; l0 < g.num_layers; l0 += per_launch) {
-    const int nl = std::min(per_launch, g.num_layers - l0);
-    char* base = g.cpu_info.dev_ptr + static_cast<int64_t>(l0) * g.cls;
-    rc = to_gpu ? launch_staging<true>(g, kids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
-                                          l0, nl, grid_cap, stream, prof, kids_split, whole_cap)
-                : launch_staging<false>(g, kids, base, g.cks, g.cls, g.cbs, 0, g.num_blocks,
-                                           l0, nl, grid_cap, stream, prof, kids_split,
-                                           whole_cap);
-    if (rc) return rc;
-  }
+  char* buffer = g.cpu_info.dev_ptr;
+  rc = to_gpu ? launch_staging<true>(g, table, buffer, false, 0, g.num_blocks, 0, g.num_layers,
+                                     dev, stream, prof)
+              : launch_staging<false>(g, table, buffer, false, 0, g.num_blocks, 0, g.num_layers,
+                                      dev, stream, prof);
+  if (rc) return rc;
   FKV_HIP(hipStreamSynchronize(stream));
   drain.armed = false;
   prof.flush();
@@ -1800,6 +1333,7 @@ struct fkv_transfer_handle_s {
   std::vector<int> null_covers;
   int null_upto = 0;              // groups the device's legacy null stream waits for (mu)
   IdBuf ids;
+  DevIdLease dev_ids;             // copy-engine pipeline: the gpu ids of its scatters
   ProfRecorder prof;
   bool enqueued = false;          // every group was enqueued
   // Copy-engine pipeline: a driver thread queues each layer group's SDMA
@@ -2114,14 +1648,17 @@ int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
     pieces.back().last = true;
   }
   const int np = static_cast<int>(pieces.size());
-  const int grid_cap = d.num_cus * d.occ_staged[1];
-  const int whole_cap = d.num_cus * d.occ_whole[1];
   std::vector<Run> runs;
   bool pending[2] = {false, false};
   int next_group = 0;   // the first group whose event is not yet recorded
   int64_t dma_copies = 0, dma_bytes = 0;
   const auto t0 = std::chrono::steady_clock::now();
   DrainOnError drain{work, &d, &ln};
+  StageTable table;
+  if (g.num_blocks > kPackInlineIds) {
+    if ((rc = stage_table(h->ids, 2, g.num_blocks, h->dev, work, h->dev_ids))) return rc;
+    table.gids = reinterpret_cast<int64_t*>(h->dev_ids.buf.dev);
+  }
   auto queue_copies = [&](int pi) -> int {
     const Piece& p = pieces[pi];
     build_runs(g, p.b0, p.nb, p.l0, p.nl, false, false, runs);
@@ -2153,13 +1690,8 @@ int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
     if ((rc = sdma_wait(d, ln, hf, /*spin=*/pi + 1 == np))) return rc;
     hipLaunchKernelGGL(acquire_system_kernel, dim3(d.num_cus), dim3(64), 0, work);
     FKV_HIP(hipGetLastError());
-    const int64_t cks = g.kv == 1 ? 0 : g.chunk;
-    const int64_t cls = static_cast<int64_t>(g.kv) * g.chunk;
-    const int64_t cbs = static_cast<int64_t>(p.nl) * cls;
-    // launch_copy reads the group's layer pointers from call layer p.l0 on
-    if ((rc = launch_staging<true>(g, h->ids, ln.staging + hf * half, cks, cls, cbs, p.b0,
-                                      p.nb, p.l0, p.nl, grid_cap, work, h->prof, 0,
-                                      whole_cap)))
+    if ((rc = launch_staging<true>(g, table, ln.staging + hf * half, false, p.b0, p.nb, p.l0,
+                                   p.nl, h->dev, work, h->prof)))
       return rc;
     if (p.last) {
       for (int gi = next_group; gi <= p.group; ++gi) FKV_HIP(hipEventRecord(h->done[gi], work));

@@ -1082,14 +1082,9 @@ def test_c_ext_releases_the_gil(dev, use_ce):
 def test_gather_scatter_match_oracle(dev, geo, buffer_on_host):
     """fkv_gather/scatter_kv_blocks against the oracle with the contiguous
     buffer described as a block-wise cache [n, L, kv, chunk] and ids 0..n-1.
-    Every packed-row kernel shape is here: 32-row span groups over chunks of
-    72, 40 and 33 KiB (two bases), 18 and 16 KiB (three), 12 KiB (four), 9
-    and 8 KiB (five), with groups that cross chunk edges and a short last
-    group, and, scattering, over 32 / 64 KiB chunks; 24 KiB (24-row groups);
-    16 / 8 / 4 KiB chunk counts that fill groups of 2 / 4 / 8 whole chunks;
-    the tiled whole-group gather of 32 / 64 KiB chunks; and the row-by-row
-    kernel's cases: partial rows (128 B, 48 B), 1 KiB chunks, 4 KiB chunks
-    whose count is not a multiple of 8, more layers than one launch holds."""
+    Chunks of many rows, whole rows and partial rows are here, with groups
+    that cross chunk edges and a short last group, and more layers than the
+    kernel arguments hold."""
     import ctypes
     from flexkv_amd import _lib
     from flexkv_amd.storage.allocator import pinned_empty
@@ -1225,3 +1220,31 @@ def test_general_kernel_edges(dev, monkeypatch, layout, chunk, n, nl, kv, cus):
                   tokens=1, heads=1, dim=chunk // 2, layout=layout).fill(seed=n + chunk)
     check_case(case, inputs.distinct_ids(n, n, n + 3), inputs.distinct_ids(n + 1, n, n + 5), 0,
                transfer_cus=cus)
+
+
+@pytest.mark.parametrize("chunk,n,layers,kv", [
+    (16, 300, 3, 2), (112, 64, 3, 1), (128, 255, 2, 2), (144, 256, 5, 1), (512, 257, 80, 2),
+    (512, 480, 80, 2), (528, 420, 80, 2), (496, 300, 130, 2), (4608, 131, 61, 1),
+    (32768, 16, 32, 2), (32768, 15, 32, 2), (73728, 91, 61, 1), (1040, 3300, 61, 2)])
+def test_pack_kernel_edges(dev, chunk, n, layers, kv):
+    """The staging kernel at the edges of its dispatch: groups of 1, 8 and 32
+    rows by chunk size and by launch size (a group for every wavefront of the
+    chip: 32 MiB on 256 compute units), the column order of large launches
+    with a short last column, ids and layer pointers in the arguments or in a
+    device table.  Blocks that are not named stay as they are."""
+    from flexkv_amd import c_ext
+    pool = n + 9
+    gen = torch.Generator(device=dev).manual_seed(chunk + n)
+    cache = torch.randint(-2**62, 2**62, (layers, kv, pool, chunk // 8), dtype=torch.int64,
+                          device=dev, generator=gen)
+    ids = torch.randperm(pool, generator=torch.Generator().manual_seed(n))[:n].contiguous()
+    ptrs = torch.tensor([cache[l].data_ptr() for l in range(layers)], dtype=torch.int64)
+    buf = torch.zeros(n, layers, kv, chunk // 8, dtype=torch.int64, device=dev)
+    want = cache[:, :, ids.to(dev)].permute(2, 0, 1, 3)
+    c_ext.gather_kv_blocks(ids, ptrs, pool * chunk, chunk, chunk, buf, kv == 1)
+    assert torch.equal(buf, want)
+    want = cache.clone()
+    buf.bitwise_xor_(0x0F0F)
+    want[:, :, ids.to(dev)] = buf.permute(1, 2, 0, 3)
+    c_ext.scatter_kv_blocks(ids, ptrs, pool * chunk, chunk, chunk, buf, kv == 1)
+    assert torch.equal(cache, want)
