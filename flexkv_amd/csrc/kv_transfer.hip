@@ -56,6 +56,21 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 // host memory); saying so lets the compiler emit global_* instead of flat_*.
 typedef __attribute__((address_space(1))) u32x4 gvec;
 
+// 16 bytes written through every cache (system scope).  Stores into pinned
+// host memory go this way: left to the caches they arrive in the order of
+// evictions, and a 16 MiB device-to-host call took 360 us instead of 317 (16
+// workgroups).  In assembly, as no builtin stores 16 bytes at system scope;
+// the s_nop keeps the two wait states a wide store needs before its data
+// registers are written again, which the compiler cannot see it needs.
+__device__ inline void store_system(char* p, u32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+}
+
+// The same with the non-temporal hint, for HBM.
+__device__ inline void store_through(char* p, u32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1 nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+}
+
 // n / d for n < 2^31 as a multiplication (Granlund and Montgomery, "Division
 // by Invariant Integers using Multiplication", 1994): with 2^(l-1) < d <= 2^l,
 // mul = ceil(2^(31+l) / d) < 2^32 and n / d = floor(n * mul / 2^(31+l)).
@@ -87,8 +102,8 @@ struct Divider {
 // HBM bounds the large launches and the launch the small ones.  Measured on
 // MI355X, us a gather / scatter call, against a kernel per chunk shape (tiled
 // groups, 2-5 bases a group, a row-by-row one) with the ids staged by a launch
-// of their own: 2 GiB of 32 KiB chunks 727 / 808 -> 706 / 796, 1 GiB of 4 KiB
-// 383 / 440 -> 379 / 416, 1 GiB of 2 KiB 462 / 462 -> 381 / 413, 47 MiB of 2
+// of their own: 2 GiB of 32 KiB chunks 727 / 808 -> 706 / 774, 1 GiB of 4 KiB
+// 383 / 440 -> 379 / 407, 1 GiB of 2 KiB 462 / 462 -> 381 / 406, 47 MiB of 2
 // KiB 57.2 / 57.0 -> 38.0 / 40.1, 64 MiB of 512 B 79.4 / 78.7 -> 47.2 / 46.3,
 // 1 MiB of 32 KiB 18.8 / 20.6 -> 15.2 / 14.6.
 constexpr int kPackInlineIds = 256;
@@ -126,7 +141,11 @@ constexpr bool pack_fits(int rows, int64_t chunk_vec) {
 // kRows: chunks are whole rows, so a row has one chunk and its address is
 // wave-uniform (scalar registers).  With per-lane addresses a 1 GiB scatter of
 // 72 KiB chunks took 404 us instead of 388.
-template <bool kH2D, int kU, bool kRows>
+// kThrough: stores bypass the caches, for scatters in column order.  Measured
+// on MI355X, us against non-temporal stores: 2 GiB of 32 KiB chunks 795 -> 774,
+// 1 GiB of 72 / 4 / 2 KiB 382 -> 368, 415 -> 407, 414 -> 406; a 2 GiB gather
+// would take 896 instead of 707 and smaller scatters gain nothing.
+template <bool kH2D, int kU, bool kRows, bool kThrough>
 __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -176,8 +195,11 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
 #pragma unroll
     for (uint32_t u = 0; u < kU; ++u)
       if (u * 64 < n) {
-        char* dst = kH2D ? scattered(u) : packed + u * 1024;
-        __builtin_nontemporal_store(v[u], (gvec*)(dst + lane_off));
+        char* dst = (kH2D ? scattered(u) : packed + u * 1024) + lane_off;
+        if (kThrough)
+          store_through(dst, v[u]);
+        else
+          __builtin_nontemporal_store(v[u], (gvec*)dst);
       }
   } else {
     // the scattered address of the lane's vector at position i of the group
@@ -199,7 +221,12 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
     for (int u = 0; u < kU; ++u) {
       const uint32_t i = u * 64 + lane;
       char* dst = kH2D ? scattered(min(i, n - 1)) : packed + i * 16;
-      if (i < n) __builtin_nontemporal_store(v[u], (gvec*)dst);
+      if (i < n) {
+        if (kThrough)
+          store_through(dst, v[u]);
+        else
+          __builtin_nontemporal_store(v[u], (gvec*)dst);
+      }
     }
   }
 }
@@ -256,16 +283,6 @@ struct ZeroCopyArgs {
   uint64_t layer_ptr[kMaxLayersPerLaunch];
   int64_t inline_ids[2 * kInlineIdsZeroCopy];
 };
-
-// 16 bytes written through every cache (system scope).  Stores into pinned
-// host memory go this way: left to the caches they arrive in the order of
-// evictions, and a 16 MiB device-to-host call took 360 us instead of 317 (16
-// workgroups).  In assembly, as no builtin stores 16 bytes at system scope;
-// the s_nop keeps the two wait states a wide store needs before its data
-// registers are written again, which the compiler cannot see it needs.
-__device__ inline void store_system(char* p, u32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
-}
 
 template <bool kH2D>
 __global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) {
@@ -576,9 +593,9 @@ int zero_copy_grid(const DeviceState& d, int transfer_cus, bool h2d) {
 //   47 MiB, 2 KiB chunks       37.2 / 39.7  38.0 / 40.1   42.1 / 39.9
 //   64 MiB, 4 KiB chunks       44.7 / 45.6  41.6 / 42.6   47.4 / 46.9
 //   256 MiB, 18 KiB chunks      114 / 119    113 / 118     114 / 117
-//   512 MiB, 32 KiB chunks      209 / 225    205 / 221     197 / 201
-//   1 GiB, 72 KiB chunks        398 / 419    376 / 406     363 / 382
-//   2 GiB, 32 KiB chunks        792 / 837    748 / 818     700 / 796
+//   512 MiB, 32 KiB chunks      209 / 225    205 / 221     194 / 198
+//   1 GiB, 72 KiB chunks        398 / 419    376 / 406     363 / 368
+//   2 GiB, 32 KiB chunks        792 / 837    748 / 818     705 / 774
 // So 8 rows until 32-row groups give every compute unit a workgroup, and
 // columns from kPackColumnWgs workgroups a compute unit.
 constexpr uint32_t kPackColumnWgs = 12;
@@ -594,12 +611,12 @@ void launch_pack(PackArgs& pa, uint32_t num_cus, hipStream_t stream, hipEvent_t 
   pa.column_wgs = (grid + pa.columns.d - 1) / pa.columns.d;
   grid = pa.column_wgs * pa.columns.d;
   const unsigned lds = columns ? kPackColumnLds : 0;
-  if (pa.chunk.d % 64 == 0)
-    hipExtLaunchKernelGGL((kv_pack_kernel<kH2D, kU, true>), dim3(grid), dim3(kThreads), lds,
-                          stream, ea, eb, 0, pa);
-  else
-    hipExtLaunchKernelGGL((kv_pack_kernel<kH2D, kU, false>), dim3(grid), dim3(kThreads), lds,
-                          stream, ea, eb, 0, pa);
+  const bool rows = pa.chunk.d % 64 == 0;
+  auto kernel = rows ? kv_pack_kernel<kH2D, kU, true, false> : kv_pack_kernel<kH2D, kU, false, false>;
+  if (kH2D && columns)
+    kernel = rows ? kv_pack_kernel<kH2D, kU, true, kH2D && kU == 32>
+                  : kv_pack_kernel<kH2D, kU, false, kH2D && kU == 32>;
+  hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, ea, eb, 0, pa);
 }
 
 // Launch the staging gather / scatter over `nb` blocks of the call starting at
