@@ -295,17 +295,24 @@ int validate(Geometry& g, int mode) {
   const __int128 glo = static_cast<__int128>(g.min_gid) * g.gbs;
   const __int128 ghi = static_cast<__int128>(g.kv - 1) * g.gks +
                        static_cast<__int128>(g.max_gid) * g.gbs + g.chunk;
-  // Every layer (or K/V) pointer is its own allocation as a rule; query each.
+  // Each layer (or K/V) pointer may be an allocation of its own or lie in one
+  // with others, as an engine's cache reserved in one piece does.  A pointer
+  // inside the allocation the last query described is not queried again: a
+  // query takes about 0.13 us of host time, 61 of them 8 us of a 28 us gather.
   if (g.ptrs_per_layer != 1 && (g.ptrs_per_layer != g.kv || g.gks != 0))
     return fail(kInval, "separate K/V pointers need kv pointers per layer and no kv stride");
   const int64_t nptr = static_cast<int64_t>(g.num_layers) * g.ptrs_per_layer;
+  PtrInfo pi;
   for (int64_t i = 0; i < nptr; ++i) {
     const char* p = static_cast<const char*>(g.layer_ptrs[i]);
     if (!p) return fail(kInval, "gpu layer pointer %lld is null", (long long)i);
     if (vec_mode && reinterpret_cast<uintptr_t>(p) % 16 != 0)
       return fail(kInval, "gpu layer pointer %lld is not 16-byte aligned", (long long)i);
-    PtrInfo pi;
-    if (query_ptr(p, &pi) != 0 || !pi.device)
+    if (!(pi.device && p >= pi.base && p < pi.base + pi.size)) {
+      pi = PtrInfo();
+      if (query_ptr(p, &pi) != 0) pi.device = false;
+    }
+    if (!pi.device)
       return fail(kInval, "gpu layer pointer %lld (%p) is not device memory", (long long)i, p);
     if (!range_inside(p, glo, ghi, pi))
       return fail(kInval,

@@ -1248,3 +1248,48 @@ def test_pack_kernel_edges(dev, chunk, n, layers, kv):
     want[:, :, ids.to(dev)] = buf.permute(1, 2, 0, 3)
     c_ext.scatter_kv_blocks(ids, ptrs, pool * chunk, chunk, chunk, buf, kv == 1)
     assert torch.equal(cache, want)
+
+
+@pytest.mark.parametrize("second,refusal", [("same", None), ("other", None),
+                                            ("host", "pointer 1 .* is not device memory"),
+                                            ("past-end", "outside the allocation of layer pointer 1"),
+                                            ("short", "outside the allocation of layer pointer 1"),
+                                            ("back", None)])
+def test_layer_pointers_are_each_checked(dev, second, refusal):
+    """Layer pointers into one allocation, into others, and bad ones after
+    good ones: each is held to its own allocation."""
+    import ctypes
+    from flexkv_amd import _lib
+    # allocations of the library's own, so their ends are known
+    hip = ctypes.CDLL("libamdhip64.so")
+    chunk, n = 4096, 6
+
+    def alloc(size):
+        p = ctypes.c_void_p()
+        assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) == 0
+        return p.value
+    layer = 2 * n * chunk
+    a, b = alloc(2 * layer), alloc(layer)
+    small = alloc(layer - 4096)
+    host = torch.zeros(layer, dtype=torch.uint8, pin_memory=True)
+    try:
+        ptrs = {"same": [a, a + layer], "other": [a, b], "host": [a, host.data_ptr()],
+                "past-end": [a, a + layer + 4096], "short": [a, small],
+                "back": [a, b, a + layer]}[second]
+        buf = torch.zeros(n, len(ptrs), 2, chunk, dtype=torch.uint8, device=dev)
+        ids = (ctypes.c_int64 * n)(*range(n))
+        table = (ctypes.c_void_p * len(ptrs))(*ptrs)
+
+        def call():
+            _lib.check(_lib.load().fkv_gather_kv_blocks(
+                n, len(ptrs), ids, table, n * chunk, chunk, chunk, buf.data_ptr(), buf.numel(),
+                torch.cuda.current_stream().cuda_stream, 0), "gather")
+        if refusal is None:
+            call()
+        else:
+            with pytest.raises(RuntimeError, match=refusal):
+                call()
+    finally:
+        torch.cuda.synchronize()
+        for p in (a, b, small):
+            assert hip.hipFree(ctypes.c_void_p(p)) == 0
