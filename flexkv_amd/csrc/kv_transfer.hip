@@ -399,19 +399,26 @@ template <bool kH2D>
 constexpr int small_piece_rows() { return kWaves * small_rows_per_wave<kH2D>(); }
 constexpr int64_t kSmallMaxBytes = int64_t(4) << 20;   // bytes moved per call
 
+// Calls of at most this many pieces pass lists of that length: the host writes
+// a launch's arguments over PCIe, 2.5 KiB of them for kSmallPieces.  Measured on
+// MI355X through the C-ABI, one block of 64 KiB with the long / short list:
+// 14.99 / 14.76 us device-to-host, 15.60 / 15.42 host-to-device.
+constexpr int kFewPieces = 16;
+
+template <int kPieces>
 struct SmallArgs {
-  uint64_t src[kSmallPieces];
-  uint64_t dst[kSmallPieces];
-  int32_t nvec[kSmallPieces];   // 16-byte vectors of each piece
+  uint64_t src[kPieces];
+  uint64_t dst[kPieces];
+  int32_t nvec[kPieces];   // 16-byte vectors of each piece
 };
 
 // One workgroup per piece (the host launches exactly as many as there are
-// pieces, at most kSmallPieces): wavefront `wave` of workgroup w takes rows
+// pieces, at most kPieces): wavefront `wave` of workgroup w takes rows
 // wave + j * kWaves of piece w, j < small_rows_per_wave.  No branch sits
 // between the argument loads and the data loads, so the piece's length and
 // both addresses arrive in one round.
-template <bool kH2D>
-__global__ __launch_bounds__(kThreads) void kv_small_copy_kernel(SmallArgs a) {
+template <bool kH2D, int kPieces>
+__global__ __launch_bounds__(kThreads) void kv_small_copy_kernel(SmallArgs<kPieces> a) {
   constexpr int kU = small_rows_per_wave<kH2D>();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -515,10 +522,10 @@ int ensure_device_basics(int dev) {
   FKV_HIP(hipDeviceGetAttribute(&d.num_cus, hipDeviceAttributeMultiprocessorCount, dev));
   int o = 0;
   FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &o, reinterpret_cast<void*>(&kv_small_copy_kernel<false>), kThreads, 0));
+      &o, reinterpret_cast<void*>(&kv_small_copy_kernel<false, kSmallPieces>), kThreads, 0));
   d.occ_small[0] = std::max(1, o);
   FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &o, reinterpret_cast<void*>(&kv_small_copy_kernel<true>), kThreads, 0));
+      &o, reinterpret_cast<void*>(&kv_small_copy_kernel<true, kSmallPieces>), kThreads, 0));
   d.occ_small[1] = std::max(1, o);
   FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
       &o, reinterpret_cast<void*>(&kv_zero_copy_kernel<false>), kThreads, 0));
@@ -794,10 +801,10 @@ int small_pieces(const Geometry& g, int grid_cap, bool h2d) {
 // One launch of kv_small_copy_kernel over the whole call.  `cpu_dev` is the
 // device-visible address of the host cache at call layer 0 (start layer and
 // start offset applied).  Chunk sizes are multiples of 16 bytes here.
-template <bool kH2D>
-int transfer_small(const Geometry& g, char* cpu_dev, int n_pieces, hipStream_t stream,
+template <bool kH2D, int kPieces>
+int launch_small(const Geometry& g, char* cpu_dev, int n_pieces, hipStream_t stream,
                    ProfRecorder& prof) {
-  SmallArgs a;
+  SmallArgs<kPieces> a;
   const int64_t piece_bytes = int64_t(small_piece_rows<kH2D>()) * 64 * 16;
   int p = 0;
   for (int l = 0; l < g.num_layers; ++l)
@@ -818,10 +825,18 @@ int transfer_small(const Geometry& g, char* cpu_dev, int n_pieces, hipStream_t s
   if (rc) return rc;
   prof.kernel_span(ea, eb, op_bytes(g));
   (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-  hipExtLaunchKernelGGL(kv_small_copy_kernel<kH2D>, dim3(n_pieces), dim3(kThreads), 0, stream,
-                        ea, eb, 0, a);
+  hipExtLaunchKernelGGL((kv_small_copy_kernel<kH2D, kPieces>), dim3(n_pieces), dim3(kThreads), 0,
+                        stream, ea, eb, 0, a);
   FKV_HIP(hipGetLastError());
   return 0;
+}
+
+template <bool kH2D>
+int transfer_small(const Geometry& g, char* cpu_dev, int n_pieces, hipStream_t stream,
+                   ProfRecorder& prof) {
+  return n_pieces <= kFewPieces
+             ? launch_small<kH2D, kFewPieces>(g, cpu_dev, n_pieces, stream, prof)
+             : launch_small<kH2D, kSmallPieces>(g, cpu_dev, n_pieces, stream, prof);
 }
 
 int transfer_zero_copy(const Geometry& g, hipStream_t stream, int dev, int transfer_cus,

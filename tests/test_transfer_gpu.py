@@ -1293,3 +1293,31 @@ def test_layer_pointers_are_each_checked(dev, second, refusal):
         torch.cuda.synchronize()
         for p in (a, b, small):
             assert hip.hipFree(ctypes.c_void_p(p)) == 0
+
+
+@pytest.mark.parametrize("pieces", [1, 15, 16, 17, 127, 128])
+def test_small_copy_piece_lists(dev, pieces):
+    """Calls around the length of the small kernel's short piece list and its
+    longest, one piece per block, both ways."""
+    from flexkv_amd import c_ext
+    from flexkv_amd.storage.allocator import pinned_empty
+    chunk, pool = 1040, pieces + 5
+    gen = torch.Generator().manual_seed(pieces)
+    gids, cids = (torch.randperm(pool, generator=gen)[:pieces].contiguous() for _ in range(2))
+    cache = torch.randint(0, 256, (1, 1, pool, chunk), dtype=torch.uint8, device=dev)
+    host = pinned_empty(pool * chunk, torch.uint8).view(pool, chunk)
+    ptrs = torch.tensor([cache.data_ptr()], dtype=torch.int64)
+
+    def move(to_device):
+        c_ext.transfer_kv_blocks(gids, ptrs, pool * chunk, chunk, cids, host, chunk, chunk, chunk,
+                                 chunk, 0, -1, to_device, False, True)
+    host.zero_()
+    want = host.clone()
+    want[cids] = cache[0, 0].cpu()[gids]
+    move(False)
+    assert torch.equal(host, want)
+    host.bitwise_xor_(0x5A)
+    after = cache.cpu()
+    after[0, 0, gids] = host[cids]
+    move(True)
+    assert torch.equal(cache.cpu(), after)
