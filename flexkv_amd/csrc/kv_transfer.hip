@@ -1534,12 +1534,30 @@ size_t layerwise_min_copy_bytes() {
   return v > 0 ? static_cast<size_t>(v) : 1;
 }
 
-constexpr int kLayerwiseCeKernelGroups = 0;
+// Smallest engine copy per block of a window, for handles of at least
+// kLayerwiseShortMinBlocks blocks (with fewer, a window's copies take no longer
+// than the host's round trip between windows).  A window takes one engine copy
+// per block, about 0.75 us each over eight engines however short, so windows
+// that grew from one layer group and shrank to one spent a layer-wise load of a
+// tensor-parallel shard (8 KiB a block and layer) on copies of 8-64 KiB.
+// Windows now hold at least this much of a block, or as many groups as gpw
+// allows, and the groups before the first of them move with the zero-copy
+// kernel, one event each.  Measured on MI355X, us with windows from one group /
+// 32 / 64 / 128 KiB a block (and on the link):
+//   Llama-3-8B, 256 blocks            11115  10819  10789  10527   (9419)
+//   Llama-3-70B TP-8, 3072 blocks     64381  50645  44956  41220  (35320)
+//     192 blocks                       4216   3381   3181   3224   (2208)
+//     80 blocks                        1904   1619   1611   1759    (920)
+//     8-bit, 1024 blocks              17677  10695   9123   8303   (5887)
+//   MLA, 16 tokens, 477 blocks        12874  11845  11059  10717   (9409)
+//   Llama-3-8B, 4 tokens, 1000        17232  14804  12952  11757   (9198)
+constexpr size_t kLayerwiseShortCopyBytes = size_t(128) << 10;
+constexpr int kLayerwiseShortMinBlocks = 64;
 
 // Leading layer groups a copy-engine layer-wise handle moves with the
 // zero-copy kernel before its engines start (FLEXKV_LAYERWISE_CE_KERNEL_GROUPS,
-// default 0: every group on the engines; at most all groups but one).  A
-// one-group window is bound by the engines' per-copy cost (one copy per block
+// default: the groups whose windows would be shorter than the shortest the
+// engines get, `window` groups; at most all groups but one).  A one-group window is bound by the engines' per-copy cost (one copy per block
 // of one group's rows), while a consumer waiting for the first group has
 // nothing else to run, so the kernel's compute units cost it little then.
 // Measured on MI355X at the Llama-3-8B shape with one layer per group, one
@@ -1547,9 +1565,9 @@ constexpr int kLayerwiseCeKernelGroups = 0;
 // ends a prefill overlapped with 8 or 12 bf16 GEMMs per layer 1.1-1.7%
 // sooner, but one with 4 GEMMs per layer, which the transfer outlasts,
 // 0.5% later.
-int layerwise_kernel_lead_groups(int ngroups) {
+int layerwise_kernel_lead_groups(int ngroups, int window) {
   const char* e = getenv("FLEXKV_LAYERWISE_CE_KERNEL_GROUPS");
-  const int v = e ? atoi(e) : kLayerwiseCeKernelGroups;
+  const int v = e ? atoi(e) : window - 1;
   return std::max(0, std::min(v, ngroups - 1));
 }
 
@@ -1642,8 +1660,8 @@ int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
   // layers are contiguous in host memory: a full window carries at least
   // layerwise_min_copy_bytes() per block, which the engines move faster than
   // one-group copies.  Every group's event is recorded when the window
-  // holding it has landed.  Windows grow from one group (1, 2, 4, ...), so
-  // the first group arrives early, and near the end hold at most half of the
+  // holding it has landed.  Windows grow from the shortest (1, 2, 4, ... groups
+  // where one group's rows are long enough), so the first group arrives early, and near the end hold at most half of the
   // groups left, so the compute a window releases ends while the rest
   // arrive: a consumer that keeps up waits for one group's compute after the
   // last transfer, as with one group per window.
@@ -1657,12 +1675,17 @@ int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
     gpw = std::max(1, std::min(gpw, lpl / G));
     while (gpw > 1 && static_cast<size_t>(gpw) * group_row > half) --gpw;
   }
+  // groups of the shortest window
+  int window = 1;
+  if (g.num_blocks >= kLayerwiseShortMinBlocks)
+    window = static_cast<int>(std::min<size_t>(
+        static_cast<size_t>(gpw), (kLayerwiseShortCopyBytes + group_row - 1) / group_row));
   // The leading groups move with the zero-copy kernel, alone on the link;
   // the engines start on the next group once they have landed.
-  const int lead = layerwise_kernel_lead_groups(ngroups);
+  const int lead = layerwise_kernel_lead_groups(ngroups, window);
   std::vector<Piece> pieces;
-  for (int grp = lead, ramp = 1; grp < ngroups; ramp = std::min(2 * ramp, gpw)) {
-    const int take = std::min({gpw, ramp, std::max(1, (ngroups - grp) / 2)});
+  for (int grp = lead, ramp = window; grp < ngroups; ramp = std::min(2 * ramp, gpw)) {
+    const int take = std::min({gpw, ramp, std::max(window, (ngroups - grp) / 2), ngroups - grp});
     const int l0 = grp * G;
     const int nl = std::min(take * G, g.num_layers - l0);
     grp += take;

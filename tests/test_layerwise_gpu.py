@@ -540,3 +540,30 @@ def test_null_stream_consumer(n, own_queue, ce):
         for l, out in outs:
             want = np.stack([hv[c, l, :, 0] for c in cids], axis=1)
             assert np.array_equal(out.cpu().numpy().view(np.uint16), want), (rnd, l)
+
+
+@pytest.mark.parametrize("layers,n,heads,gran", [(20, 63, 1, 1), (20, 64, 1, 1), (20, 65, 1, 3),
+                                                 (5, 70, 1, 1), (40, 64, 1, 1), (2, 64, 8, 1),
+                                                 (1, 64, 1, 1), (33, 80, 4, 2)])
+def test_ce_pipeline_short_rows(layers, n, heads, gran):
+    """Copy-engine handles whose rows are short: the leading groups move with
+    the zero-copy kernel and the others in windows of several groups, from
+    64 blocks on.  Every group has landed when it alone is waited for."""
+    from gpu_util import DeviceCase
+    case = KVCase(layers_total=layers, num_layers=layers, start_layer=0, kv=2, ng=96, nh=90,
+                  tokens=16, heads=heads, dim=64).fill(seed=70 + n)
+    s = case.strides()
+    gids = inputs.distinct_ids(71, n, 96)
+    cids = inputs.distinct_ids(72, n, 90)
+    dc = DeviceCase(case)
+    dc.set_gpu([np.zeros_like(g) for g in case.gpu])
+    exp = [np.zeros_like(g) for g in case.gpu]
+    oracle.transfer_kv_blocks(gids, exp, s["gpu_kv"], s["gpu_block"], cids, case.host, s["cpu_kv"],
+                              s["cpu_layer"], s["cpu_block"], s["chunk"], 0, True)
+    with _abi_layerwise(dc, gids.copy(), cids.copy(), True, gran, ce=True) as hnd:
+        assert hnd.num_groups == -(-layers // gran)
+        for g in range(hnd.num_groups):
+            hnd.wait(g)
+            got = dc.gpu_np()
+            for l in range(g * gran, min(layers, (g + 1) * gran)):
+                assert np.array_equal(got[l], exp[l]), (g, l)
