@@ -457,12 +457,11 @@ constexpr int kAutoSmallCus = 8;
 // Copy-engine size policy: smallest transfer, and smallest bytes per engine
 // copy, worth handing to the SDMA engines (ce_pays_off).  Measured on MI355X
 // (block-wise host caches, random ids, GB/s zero-copy kernel / engines): the
-// kernel is as fast or faster up to 32 MiB in both directions at every shape
-// (16 MiB of 256 KiB rows: D2H 48.9 / 46.1, H2D 53.8 / 49.5; 8 MiB of 2 MiB
-// rows: 46.1 / 45.9, 50.0 / 45.8), and from 32-64 MiB the engines come
-// within 1-3% (32 MiB of 2 MiB rows: D2H 53.1 / 53.5, H2D 55.2 / 53.5; 64 MiB:
-// 54.8 / 55.2, 56.2 / 55.2).  Below 32 MiB the kernel holds its compute units
-// for at most about 0.6 ms per transfer.
+// kernel is faster at every size (8 MiB of 2 MiB rows: D2H 46.1 / 45.9, H2D
+// 50.0 / 45.8; 32 MiB: 55.3 / 53.5, 55.8 / 54.5; 64 MiB: 56.1 / 54.9, 56.7 /
+// 55.2; 256 MiB: 56.8 / 55.9, 57.3 / 56.2), by 2-4% from 32 MiB, where the
+// engines' leaving the compute units alone is worth more.  Below 32 MiB the
+// kernel holds its workgroups for at most about 0.6 ms per transfer.
 constexpr int64_t kCeMinBytesDefault = int64_t(32) << 20;
 constexpr int64_t kCeMinRunBytes = int64_t(128) << 10;
 // The copy-engine policy set through fkv_set_copy_engine_policy; -1: unset,
