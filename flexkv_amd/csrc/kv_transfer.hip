@@ -249,11 +249,13 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
 //   H2D 1 GiB       18781   18755   18673   18721   19112   19778
 //   D2H 16 MiB      315.6   311.1   312.6   317.3   315.0   312.7   310.1
 //   D2H 320 MiB      6083    5921    5954            6079    5967    5910
-// so 14 workgroups read (groups of 4 rows) and 12 write (8 rows).  A tiled
-// kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
+// so 14 workgroups read (groups of 4 rows).  Writing (8 rows) 12 and 32 are as
+// fast alone, but beside a transfer the other way 12 starve: 2 GiB each way at
+// once moves 69 GB/s with 12, 82-84 with 24-32 and 80 with 48, so 32 write.  A
+// tiled kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
 // 1 MiB host-to-device call of one layer (here 33.5).
 template <bool kH2D>
-constexpr int zero_copy_workgroups() { return kH2D ? 14 : 12; }
+constexpr int zero_copy_workgroups() { return kH2D ? 14 : 32; }
 template <bool kH2D>
 constexpr int zero_copy_rows() { return kH2D ? 4 : 8; }
 constexpr int kMaxItems = 2 * kMaxLayersPerLaunch;   // (layer, K|V) pairs of a launch
@@ -1880,8 +1882,8 @@ Geometry make_geometry(int num_blocks, int start_layer_id, int num_layers,
 // (D2H / H2D) at the Llama-3-8B shape, 82% of the link, against 56.5 /
 // 57.2 GB/s for the zero-copy kernel.  Such transfers therefore move with
 // the zero-copy kernel, which holds compute units for the whole transfer
-// (160 bf16 GEMMs queued after a 2 GiB D2H starts take 71 ms instead of
-// 36 ms beside the rect copies); fkv_set_copy_engine_policy (or
+// (bf16 GEMMs beside it take 1.05-2 times as long, by their order, and 1.02
+// times beside the rect copies); fkv_set_copy_engine_policy (or
 // FLEXKV_CE_RECT_COPIES=1) keeps them on the engines.
 bool ce_pays_off(const Geometry& g, bool h2d) {
   // a "host" cache that is device memory has no PCIe copy to offload

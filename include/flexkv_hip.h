@@ -92,7 +92,7 @@ enum {
  * Arguments follow flexkv::transfer_kv_blocks (csrc/transfer.cu:63-70) one for
  * one; `transfer_cus` plays the role of `transfer_sms` (compute units the
  * zero-copy kernel may occupy; -1 = no bound: it runs at most 14 workgroups
- * host-to-device and 12 device-to-host, which fill the link).
+ * host-to-device and 32 device-to-host, which fill the link).
  *
  * Host requirements (checked; violations return hipErrorInvalidValue):
  *   - gpu_block_ids, cpu_block_ids: host memory, num_blocks int64 each,
@@ -196,7 +196,7 @@ int fkv_scatter_kv_blocks(int num_blocks, int num_layers, const int64_t* gpu_blo
  * enqueued on `stream` before the call returns; fkv_handle_stream_wait makes
  * the other stream wait on the device, without a host round trip.
  * Small groups share launches of 1-4 MiB, and the event of the launch.
- * It runs at most 14 workgroups host-to-device and 12 device-to-host (enough
+ * It runs at most 14 workgroups host-to-device and 32 device-to-host (enough
  * for the link; the rest of the chip stays with the compute the transfer
  * overlaps), within transfer_cus compute units when that is given.
  * use_ce_transfer = FKV_XFER_CE (host to device from block-wise host rows;
