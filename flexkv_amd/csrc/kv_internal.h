@@ -101,7 +101,8 @@ struct CopyLane {
 struct DeviceState {
   bool init = false;
   int num_cus = 0;
-  int occ_zero_copy[2] = {0, 0};
+  // kv_zero_copy_kernel, [D2H, H2D][host cache in device memory, in host memory]
+  int occ_zero_copy[2][2] = {{1, 1}, {1, 1}};
   int occ_small[2] = {1, 1};   // kv_small_copy_kernel, D2H / H2D
   // Copy engines: the HSA agents of this GPU and of the host and the SDMA
   // engines each direction pins its copies to (disjoint sets where the device

@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "kv_internal.h"
+#include "kv_plan.h"
 
 using namespace fkv_detail;
 
@@ -254,10 +255,20 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
 // once moves 69 GB/s with 12, 82-84 with 24-32 and 80 with 48, so 32 write.  A
 // tiled kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
 // 1 MiB host-to-device call of one layer (here 33.5).
-template <bool kH2D>
-constexpr int zero_copy_workgroups() { return kH2D ? 14 : 32; }
-template <bool kH2D>
-constexpr int zero_copy_rows() { return kH2D ? 4 : 8; }
+//
+// kHost: the host cache lies in host memory.  One in device memory (!kHost) has
+// no link to wait for: loads in flight bound the launch, so it takes every
+// compute unit (zero_copy_workgroups), stores both ways with the non-temporal
+// hint alone, and finds a group's addresses once for the loads and again for
+// the stores, which leaves 44 registers and 8 wavefronts a SIMD (held through
+// 8 rows: 80 and 6; the copy then takes a third longer within few compute
+// units).  Measured on MI355X, us a device-to-host / host-to-device call,
+// within the host cache's grid and stores -> now: 64 MiB of 32 KiB chunks
+// 152 / 341 -> 38.3 / 38.5, 1 GiB 2208 / 5238 -> 433 / 435, 47 MiB of 2 KiB
+// chunks 118 / 258 -> 33.5 / 33.8; within 8 compute units 64 MiB 73.3 / 72.2,
+// 1 GiB 976 / 950.  12 and 16 rows: 1 GiB 440 / 445 and 440 / 440.
+template <bool kH2D, bool kHost>
+constexpr int zero_copy_rows() { return kHost && kH2D ? 4 : 8; }
 constexpr int kMaxItems = 2 * kMaxLayersPerLaunch;   // (layer, K|V) pairs of a launch
 // LDS for block offsets: with the item table, within the 64 KiB of a launch
 constexpr int kZeroCopyMaxLds = 56 << 10;
@@ -286,9 +297,9 @@ struct ZeroCopyArgs {
   int64_t inline_ids[2 * kInlineIdsZeroCopy];
 };
 
-template <bool kH2D>
+template <bool kH2D, bool kHost>
 __global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) {
-  constexpr int kU = zero_copy_rows<kH2D>();
+  constexpr int kU = zero_copy_rows<kH2D, kHost>();
   constexpr uint32_t kGroupVec = kU * 64;
   extern __shared__ int64_t s_block[];      // byte offsets (gpu, cpu) of the run's blocks
   __shared__ int64_t s_item[2 * kMaxItems]; // address (gpu), byte offset (cpu) of (layer, K|V)
@@ -328,32 +339,48 @@ __global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) 
   }
   __syncthreads();
   for (uint32_t g = g0 + wave; g < g1; g += kWaves) {
-    const uint32_t v0 = g * kGroupVec + lane;
-    const char* src[kU];
-    char* dst[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      // past the end a lane reloads the last vector and stores nothing
+    uint32_t v0 = g * kGroupVec + lane;
+    // the two addresses of the lane's vector in row u; past the end it reloads
+    // the last vector and stores nothing
+    auto locate = [&](int u, char** gpu, char** cpu) {
       const uint32_t v = min(v0 + u * 64, a.num_vec - 1);
       const uint32_t c = a.chunk.div(v);
       const uint32_t b = a.items.div(c);
       const uint32_t item = c - b * a.items.d;
       const int64_t off = static_cast<int64_t>(v - c * a.chunk.d) * 16;
-      char* gpu = reinterpret_cast<char*>(s_item[2 * item] + s_block[2 * (b - b0)] + off);
-      char* cpu = a.cpu_base + s_item[2 * item + 1] + s_block[2 * (b - b0) + 1] + off;
-      src[u] = kH2D ? cpu : gpu;
-      dst[u] = kH2D ? gpu : cpu;
-    }
+      *gpu = reinterpret_cast<char*>(s_item[2 * item] + s_block[2 * (b - b0)] + off);
+      *cpu = a.cpu_base + s_item[2 * item + 1] + s_block[2 * (b - b0) + 1] + off;
+    };
     u32x4 v[kU];
+    if constexpr (kHost) {
+      char *gpu[kU], *cpu[kU];
 #pragma unroll
-    for (int u = 0; u < kU; ++u) v[u] = __builtin_nontemporal_load((const gvec*)src[u]);
+      for (int u = 0; u < kU; ++u) locate(u, &gpu[u], &cpu[u]);
 #pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      if (v0 + u * 64 < a.num_vec) {
-        if (kH2D)
-          __builtin_nontemporal_store(v[u], (gvec*)dst[u]);
-        else
-          store_system(dst[u], v[u]);
+      for (int u = 0; u < kU; ++u)
+        v[u] = __builtin_nontemporal_load((const gvec*)(kH2D ? cpu[u] : gpu[u]));
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        if (v0 + u * 64 < a.num_vec) {
+          if (kH2D)
+            __builtin_nontemporal_store(v[u], (gvec*)gpu[u]);
+          else
+            store_system(cpu[u], v[u]);
+        }
+      }
+    } else {
+      char *gpu, *cpu;
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        locate(u, &gpu, &cpu);
+        v[u] = __builtin_nontemporal_load((const gvec*)(kH2D ? cpu : gpu));
+      }
+      asm("" : "+v"(v0));   // nothing of the addresses is kept for the stores
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        locate(u, &gpu, &cpu);
+        if (v0 + u * 64 < a.num_vec)
+          __builtin_nontemporal_store(v[u], (gvec*)(kH2D ? gpu : cpu));
       }
     }
   }
@@ -528,12 +555,16 @@ int ensure_device_basics(int dev) {
   FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
       &o, reinterpret_cast<void*>(&kv_small_copy_kernel<true, kSmallPieces>), kThreads, 0));
   d.occ_small[1] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &o, reinterpret_cast<void*>(&kv_zero_copy_kernel<false>), kThreads, 0));
-  d.occ_zero_copy[0] = std::max(1, o);
-  FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &o, reinterpret_cast<void*>(&kv_zero_copy_kernel<true>), kThreads, 0));
-  d.occ_zero_copy[1] = std::max(1, o);
+  const void* zero_copy[2][2] = {   // [D2H, H2D][device memory, host memory]
+      {reinterpret_cast<void*>(&kv_zero_copy_kernel<false, false>),
+       reinterpret_cast<void*>(&kv_zero_copy_kernel<false, true>)},
+      {reinterpret_cast<void*>(&kv_zero_copy_kernel<true, false>),
+       reinterpret_cast<void*>(&kv_zero_copy_kernel<true, true>)}};
+  for (int dir = 0; dir < 2; ++dir)
+    for (int host = 0; host < 2; ++host) {
+      FKV_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, zero_copy[dir][host], kThreads, 0));
+      d.occ_zero_copy[dir][host] = std::max(1, o);
+    }
   d.init = true;
   return 0;
 }
@@ -581,13 +612,10 @@ int64_t op_bytes(const Geometry& g) {
   return static_cast<int64_t>(g.num_blocks) * g.num_layers * g.kv * g.chunk;
 }
 
-// Workgroups of a zero-copy transfer on device `d`: the fastest count, within
-// `transfer_cus` compute units when the caller bounds them.
-int zero_copy_grid(const DeviceState& d, int transfer_cus, bool h2d) {
-  const int best = h2d ? zero_copy_workgroups<true>() : zero_copy_workgroups<false>();
-  return transfer_cus <= 0 ? best
-                           : std::min(best, std::min(transfer_cus, d.num_cus) *
-                                                d.occ_zero_copy[h2d ? 1 : 0]);
+// Workgroups of a zero-copy transfer of `g` on device `d`.
+int zero_copy_grid(const Geometry& g, const DeviceState& d, int transfer_cus, bool h2d) {
+  const bool host = !g.cpu_info.device;
+  return zero_copy_workgroups(h2d, host, transfer_cus, d.num_cus, d.occ_zero_copy[h2d][host]);
 }
 
 // Shape of a staging launch, by its size.  Measured on MI355X, us a gather /
@@ -722,7 +750,9 @@ template <bool kH2D>
 int launch_zero_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int l0, int nl,
                      int grid_cap, hipStream_t stream, ProfRecorder& prof, int32_t split = 0,
                      hipEvent_t done = nullptr) {
-  constexpr int64_t kGroupVec = zero_copy_rows<kH2D>() * 64;
+  const bool host = !g.cpu_info.device;
+  const int64_t group_vec = (host ? zero_copy_rows<kH2D, true>() : zero_copy_rows<kH2D, false>()) * 64;
+  const auto kernel = host ? kv_zero_copy_kernel<kH2D, true> : kv_zero_copy_kernel<kH2D, false>;
   const int64_t chunk_vec = g.chunk / 16;
   const int64_t part_max = std::min(chunk_vec, kZeroCopyMaxChunkVec);
   const int lw_max = static_cast<int>(std::min<int64_t>(
@@ -738,10 +768,10 @@ int launch_zero_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int l0
         int64_t nb = std::min<int64_t>(g.num_blocks - b0, kZeroCopyMaxVec / block_vec);
         int64_t groups, per_wg, span;
         for (;; nb = (nb + 1) / 2) {
-          groups = (nb * block_vec + kGroupVec - 1) / kGroupVec;
+          groups = (nb * block_vec + group_vec - 1) / group_vec;
           const int64_t wgs = std::min<int64_t>(std::max(1, grid_cap), (groups + kWaves - 1) / kWaves);
           per_wg = (groups + wgs - 1) / wgs;
-          span = std::min(nb, per_wg * kGroupVec / block_vec + 2);
+          span = std::min(nb, per_wg * group_vec / block_vec + 2);
           if (span * 16 <= kZeroCopyMaxLds || nb == 1) break;
         }
         a.ids = reinterpret_cast<const int64_t*>(ids.dev) + (split ? 1 : 2) * static_cast<int64_t>(b0);
@@ -775,8 +805,7 @@ int launch_zero_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int l0
         if (!eb && b0 == g.num_blocks && off + part == chunk_vec && lw + n_layers == l0 + nl)
           eb = done;
         (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-        hipExtLaunchKernelGGL((kv_zero_copy_kernel<kH2D>),
-                              dim3(static_cast<uint32_t>((groups + per_wg - 1) / per_wg)),
+        hipExtLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((groups + per_wg - 1) / per_wg)),
                               dim3(kThreads), static_cast<uint32_t>(span * 16), stream, ea, eb, 0, a);
         FKV_HIP(hipGetLastError());
       }
@@ -862,7 +891,7 @@ int transfer_zero_copy(const Geometry& g, hipStream_t stream, int dev, int trans
   int rc = pack_ids(g, ids);
   if (rc) return rc;
   DrainOnError drain{stream};
-  const int grid_cap = zero_copy_grid(d, transfer_cus, h2d);
+  const int grid_cap = zero_copy_grid(g, d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff +
                   static_cast<int64_t>(g.start_layer) * g.cls;
   ProfRecorder prof;
@@ -962,7 +991,7 @@ int transfer_zero_copy_noalloc(const Geometry& g, hipStream_t stream, int dev, i
     split = kScratchMaxBlocks;
   }
   DrainOnError drain{stream};
-  const int grid_cap = zero_copy_grid(d, transfer_cus, h2d);
+  const int grid_cap = zero_copy_grid(g, d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
   ProfRecorder prof;
   prof.on = false;   // profiling events are allocations
@@ -1452,7 +1481,7 @@ int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transf
   int rc = ids_acquire(static_cast<size_t>(g.num_blocks) * 16, &h->ids);
   if (rc) return rc;
   pack_ids_into(g, h->ids.host);
-  const int grid_cap = zero_copy_grid(d, transfer_cus, h2d);
+  const int grid_cap = zero_copy_grid(g, d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
   // Under capture the launches record plain events, as graph nodes.
   const bool captured = stream_captured(stream);
@@ -1601,7 +1630,7 @@ int layerwise_kernel_groups(fkv_transfer_handle_s* h, hipStream_t work, int firs
                             int end_group = -1) {
   const Geometry& g = h->geo;
   DeviceState& d = g_dev[h->dev];
-  const int grid_cap = zero_copy_grid(d, -1, true);
+  const int grid_cap = zero_copy_grid(g, d, -1, true);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;
   const int end_layer = end_group < 0 ? g.num_layers
                                       : std::min(g.num_layers, end_group * h->granularity);

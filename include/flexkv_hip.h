@@ -92,7 +92,8 @@ enum {
  * Arguments follow flexkv::transfer_kv_blocks (csrc/transfer.cu:63-70) one for
  * one; `transfer_cus` plays the role of `transfer_sms` (compute units the
  * zero-copy kernel may occupy; -1 = no bound: it runs at most 14 workgroups
- * host-to-device and 32 device-to-host, which fill the link).
+ * host-to-device and 32 device-to-host, which fill the link, and on every
+ * compute unit when cpu_ptr is device memory).
  *
  * Host requirements (checked; violations return hipErrorInvalidValue):
  *   - gpu_block_ids, cpu_block_ids: host memory, num_blocks int64 each,

@@ -1,0 +1,44 @@
+// CPU-only check of how transfers are cut and sized
+// (flexkv_amd/csrc/kv_plan.h): no HIP, no device.  Prints one line per case
+// and exits non-zero when one fails.
+#include "kv_plan.h"
+
+#include <cstdio>
+
+using namespace fkv_detail;
+
+namespace {
+
+int failures = 0;
+
+void check(bool ok, const char* what) {
+  std::printf("%s: %s\n", ok ? "ok" : "FAIL", what);
+  if (!ok) ++failures;
+}
+
+void device_memory_takes_the_chip() {
+  bool all = true, bounded = true, host = true;
+  for (int cus : {1, 32, 256})
+    for (int occ : {1, 4, 8})
+      for (bool h2d : {false, true}) {
+        all = all && zero_copy_workgroups(h2d, false, -1, cus, occ) == cus * occ;
+        all = all && zero_copy_workgroups(h2d, false, 0, cus, occ) == cus * occ;
+        for (int bound : {1, 2, 8, 31, 256, 1000}) {
+          const int n = zero_copy_workgroups(h2d, false, bound, cus, occ);
+          bounded = bounded && n == (bound < cus ? bound : cus) * occ;
+        }
+        const int most = h2d ? 14 : 32;
+        const int n = zero_copy_workgroups(h2d, true, -1, cus, occ);
+        host = host && n == (most < cus * occ ? most : cus * occ);
+      }
+  check(all, "a host cache in device memory takes every workgroup the device holds");
+  check(bounded, "and those of the caller's compute units when bounded");
+  check(host, "one in host memory takes what fills the link");
+}
+
+}  // namespace
+
+int main() {
+  device_memory_takes_the_chip();
+  return failures ? 1 : 0;
+}

@@ -425,6 +425,77 @@ def test_device_resident_cache_matches_oracle(dev, mode):
     assert np.array_equal(got, _oracle_d2h(case, gids, cids, mode))
 
 
+class ResidentCache:
+    """A block-wise "host" cache in device memory beside a device cache
+    [layer][kv][pool][chunk], both random."""
+
+    def __init__(self, dev, chunk, n, layers, kv, seed=0):
+        self.chunk, self.n, self.layers, self.kv, self.pool = chunk, n, layers, kv, n + 7
+        gen = torch.Generator(device=dev).manual_seed(seed + n)
+        self.gpu = torch.randint(-2**62, 2**62, (layers, kv, self.pool, chunk // 8),
+                                 dtype=torch.int64, device=dev, generator=gen)
+        self.host = torch.randint(-2**62, 2**62, (self.pool, layers, kv, chunk // 8),
+                                  dtype=torch.int64, device=dev, generator=gen)
+        perm = torch.Generator().manual_seed(seed)
+        self.gids, self.cids = (torch.randperm(self.pool, generator=perm)[:n].contiguous()
+                                for _ in range(2))
+        self.ptrs = torch.tensor([self.gpu[l].data_ptr() for l in range(layers)],
+                                 dtype=torch.int64)
+
+    def move(self, h2d, cus=-1):
+        from flexkv_amd import _lib
+        block = self.layers * self.kv * self.chunk
+        _lib.check(_lib.load().fkv_transfer_kv_blocks(
+            self.n, 0, self.layers, self.gids.data_ptr(), self.ptrs.data_ptr(),
+            self.pool * self.chunk, self.chunk, self.cids.data_ptr(), self.host.data_ptr(),
+            self.chunk, self.kv * self.chunk, block, 0, self.chunk,
+            torch.cuda.current_stream().cuda_stream, cus, int(h2d), 0, int(self.kv == 1)),
+            "fkv_transfer_kv_blocks")
+
+    def check_both_ways(self, cus=-1):
+        want = self.host.clone()
+        want[self.cids] = self.gpu[:, :, self.gids].permute(2, 0, 1, 3)
+        self.move(False, cus)
+        assert torch.equal(self.host, want)
+        self.host.bitwise_xor_(0x0F0F)
+        want = self.gpu.clone()
+        want[:, :, self.gids] = self.host[self.cids].permute(1, 2, 0, 3)
+        self.move(True, cus)
+        assert torch.equal(self.gpu, want)
+
+
+@pytest.mark.parametrize("chunk,n,layers,kv,cus", [
+    (16, 1, 1, 1, -1), (16, 97, 3, 2, 1), (1008, 96, 2, 1, -1), (8192, 7, 2, 2, 8),
+    (8208, 131, 1, 2, -1), (2304, 61, 61, 1, 1), (512, 700, 40, 2, -1), (16, 30000, 2, 2, 1),
+    (16, 30000, 2, 2, -1), (32768, 130, 32, 2, -1)])
+def test_device_resident_kernel_edges(dev, monkeypatch, chunk, n, layers, kv, cus):
+    """The zero-copy kernel's form for a "host" cache in device memory where
+    its rows meet chunk, block, group and launch ends, both ways."""
+    monkeypatch.setenv("FLEXKV_SMALL_KERNEL", "0")
+    ResidentCache(dev, chunk, n, layers, kv).check_both_ways(cus)
+
+
+@pytest.mark.parametrize("h2d", [False, True])
+@pytest.mark.parametrize("cus,rate", [(-1, 2.0e12), (8, 1.2e12)])
+def test_device_resident_cache_is_not_held_to_the_link(dev, h2d, cus, rate):
+    """A "host" cache in device memory moves at HBM rates, not with the few
+    workgroups that fill the host link: those give 0.4 / 1.0 TB/s (read and
+    write; host to device / back), the compute units' own 5 TB/s, and those
+    of 8 compute units 2.2 TB/s."""
+    from flexkv_amd import _lib
+    cache = ResidentCache(dev, 32768, 128, 32, 2)
+    cache.move(h2d, cus)
+    try:
+        _lib.profile_enable(True)
+        for _ in range(5):
+            cache.move(h2d, cus)
+        prof = _lib.profile_read()
+    finally:
+        _lib.profile_enable(False)
+    assert prof["kernel_launches"] == 5
+    assert 2 * prof["kernel_bytes"] / (prof["kernel_ms"] * 1e-3) > rate
+
+
 @pytest.mark.parametrize("layout", ["BLOCKWISE", "LAYERWISE"])
 def test_concurrent_threads_mixed_paths(dev, layout):
     """Four host threads, each with its own stream, move disjoint block sets
