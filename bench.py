@@ -850,9 +850,9 @@ def overlap_with_compute(wl: Workload, steps: int = 3, gemms: int = 160,
             finally:
                 if ce and rect_copies:
                     c_ext.set_copy_engine_policy(layerwise_scattered="unset")
-    # The zero-copy H2D bounded by a larger compute-unit count (transfer_cus = a
-    # CU count / 8) than the 14 workgroups it uses at most: the bound should
-    # change nothing.
+    # The zero-copy H2D with its grid spread over the chip (transfer_cus = a CU
+    # count / 8: about one workgroup per compute unit) instead of the 14
+    # workgroups it takes by itself.
     spread = max(1, torch.cuda.get_device_properties(wl.dev).multi_processor_count // 8)
     for key, window, store, alone in (("h2d_kernel_spread", gemm_window, out, out),
                                       ("h2d_kernel_spread", gemm_window_transfer_first, tf,

@@ -82,8 +82,9 @@ def transfer_kv_blocks(gpu_block_id_tensor: torch.Tensor,
     engines behind an on-device gather/scatter through staging; the integer 2
     selects the reference's one-DMA-per-chunk loop (csrc/transfer.cu:97-121).
     ``transfer_sms`` bounds the compute units of the zero-copy kernel
-    (-1 = automatic).  ``stream`` (keyword only, an extension) is a raw
-    stream handle to run on instead of the current torch stream.
+    (-1 = automatic; more than 8 spread its grid over as many).  ``stream``
+    (keyword only, an extension) is a raw stream handle to run on instead of
+    the current torch stream.
 
     The compiled module ``_fkv_py`` unpacks and checks the tensors, takes the
     current stream and calls ``fkv_transfer_kv_blocks`` with the GIL released;

@@ -91,9 +91,11 @@ enum {
  *
  * Arguments follow flexkv::transfer_kv_blocks (csrc/transfer.cu:63-70) one for
  * one; `transfer_cus` plays the role of `transfer_sms` (compute units the
- * zero-copy kernel may occupy; -1 = no bound: it runs at most 14 workgroups
- * host-to-device and 32 device-to-host, which fill the link, and on every
- * compute unit when cpu_ptr is device memory).
+ * zero-copy kernel may occupy; -1 = no bound).  Over host memory it runs at most
+ * 14 workgroups host-to-device and 32 device-to-host, which fill the link, and
+ * with more than 8 compute units named every workgroup those hold, a grid spread
+ * over the chip.  When cpu_ptr is device memory it fills the compute units it may
+ * occupy.
  *
  * Host requirements (checked; violations return hipErrorInvalidValue):
  *   - gpu_block_ids, cpu_block_ids: host memory, num_blocks int64 each,
@@ -199,7 +201,7 @@ int fkv_scatter_kv_blocks(int num_blocks, int num_layers, const int64_t* gpu_blo
  * Small groups share launches of 1-4 MiB, and the event of the launch.
  * It runs at most 14 workgroups host-to-device and 32 device-to-host (enough
  * for the link; the rest of the chip stays with the compute the transfer
- * overlaps), within transfer_cus compute units when that is given.
+ * overlaps); transfer_cus bounds or raises that as in fkv_transfer_kv_blocks.
  * use_ce_transfer = FKV_XFER_CE (host to device from block-wise host rows;
  * other transfers take the kernel): the copy engines, so the transfer holds
  * no compute unit while its bytes cross the link.  A library thread moves

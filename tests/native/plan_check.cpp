@@ -36,9 +36,27 @@ void device_memory_takes_the_chip() {
   check(host, "one in host memory takes what fills the link");
 }
 
+void transfer_cus_bounds_and_spreads() {
+  bool bounds = true, spreads = true;
+  for (bool h2d : {false, true})
+    for (int occ : {4, 8}) {
+      const int most = h2d ? 14 : 32;
+      for (int cus = 1; cus <= 8; ++cus) {
+        const int n = zero_copy_workgroups(h2d, true, cus, 256, occ);
+        bounds = bounds && n == (most < cus * occ ? most : cus * occ);
+      }
+      for (int cus : {9, 32, 64, 256, 4096})
+        spreads = spreads && zero_copy_workgroups(h2d, true, cus, 256, occ) ==
+                                 (cus < 256 ? cus : 256) * occ;
+    }
+  check(bounds, "up to 8 compute units bound a transfer over the link");
+  check(spreads, "more of them are all filled");
+}
+
 }  // namespace
 
 int main() {
   device_memory_takes_the_chip();
+  transfer_cus_bounds_and_spreads();
   return failures ? 1 : 0;
 }
