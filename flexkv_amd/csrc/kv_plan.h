@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <vector>
 
 namespace fkv_detail {
 
@@ -35,6 +36,18 @@ inline int zero_copy_workgroups(bool h2d, bool host_memory, int transfer_cus, in
   return !host_memory || transfer_cus > kZeroCopySpreadCus
              ? held
              : std::min(h2d ? kZeroCopyReaders : kZeroCopyWriters, held);
+}
+
+// One past the last layer group that a legacy null stream's wait on `group`'s
+// event also waits for: with `ordered` (the stream that records the events is
+// one the null stream waits for by itself) every group queued so far, else only
+// the groups after `group` that share its event.
+template <class Event>
+int null_wait_covers(const std::vector<Event>& done, int group, int queued, bool ordered) {
+  if (ordered) return queued;
+  int end = group + 1;
+  while (end < static_cast<int>(done.size()) && done[end] == done[group]) ++end;
+  return end;
 }
 
 }  // namespace fkv_detail

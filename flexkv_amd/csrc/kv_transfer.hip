@@ -1390,9 +1390,9 @@ struct fkv_transfer_handle_s {
   hipStream_t stream = nullptr;
   std::vector<hipEvent_t> done;   // per layer group, in order; groups of one launch share one
   std::vector<hipEvent_t> events; // the distinct events of `done`
-  // Kernel path: one past the last group whose transfer group i's event also
-  // covers on the legacy null stream (see fkv_handle_stream_wait).
-  std::vector<int> null_covers;
+  // the stream that records the groups' events is one the legacy null stream
+  // waits for by itself (see fkv_handle_stream_wait)
+  bool null_ordered = false;
   int null_upto = 0;              // groups the device's legacy null stream waits for (mu)
   IdBuf ids;
   DevIdLease dev_ids;             // copy-engine pipeline: the gpu ids of its scatters
@@ -1488,7 +1488,7 @@ int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transf
   // A launch's event rides on its kernel's packet, host-to-device only: a
   // device-to-host group's event has to release to the host.
   const bool on_kernel = h2d && !h->prof.on && !captured;
-  const bool null_ordered = !captured && stream_blocks_null(stream);
+  h->null_ordered = !captured && stream_blocks_null(stream);
   const int ngroups = (g.num_layers + granularity - 1) / granularity;
   const int64_t group_bytes = static_cast<int64_t>(g.num_blocks) *
                               std::min(granularity, g.num_layers) * g.kv * g.chunk;
@@ -1516,8 +1516,6 @@ int layerwise_enqueue(const Geometry& g, hipStream_t stream, int dev, int transf
     if (rc) return rc;
     if (!on_kernel) FKV_HIP(hipEventRecord(ev, stream));
     h->done.insert(h->done.end(), static_cast<size_t>(take), ev);
-    h->null_covers.insert(h->null_covers.end(), static_cast<size_t>(take),
-                          null_ordered ? ngroups : gend);
     grp = gend;
   }
   h->enqueued = true;
@@ -1847,6 +1845,7 @@ int layerwise_ce_start(const Geometry& g, hipStream_t stream, int dev, int granu
   pack_ids_into(h->geo, h->ids.host);
   hipStream_t work = nullptr;
   if ((rc = pipeline_stream(g_dev[dev].lane[1], dev, &work))) return rc;
+  h->null_ordered = stream_blocks_null(work);
   for (int g0 = 0; g0 < g.num_layers; g0 += granularity) {
     hipEvent_t ev = nullptr;
     FKV_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -2182,9 +2181,8 @@ int fkv_handle_stream_wait(fkv_transfer_handle h, int group, fkv_stream_t other)
   if (!st && cur == h->dev) {
     std::lock_guard<std::mutex> lk(h->mu);
     if (group < h->null_upto) return 0;
-    // the pipeline stream, which records a copy-engine handle's events, is a
-    // blocking one
-    const int covers = h->ce ? h->recorded : h->null_covers[group];
+    const int queued = h->ce ? h->recorded : static_cast<int>(h->done.size());
+    const int covers = null_wait_covers(h->done, group, queued, h->null_ordered);
     FKV_HIP(hipStreamWaitEvent(st, h->done[group], 0));
     h->null_upto = std::max(h->null_upto, covers);
     return 0;

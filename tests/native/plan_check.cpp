@@ -53,9 +53,23 @@ void transfer_cus_bounds_and_spreads() {
   check(spreads, "more of them are all filled");
 }
 
+void null_stream_waits_cover_what_they_wait_for() {
+  const std::vector<int> done = {1, 1, 1, 2, 3, 3};   // groups of one launch share an event
+  bool ordered = true, alone = true;
+  const int shared_end[] = {3, 3, 3, 4, 6, 6};
+  for (int g = 0; g < 6; ++g)
+    for (int queued = g + 1; queued <= 6; ++queued) {
+      ordered = ordered && null_wait_covers(done, g, queued, true) == queued;
+      alone = alone && null_wait_covers(done, g, queued, false) == shared_end[g];
+    }
+  check(ordered, "a wait behind a blocking stream covers every group queued on it");
+  check(alone, "one behind any other stream covers the groups of its own event");
+}
+
 }  // namespace
 
 int main() {
+  null_stream_waits_cover_what_they_wait_for();
   device_memory_takes_the_chip();
   transfer_cus_bounds_and_spreads();
   return failures ? 1 : 0;
