@@ -567,3 +567,82 @@ def test_ce_pipeline_short_rows(layers, n, heads, gran):
             got = dc.gpu_np()
             for l in range(g * gran, min(layers, (g + 1) * gran)):
                 assert np.array_equal(got[l], exp[l]), (g, l)
+
+
+class EngineReader:
+    """Copies device memory to host memory with an SDMA engine through HSA
+    alone: no HIP stream, no kernel and no packet of its own that would write
+    the compute units' caches back first."""
+
+    def __init__(self):
+        # the runtime HIP has loaded (torch brings one of its own)
+        with open("/proc/self/maps") as f:
+            lib = next(l.split()[-1] for l in f if "libhsa-runtime64" in l)
+        self.hsa = ctypes.CDLL(lib)
+        u64, p = ctypes.c_uint64, ctypes.c_void_p
+        self.hsa.hsa_amd_memory_async_copy.argtypes = [p, u64, p, u64, ctypes.c_size_t,
+                                                       ctypes.c_uint32, p, u64]
+        self.hsa.hsa_signal_store_screlease.argtypes = [u64, ctypes.c_int64]
+        self.hsa.hsa_signal_wait_scacquire.argtypes = [u64, ctypes.c_int, ctypes.c_int64, u64,
+                                                       ctypes.c_int]
+        self.hsa.hsa_signal_wait_scacquire.restype = ctypes.c_int64
+        assert self.hsa.hsa_init() == 0
+        agents = {}
+
+        @ctypes.CFUNCTYPE(ctypes.c_int, u64, p)
+        def each(agent, _):
+            kind = ctypes.c_int()
+            self.hsa.hsa_agent_get_info(u64(agent), 17, ctypes.byref(kind))   # HSA_AGENT_INFO_DEVICE
+            agents.setdefault(kind.value, agent)                              # 0: CPU, 1: GPU
+            return 0
+        assert self.hsa.hsa_iterate_agents(each, None) == 0
+        self.cpu, self.gpu = agents[0], agents[1]
+        self.signal = u64()
+        assert self.hsa.hsa_signal_create(ctypes.c_int64(1), 0, None,
+                                          ctypes.byref(self.signal)) == 0
+
+    def read(self, dst: torch.Tensor, src: int) -> None:
+        sig = self.signal.value
+        self.hsa.hsa_signal_store_screlease(sig, 1)
+        assert self.hsa.hsa_amd_memory_async_copy(dst.data_ptr(), self.cpu, src, self.gpu,
+                                                  dst.numel() * dst.element_size(), 0, None,
+                                                  sig) == 0
+        # HSA_SIGNAL_CONDITION_LT 1; in the timestamp clock's ticks, seconds
+        assert self.hsa.hsa_signal_wait_scacquire(sig, 2, 1, 1 << 30, 0) == 0
+
+    def close(self):
+        self.hsa.hsa_signal_destroy(self.signal)
+        self.hsa.hsa_shut_down()
+
+
+@pytest.mark.parametrize("ce", [False, True], ids=["kernel", "ce"])
+@pytest.mark.parametrize("n", [1, 3, 16, 40])
+def test_groups_are_in_memory_when_their_event_is_seen(n, ce):
+    """A group the host has waited for is read from memory by an SDMA engine,
+    which does not look into the compute units' caches (as a network card or
+    another GPU would not): the bytes of groups whose event rides on the
+    transfer kernel's own packet have left those caches too."""
+    from flexkv_amd.storage.allocator import pinned_empty
+    from gpu_util import DeviceCase
+    L = 12
+    case = KVCase(layers_total=L, num_layers=L, start_layer=0, kv=2, ng=n, nh=n, tokens=16,
+                  heads=8, dim=128).fill(seed=130 + n)
+    ids = np.arange(n, dtype=np.int64)
+    dc = DeviceCase(case)
+    got = pinned_empty(dc.gpu[0].numel(), dc.gpu[0].dtype)
+    reader = EngineReader()
+    try:
+        for rnd in range(6):
+            fresh = case.host ^ np.uint16(0x1111 * (rnd + 1))
+            hv = case.host_view(fresh)
+            dc.set_host(fresh)
+            torch.cuda.synchronize()
+            with _abi_layerwise(dc, ids.copy(), ids.copy(), True, 1, ce=ce) as hnd:
+                for l in range(L):
+                    hnd.wait(l)
+                    reader.read(got, dc.gpu[l].data_ptr())
+                    want = np.stack([hv[c, l, :, 0] for c in ids], axis=1)
+                    assert np.array_equal(got.numpy().view(np.uint16).reshape(want.shape), want), \
+                        (rnd, l)
+    finally:
+        reader.close()
