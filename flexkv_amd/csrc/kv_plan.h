@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cstdint>
 #include <vector>
 
 namespace fkv_detail {
@@ -36,6 +37,99 @@ inline int zero_copy_workgroups(bool h2d, bool host_memory, int transfer_cus, in
   return !host_memory || transfer_cus > kZeroCopySpreadCus
              ? held
              : std::min(h2d ? kZeroCopyReaders : kZeroCopyWriters, held);
+}
+
+// What one staging launch moves: blocks [b, b + nb) of the piece, items (layer,
+// K|V) [item, item + items), and of each of their chunks the 16-byte vectors
+// [off, off + vec).  `packed`: where in the staging buffer, in vectors.
+struct StagingPart {
+  int b, nb;
+  int64_t item, items, off, vec, packed;
+};
+
+// Cuts a staging gather / scatter of `nb` blocks of `items` chunks of `chunk_vec`
+// vectors into launches of at most `max_vec` vectors, each contiguous in the
+// staging buffer (block -> item -> chunk or, `layer_major`, item -> block ->
+// chunk): one, or whole blocks at a time, or one item at a time over as many
+// blocks as are contiguous there, or parts of one chunk.  Ends at the first
+// launch that returns an error, and returns it.
+template <class Launch>
+int staging_launches(int nb, int64_t items, int64_t chunk_vec, bool layer_major, int64_t max_vec,
+                     Launch&& launch) {
+  const int64_t block_vec = items * chunk_vec;
+  int rc = 0;
+  if (nb * block_vec <= max_vec) return launch(StagingPart{0, nb, 0, items, 0, chunk_vec, 0});
+  if (!layer_major && block_vec <= max_vec) {
+    const int step = static_cast<int>(max_vec / block_vec);
+    for (int b = 0; b < nb && !rc; b += step)
+      rc = launch(StagingPart{b, std::min(step, nb - b), 0, items, 0, chunk_vec, b * block_vec});
+    return rc;
+  }
+  const int64_t part = std::min(chunk_vec, max_vec);
+  const int step =
+      layer_major && part == chunk_vec ? static_cast<int>(std::min<int64_t>(nb, max_vec / part)) : 1;
+  for (int64_t i = 0; i < items && !rc; ++i)
+    for (int b = 0; b < nb && !rc; b += step)
+      for (int64_t off = 0; off < chunk_vec && !rc; off += part)
+        rc = launch(StagingPart{b, std::min(step, nb - b), i, 1, off, std::min(part, chunk_vec - off),
+                                (layer_major ? i * nb + b : b * items + i) * chunk_vec + off});
+  return rc;
+}
+
+// What one zero-copy launch moves: blocks [b, b + nb) of the call, layers
+// [layer, layer + layers) of the window, and of each of their chunks the vectors
+// [off, off + vec).  Its num_vec vectors are cut into `groups`, groups_per_wg
+// consecutive ones a workgroup, whose run touches at most run_blocks blocks.
+struct ZeroCopyPart {
+  int b, nb, layer, layers;
+  int64_t off, vec, num_vec, groups, groups_per_wg, run_blocks;
+  bool last;   // of the transfer's launches
+  int64_t workgroups() const { return (groups + groups_per_wg - 1) / groups_per_wg; }
+};
+
+struct ZeroCopyLimits {
+  int64_t max_vec;       // vectors of a launch
+  int64_t max_part;      // vectors of a launch's chunk parts
+  int64_t run_blocks;    // blocks of a workgroup's run
+  int layers;            // layers of a launch
+};
+
+// Cuts a zero-copy transfer of `num_blocks` blocks and `nl` layers of `kv` chunks
+// of `chunk_vec` vectors into launches of groups of `group_vec` vectors over at
+// most `grid` workgroups of `waves` wavefronts: one launch, but for layers, parts
+// of chunks and blocks beyond the limits.  Ends at the first launch that returns
+// an error, and returns it.
+template <class Launch>
+int zero_copy_launches(int num_blocks, int nl, int kv, int64_t chunk_vec, int64_t group_vec,
+                       int waves, int grid, const ZeroCopyLimits& lim, Launch&& launch) {
+  const int64_t part_max = std::min(chunk_vec, lim.max_part);
+  const int layers_max = static_cast<int>(std::min<int64_t>(
+      {nl, lim.layers, std::max<int64_t>(1, lim.max_vec / (kv * part_max))}));
+  for (int layer = 0; layer < nl; layer += layers_max)
+    for (int64_t off = 0; off < chunk_vec; off += part_max) {
+      ZeroCopyPart p;
+      p.layer = layer;
+      p.layers = std::min(layers_max, nl - layer);
+      p.off = off;
+      p.vec = std::min(part_max, chunk_vec - off);
+      const int64_t block_vec = static_cast<int64_t>(p.layers) * kv * p.vec;
+      for (p.b = 0; p.b < num_blocks; p.b += p.nb) {
+        int64_t nb = std::min<int64_t>(num_blocks - p.b, lim.max_vec / block_vec);
+        for (;; nb = (nb + 1) / 2) {
+          p.groups = (nb * block_vec + group_vec - 1) / group_vec;
+          const int64_t wgs = std::min<int64_t>(std::max(1, grid), (p.groups + waves - 1) / waves);
+          p.groups_per_wg = (p.groups + wgs - 1) / wgs;
+          p.run_blocks = std::min(nb, p.groups_per_wg * group_vec / block_vec + 2);
+          if (p.run_blocks <= lim.run_blocks || nb == 1) break;
+        }
+        p.nb = static_cast<int>(nb);
+        p.num_vec = nb * block_vec;
+        p.last = p.b + p.nb == num_blocks && off + p.vec == chunk_vec && layer + p.layers == nl;
+        const int rc = launch(static_cast<const ZeroCopyPart&>(p));
+        if (rc) return rc;
+      }
+    }
+  return 0;
 }
 
 // One past the last layer group that a legacy null stream's wait on `group`'s

@@ -664,88 +664,67 @@ template <bool kH2D>
 int launch_staging(const Geometry& g, const StageTable& table, char* packed, bool layer_major,
                    int b0, int nb, int l0, int nl, int dev, hipStream_t stream,
                    ProfRecorder& prof) {
-  const int64_t chunk_vec = g.chunk / 16;
-  // chunks of blocks [b, b + cb) and items (layer x K|V) [i, i + ci), all but
-  // `off` vectors of them
+  const int64_t items = static_cast<int64_t>(nl) * g.kv;
   PackArgs pa;
-  auto launch = [&](int b, int cb, int64_t i, int64_t ci, int64_t off, int64_t part,
-                    char* at) -> int {
-    const int64_t chunks = cb * ci;
+  return staging_launches(nb, items, g.chunk / 16, layer_major, kPackMaxVec,
+                          [&](const StagingPart& p) -> int {
+    const int b = b0 + p.b;
+    const int64_t chunks = p.nb * p.items;
     // one item: its pointer with K|V applied
-    const bool one = ci == 1;
-    const int64_t l = i / g.kv;
-    const int lp = static_cast<int>(one ? 1 : ci / g.kv);
+    const bool one = p.items == 1;
+    const int64_t l = p.item / g.kv;
+    const int lp = static_cast<int>(one ? 1 : p.items / g.kv);
     const bool wide = !one && lp > g.layers_per_launch();
-    if ((cb > kPackInlineIds && !table.gids) || (wide && !table.ptrs))
+    if ((p.nb > kPackInlineIds && !table.gids) || (wide && !table.ptrs))
       return fail(kInval, "internal: a staging launch of %d blocks and %d layers without its "
-                  "tables", cb, lp);
+                  "tables", p.nb, lp);
     pa.gids = table.gids ? table.gids + b : nullptr;
-    if (!pa.gids) memcpy(pa.inline_ids, g.gids + b, sizeof(int64_t) * cb);
+    if (!pa.gids) memcpy(pa.inline_ids, g.gids + b, sizeof(int64_t) * p.nb);
     pa.ptrs = nullptr;
     if (one)
       pa.layer_ptr[0] = reinterpret_cast<uint64_t>(
-          g.gpu_base(l0 + static_cast<int>(l), static_cast<int>(i % g.kv)) + off * 16);
+          g.gpu_base(l0 + static_cast<int>(l), static_cast<int>(p.item % g.kv)) + p.off * 16);
     else if (wide)
       pa.ptrs = table.ptrs + (l0 + l) * g.ptrs_per_layer;
     else
       memcpy(pa.layer_ptr, g.layer_ptrs + (l0 + l) * g.ptrs_per_layer,
              sizeof(uint64_t) * lp * g.ptrs_per_layer);
-    pa.packed = at;
+    pa.packed = packed + p.packed * 16;
     pa.gpu_kv_stride = g.gks;
     pa.gpu_block_stride = g.gbs;
-    pa.chunk = Divider(static_cast<uint32_t>(part));
-    pa.inner = Divider(static_cast<uint32_t>(layer_major ? cb : ci));
+    pa.chunk = Divider(static_cast<uint32_t>(p.vec));
+    pa.inner = Divider(static_cast<uint32_t>(layer_major ? p.nb : p.items));
     pa.layer_major = layer_major;
     pa.kv_dim = one ? 1 : static_cast<uint32_t>(g.kv);
     pa.ptrs_per_layer = one ? 1 : g.ptrs_per_layer;
     pa.num_chunks = static_cast<uint32_t>(chunks);
-    pa.num_vec = static_cast<uint32_t>(chunks * part);
+    pa.num_vec = static_cast<uint32_t>(chunks * p.vec);
     hipEvent_t ea = nullptr, eb = nullptr;
     int rc = prof.kernel_events(&ea, &eb);
     if (rc) return rc;
-    prof.kernel_span(ea, eb, chunks * part * 16);   // owns the events from here on
+    prof.kernel_span(ea, eb, chunks * p.vec * 16);   // owns the events from here on
     (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
     const uint32_t num_cus = static_cast<uint32_t>(g_dev[dev].num_cus);
-    if (pack_fits(32, part) && pa.num_vec >= int64_t(num_cus) * kWaves * 32 * 64)
+    if (pack_fits(32, p.vec) && pa.num_vec >= int64_t(num_cus) * kWaves * 32 * 64)
       launch_pack<kH2D, 32>(pa, num_cus, stream, ea, eb);
-    else if (pack_fits(8, part))
+    else if (pack_fits(8, p.vec))
       launch_pack<kH2D, 8>(pa, num_cus, stream, ea, eb);
     else
       launch_pack<kH2D, 1>(pa, num_cus, stream, ea, eb);
     FKV_HIP(hipGetLastError());
     return 0;
-  };
-  const int64_t items = static_cast<int64_t>(nl) * g.kv;
-  const int64_t block_vec = items * chunk_vec;
-  int rc = 0;
-  if (nb * block_vec <= kPackMaxVec) return launch(b0, nb, 0, items, 0, chunk_vec, packed);
-  if (!layer_major && block_vec <= kPackMaxVec) {
-    const int step = static_cast<int>(kPackMaxVec / block_vec);
-    for (int b = 0; b < nb && !rc; b += step)
-      rc = launch(b0 + b, std::min(step, nb - b), 0, items, 0, chunk_vec,
-                  packed + b * block_vec * 16);
-    return rc;
-  }
-  // one (layer, K|V) at a time: runs of blocks where they are contiguous
-  const int64_t part_max = std::min(chunk_vec, kPackMaxVec);
-  const int step = layer_major ? static_cast<int>(std::min<int64_t>(nb, kPackMaxVec / part_max)) : 1;
-  for (int64_t i = 0; i < items && !rc; ++i)
-    for (int b = 0; b < nb && !rc; b += step)
-      for (int64_t off = 0; off < chunk_vec && !rc; off += part_max)
-        rc = launch(b0 + b, std::min(step, nb - b), i, 1, off, std::min(part_max, chunk_vec - off),
-                    packed + ((layer_major ? i * nb + b : b * items + i) * chunk_vec + off) * 16);
-  return rc;
+  });
 }
 
 // Launch kv_zero_copy_kernel over call layers [l0, l0 + nl) of every block of
 // the call.  `cpu_base` is the host-side address of call layer 0 of block id
 // 0; `ids` holds the packed pairs: `host` for the host's view, `dev` for the
 // device's (the same pinned buffer), or with `split` > 0 `dev` holds the gpu
-// ids and, `split` entries later, the cpu ids, and `host` is null; at most `grid_cap` workgroups a
-// launch.  One launch, but for layers beyond the pointers a launch carries
-// and for runs beyond what Divider or a workgroup's LDS takes.  `done` (null
-// while profiling): an event the last launch completes, carried by its own
-// packet instead of a marker behind it.
+// ids and, `split` entries later, the cpu ids, and `host` is null; at most
+// `grid_cap` workgroups a launch.  The limits are those of the layer pointers a
+// launch carries, of Divider and of a workgroup's LDS.  `done` (null while
+// profiling): an event the last launch completes, carried by its own packet
+// instead of a marker behind it.
 template <bool kH2D>
 int launch_zero_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int l0, int nl,
                      int grid_cap, hipStream_t stream, ProfRecorder& prof, int32_t split = 0,
@@ -753,64 +732,46 @@ int launch_zero_copy(const Geometry& g, const IdBuf& ids, char* cpu_base, int l0
   const bool host = !g.cpu_info.device;
   const int64_t group_vec = (host ? zero_copy_rows<kH2D, true>() : zero_copy_rows<kH2D, false>()) * 64;
   const auto kernel = host ? kv_zero_copy_kernel<kH2D, true> : kv_zero_copy_kernel<kH2D, false>;
-  const int64_t chunk_vec = g.chunk / 16;
-  const int64_t part_max = std::min(chunk_vec, kZeroCopyMaxChunkVec);
-  const int lw_max = static_cast<int>(std::min<int64_t>(
-      {nl, g.layers_per_launch(), std::max<int64_t>(1, kZeroCopyMaxVec / (g.kv * part_max))}));
+  const ZeroCopyLimits limits{kZeroCopyMaxVec, kZeroCopyMaxChunkVec, kZeroCopyMaxLds / 16,
+                              g.layers_per_launch()};
   ZeroCopyArgs a;
-  for (int lw = l0; lw < l0 + nl; lw += lw_max)
-    for (int64_t off = 0; off < chunk_vec; off += part_max) {
-      const int n_layers = std::min(lw_max, l0 + nl - lw);
-      const int64_t part = std::min(part_max, chunk_vec - off);
-      const int64_t block_vec = n_layers * g.kv * part;
-      for (int b0 = 0; b0 < g.num_blocks;) {
-        // blocks of the launch: as many as its vectors and a run's LDS allow
-        int64_t nb = std::min<int64_t>(g.num_blocks - b0, kZeroCopyMaxVec / block_vec);
-        int64_t groups, per_wg, span;
-        for (;; nb = (nb + 1) / 2) {
-          groups = (nb * block_vec + group_vec - 1) / group_vec;
-          const int64_t wgs = std::min<int64_t>(std::max(1, grid_cap), (groups + kWaves - 1) / kWaves);
-          per_wg = (groups + wgs - 1) / wgs;
-          span = std::min(nb, per_wg * group_vec / block_vec + 2);
-          if (span * 16 <= kZeroCopyMaxLds || nb == 1) break;
-        }
-        a.ids = reinterpret_cast<const int64_t*>(ids.dev) + (split ? 1 : 2) * static_cast<int64_t>(b0);
-        a.ids_split = split;
-        a.inline_n = 0;
-        if (nb <= kInlineIdsZeroCopy && ids.host) {
-          a.inline_n = static_cast<int32_t>(nb);
-          memcpy(a.inline_ids, ids.host + 2 * static_cast<int64_t>(b0), sizeof(int64_t) * 2 * nb);
-        }
-        a.cpu_base = cpu_base + static_cast<int64_t>(lw) * g.cls + off * 16;
-        a.gpu_kv_stride = g.gks;
-        a.gpu_block_stride = g.gbs;
-        a.cpu_kv_stride = g.cks;
-        a.cpu_layer_stride = g.cls;
-        a.cpu_block_stride = g.cbs;
-        a.chunk = Divider(static_cast<uint32_t>(part));
-        a.items = Divider(static_cast<uint32_t>(n_layers * g.kv));
-        a.kv_dim = static_cast<uint32_t>(g.kv);
-        a.num_vec = static_cast<uint32_t>(nb * block_vec);
-        a.num_groups = static_cast<uint32_t>(groups);
-        a.groups_per_wg = static_cast<uint32_t>(per_wg);
-        a.ptrs_per_layer = g.ptrs_per_layer;
-        for (int i = 0; i < n_layers * g.ptrs_per_layer; ++i)
-          a.layer_ptr[i] = reinterpret_cast<uint64_t>(g.layer_ptrs[lw * g.ptrs_per_layer + i]) +
-                           static_cast<uint64_t>(off) * 16;
-        b0 += static_cast<int>(nb);
-        hipEvent_t ea = nullptr, eb = nullptr;
-        int rc = prof.kernel_events(&ea, &eb);
-        if (rc) return rc;
-        prof.kernel_span(ea, eb, nb * block_vec * 16);
-        if (!eb && b0 == g.num_blocks && off + part == chunk_vec && lw + n_layers == l0 + nl)
-          eb = done;
-        (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
-        hipExtLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((groups + per_wg - 1) / per_wg)),
-                              dim3(kThreads), static_cast<uint32_t>(span * 16), stream, ea, eb, 0, a);
-        FKV_HIP(hipGetLastError());
-      }
+  return zero_copy_launches(g.num_blocks, nl, g.kv, g.chunk / 16, group_vec, kWaves, grid_cap,
+                            limits, [&](const ZeroCopyPart& p) -> int {
+    const int lw = l0 + p.layer;
+    a.ids = reinterpret_cast<const int64_t*>(ids.dev) + (split ? 1 : 2) * static_cast<int64_t>(p.b);
+    a.ids_split = split;
+    a.inline_n = 0;
+    if (p.nb <= kInlineIdsZeroCopy && ids.host) {
+      a.inline_n = p.nb;
+      memcpy(a.inline_ids, ids.host + 2 * static_cast<int64_t>(p.b), sizeof(int64_t) * 2 * p.nb);
     }
-  return 0;
+    a.cpu_base = cpu_base + static_cast<int64_t>(lw) * g.cls + p.off * 16;
+    a.gpu_kv_stride = g.gks;
+    a.gpu_block_stride = g.gbs;
+    a.cpu_kv_stride = g.cks;
+    a.cpu_layer_stride = g.cls;
+    a.cpu_block_stride = g.cbs;
+    a.chunk = Divider(static_cast<uint32_t>(p.vec));
+    a.items = Divider(static_cast<uint32_t>(p.layers * g.kv));
+    a.kv_dim = static_cast<uint32_t>(g.kv);
+    a.num_vec = static_cast<uint32_t>(p.num_vec);
+    a.num_groups = static_cast<uint32_t>(p.groups);
+    a.groups_per_wg = static_cast<uint32_t>(p.groups_per_wg);
+    a.ptrs_per_layer = g.ptrs_per_layer;
+    for (int i = 0; i < p.layers * g.ptrs_per_layer; ++i)
+      a.layer_ptr[i] = reinterpret_cast<uint64_t>(g.layer_ptrs[lw * g.ptrs_per_layer + i]) +
+                       static_cast<uint64_t>(p.off) * 16;
+    hipEvent_t ea = nullptr, eb = nullptr;
+    int rc = prof.kernel_events(&ea, &eb);
+    if (rc) return rc;
+    prof.kernel_span(ea, eb, p.num_vec * 16);
+    if (!eb && p.last) eb = done;
+    (void)hipGetLastError();  // a stale error from elsewhere must not be blamed on this launch
+    hipExtLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(p.workgroups())), dim3(kThreads),
+                          static_cast<uint32_t>(p.run_blocks * 16), stream, ea, eb, 0, a);
+    FKV_HIP(hipGetLastError());
+    return 0;
+  });
 }
 
 // Pieces a call takes in kv_small_copy_kernel when it fits (at most

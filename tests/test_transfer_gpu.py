@@ -429,8 +429,8 @@ class ResidentCache:
     """A block-wise "host" cache in device memory beside a device cache
     [layer][kv][pool][chunk], both random."""
 
-    def __init__(self, dev, chunk, n, layers, kv, seed=0):
-        self.chunk, self.n, self.layers, self.kv, self.pool = chunk, n, layers, kv, n + 7
+    def __init__(self, dev, chunk, n, layers, kv, seed=0, spare=7):
+        self.chunk, self.n, self.layers, self.kv, self.pool = chunk, n, layers, kv, n + spare
         gen = torch.Generator(device=dev).manual_seed(seed + n)
         self.gpu = torch.randint(-2**62, 2**62, (layers, kv, self.pool, chunk // 8),
                                  dtype=torch.int64, device=dev, generator=gen)
@@ -473,6 +473,67 @@ def test_device_resident_kernel_edges(dev, monkeypatch, chunk, n, layers, kv, cu
     its rows meet chunk, block, group and launch ends, both ways."""
     monkeypatch.setenv("FLEXKV_SMALL_KERNEL", "0")
     ResidentCache(dev, chunk, n, layers, kv).check_both_ways(cus)
+
+
+@pytest.fixture
+def whole_card(dev):
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 230 << 30:
+        pytest.skip("needs 230 GiB of free device memory")
+    yield
+    torch.cuda.empty_cache()
+
+
+MIB, GIB = 1 << 20, 1 << 30
+
+
+@pytest.mark.parametrize("chunk,n,layers,kv", [
+    # blocks, layers and chunk parts beyond what a launch takes (32 GiB, 32 GiB
+    # a block row, 8 GiB of a chunk)
+    (MIB, 520, 32, 2), (7 * GIB + 48, 1, 5, 1), (8 * GIB + 4112, 2, 1, 1)],
+    ids=["blocks", "layers", "parts"])
+def test_zero_copy_beyond_one_launch(whole_card, dev, chunk, n, layers, kv):
+    """Zero-copy transfers of more than a launch's vectors are cut into
+    several, here over a cache in device memory."""
+    cache = ResidentCache(dev, chunk, n, layers, kv, spare=2 if n > 2 else 0)
+    pairs = list(zip(cache.gids.tolist(), cache.cids.tolist()))
+    cache.move(False)
+    for gid, cid in pairs:
+        for l in range(layers):
+            assert torch.equal(cache.host[cid, l], cache.gpu[l, :, gid]), (gid, cid, l)
+    cache.gpu.zero_()
+    cache.move(True)
+    for gid, cid in pairs:
+        for l in range(layers):
+            assert torch.equal(cache.gpu[l, :, gid], cache.host[cid, l]), (gid, cid, l)
+    for gid in set(range(cache.pool)) - {g for g, _ in pairs}:
+        assert not cache.gpu[:, :, gid].any(), gid
+
+
+@pytest.mark.parametrize("chunk,n,layers,kv", [
+    # whole blocks, one item at a time, parts of one chunk: 16 GiB a launch
+    (MIB, 270, 32, 2), (2 * GIB + 16, 2, 9, 1), (16 * GIB + 1040, 1, 1, 1), (5 * GIB, 1, 2, 2)],
+    ids=["blocks", "items", "parts", "items-kv"])
+def test_gather_scatter_beyond_one_launch(whole_card, dev, chunk, n, layers, kv):
+    """Gathers and scatters of more than 16 GiB are cut into several launches."""
+    from flexkv_amd import c_ext
+    cache = ResidentCache(dev, chunk, n, layers, kv, spare=1)
+    buf = cache.host[:n]
+
+    def same():
+        for i, gid in enumerate(cache.gids.tolist()):
+            for l in range(layers):
+                assert torch.equal(buf[i, l], cache.gpu[l, :, gid]), (i, gid, l)
+    args = (cache.gids, cache.ptrs, cache.pool * chunk, chunk, chunk, buf, kv == 1)
+    c_ext.gather_kv_blocks(*args)
+    same()
+    left = (set(range(cache.pool)) - set(cache.gids.tolist())).pop()
+    rest = cache.gpu[:, :, left].clone()
+    for i in range(n):
+        buf[i].bitwise_xor_(0x0F0F)
+    c_ext.scatter_kv_blocks(*args)
+    same()
+    assert torch.equal(cache.gpu[:, :, left], rest)
 
 
 @pytest.mark.parametrize("h2d", [False, True])
