@@ -128,12 +128,15 @@ struct DeviceState {
   std::vector<hsa_amd_sdma_engine_id_t> engines_duplex[2];
   // copy-engine transfers in flight per direction [D2H, H2D]
   std::atomic<int> busy[2] = {0, 0};
+  // synchronous zero-copy transfers into host memory in flight: host-to-device
+  // ones that start meanwhile take more workgroups (zero_copy_workgroups)
+  std::atomic<int> zero_copy_writes{0};
   CopyLane lane[2];                                    // [D2H, H2D]
 };
 
-// Counts a copy-engine transfer of one direction as in flight on a device
-// for its lifetime (DeviceState::busy), so the other direction's copies take
-// the duplex engine split meanwhile.
+// Counts a transfer of one direction as in flight on a device for its lifetime
+// (DeviceState::busy, so the other direction's engine copies take the duplex
+// engine split meanwhile; DeviceState::zero_copy_writes).
 struct BusyMark {
   std::atomic<int>& n;
   explicit BusyMark(std::atomic<int>& c) : n(c) { n.fetch_add(1, std::memory_order_relaxed); }

@@ -14,6 +14,20 @@ namespace fkv_detail {
 constexpr int kZeroCopyReaders = 14;    // host to device
 constexpr int kZeroCopyWriters = 32;    // device to host
 
+// Readers of a call that starts while a zero-copy transfer writes to host memory
+// on the same device.  Beside 32 writers 14 readers fall behind; 28, which alone
+// are 5% slower than 14, keep pace.  MI355X, GB/s of both directions with 14 / 28
+// readers (and in tiled kernels of 28 writers and 56 readers):
+//   begun together, 1-2 GiB each        81-84 / 85-91  (88)
+//   each direction call after call:
+//     4 MiB     65 / 71  (59)       64 MiB    73 / 77  (65)
+//     16 MiB    73 / 86  (64)       320 MiB   74 / 69  (67)
+//     32 MiB    73 / 88  (71)       1 GiB     74 / 69  (67)
+// Calls that began together run at 45 + 45 as long as they last; a long one that
+// begins in the middle of the other way's gets 33 + 33, or 25 + 48 with 14
+// readers.  48-56 writers and readers: 89-93 together, 69-71 from 320 MiB.
+constexpr int kZeroCopyReadersBeside = 28;
+
 // Compute units up to which a caller's number bounds the grid over host
 // memory; a larger one spreads it.  Eight (the workers' default) hold more
 // than the fastest counts of either direction.  All the workgroups of more are
@@ -26,17 +40,18 @@ constexpr int kZeroCopySpreadCus = 8;
 
 // Workgroups of a zero-copy transfer.  `transfer_cus`: compute units the
 // caller lets it occupy, <= 0 for no bound; `occupancy`: workgroups of the
-// kernel a compute unit holds.  A host cache in host memory takes the counts
-// above, or all that more than kZeroCopySpreadCus compute units hold when the
-// caller names them.  One in device memory has no link to wait for: it takes
-// every workgroup the compute units hold.
+// kernel a compute unit holds; `writing`: a zero-copy transfer to host memory is
+// in flight on the device.  A host cache in host memory takes the counts above,
+// or all that more than kZeroCopySpreadCus compute units hold when the caller
+// names them.  One in device memory has no link to wait for: it takes every
+// workgroup the compute units hold.
 inline int zero_copy_workgroups(bool h2d, bool host_memory, int transfer_cus, int num_cus,
-                                int occupancy) {
+                                int occupancy, bool writing) {
   const int cus = transfer_cus <= 0 ? num_cus : std::min(transfer_cus, num_cus);
   const int held = cus * occupancy;
-  return !host_memory || transfer_cus > kZeroCopySpreadCus
-             ? held
-             : std::min(h2d ? kZeroCopyReaders : kZeroCopyWriters, held);
+  if (!host_memory || transfer_cus > kZeroCopySpreadCus) return held;
+  const int readers = writing ? kZeroCopyReadersBeside : kZeroCopyReaders;
+  return std::min(h2d ? readers : kZeroCopyWriters, held);
 }
 
 // What one staging launch moves: blocks [b, b + nb) of the piece, items (layer,

@@ -32,6 +32,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <thread>
 #include <vector>
@@ -252,8 +253,8 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
 //   D2H 320 MiB      6083    5921    5954            6079    5967    5910
 // so 14 workgroups read (groups of 4 rows).  Writing (8 rows) 12 and 32 are as
 // fast alone, but beside a transfer the other way 12 starve: 2 GiB each way at
-// once moves 69 GB/s with 12, 82-84 with 24-32 and 80 with 48, so 32 write.  A
-// tiled kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
+// once moves 69 GB/s with 12 and 82-84 with 24-32, so 32 write; reading beside
+// them takes 28 (kZeroCopyReadersBeside).  A tiled kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
 // 1 MiB host-to-device call of one layer (here 33.5).
 //
 // kHost: the host cache lies in host memory.  One in device memory (!kHost) has
@@ -615,7 +616,15 @@ int64_t op_bytes(const Geometry& g) {
 // Workgroups of a zero-copy transfer of `g` on device `d`.
 int zero_copy_grid(const Geometry& g, const DeviceState& d, int transfer_cus, bool h2d) {
   const bool host = !g.cpu_info.device;
-  return zero_copy_workgroups(h2d, host, transfer_cus, d.num_cus, d.occ_zero_copy[h2d][host]);
+  return zero_copy_workgroups(h2d, host, transfer_cus, d.num_cus, d.occ_zero_copy[h2d][host],
+                              d.zero_copy_writes.load(std::memory_order_relaxed) > 0);
+}
+
+// Marks a synchronous zero-copy transfer of `g` that writes host memory as in
+// flight for the lifetime of `mark`.  Layer-wise handles are not marked: a
+// finished one may wait long for its release.
+void mark_zero_copy(std::optional<BusyMark>& mark, const Geometry& g, DeviceState& d, bool h2d) {
+  if (!h2d && !g.cpu_info.device) mark.emplace(d.zero_copy_writes);
 }
 
 // Shape of a staging launch, by its size.  Measured on MI355X, us a gather /
@@ -851,6 +860,8 @@ int transfer_zero_copy(const Geometry& g, hipStream_t stream, int dev, int trans
   IdLease ids;
   int rc = pack_ids(g, ids);
   if (rc) return rc;
+  std::optional<BusyMark> writing;
+  mark_zero_copy(writing, g, d, h2d);
   DrainOnError drain{stream};
   const int grid_cap = zero_copy_grid(g, d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff +
@@ -951,6 +962,8 @@ int transfer_zero_copy_noalloc(const Geometry& g, hipStream_t stream, int dev, i
     ids.dev = reinterpret_cast<char*>(sp);
     split = kScratchMaxBlocks;
   }
+  std::optional<BusyMark> writing;
+  mark_zero_copy(writing, g, d, h2d);
   DrainOnError drain{stream};
   const int grid_cap = zero_copy_grid(g, d, transfer_cus, h2d);
   char* cpu_dev = g.cpu_info.dev_ptr + g.startoff + static_cast<int64_t>(g.start_layer) * g.cls;

@@ -24,14 +24,14 @@ void device_memory_takes_the_chip() {
   for (int cus : {1, 32, 256})
     for (int occ : {1, 4, 8})
       for (bool h2d : {false, true}) {
-        all = all && zero_copy_workgroups(h2d, false, -1, cus, occ) == cus * occ;
-        all = all && zero_copy_workgroups(h2d, false, 0, cus, occ) == cus * occ;
+        all = all && zero_copy_workgroups(h2d, false, -1, cus, occ, occ == 4) == cus * occ;
+        all = all && zero_copy_workgroups(h2d, false, 0, cus, occ, occ == 4) == cus * occ;
         for (int bound : {1, 2, 8, 31, 256, 1000}) {
-          const int n = zero_copy_workgroups(h2d, false, bound, cus, occ);
+          const int n = zero_copy_workgroups(h2d, false, bound, cus, occ, occ == 4);
           bounded = bounded && n == (bound < cus ? bound : cus) * occ;
         }
         const int most = h2d ? 14 : 32;
-        const int n = zero_copy_workgroups(h2d, true, -1, cus, occ);
+        const int n = zero_copy_workgroups(h2d, true, -1, cus, occ, false);
         host = host && n == (most < cus * occ ? most : cus * occ);
       }
   check(all, "a host cache in device memory takes every workgroup the device holds");
@@ -159,11 +159,11 @@ void transfer_cus_bounds_and_spreads() {
     for (int occ : {4, 8}) {
       const int most = h2d ? 14 : 32;
       for (int cus = 1; cus <= 8; ++cus) {
-        const int n = zero_copy_workgroups(h2d, true, cus, 256, occ);
+        const int n = zero_copy_workgroups(h2d, true, cus, 256, occ, false);
         bounds = bounds && n == (most < cus * occ ? most : cus * occ);
       }
       for (int cus : {9, 32, 64, 256, 4096})
-        spreads = spreads && zero_copy_workgroups(h2d, true, cus, 256, occ) ==
+        spreads = spreads && zero_copy_workgroups(h2d, true, cus, 256, occ, false) ==
                                  (cus < 256 ? cus : 256) * occ;
     }
   check(bounds, "up to 8 compute units bound a transfer over the link");
@@ -183,9 +183,22 @@ void null_stream_waits_cover_what_they_wait_for() {
   check(alone, "one behind any other stream covers the groups of its own event");
 }
 
+void readers_keep_pace_with_writers() {
+  bool beside = true, writers = true;
+  for (int occ : {1, 4, 8})
+    for (int cus : {-1, 1, 2, 4, 8}) {
+      const int held = (cus < 0 ? 256 : cus) * occ;
+      beside = beside && zero_copy_workgroups(true, true, cus, 256, occ, true) == std::min(28, held);
+      writers = writers && zero_copy_workgroups(false, true, cus, 256, occ, true) == std::min(32, held);
+    }
+  check(beside, "readers that start beside writers are 28, within the caller's compute units");
+  check(writers, "writers are as many beside one another");
+}
+
 }  // namespace
 
 int main() {
+  readers_keep_pace_with_writers();
   null_stream_waits_cover_what_they_wait_for();
   device_memory_takes_the_chip();
   staging_launches_cover_the_piece();

@@ -21,4 +21,4 @@ def test_plans(tmp_path):
     assert build.returncode == 0, build.stderr
     res = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert res.returncode == 0 and "FAIL" not in res.stdout, res.stdout + res.stderr
-    assert res.stdout.count("ok:") == 18
+    assert res.stdout.count("ok:") == 20

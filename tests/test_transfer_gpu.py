@@ -669,6 +669,51 @@ def test_duplex_copy_engine_transfers(dev):
             assert np.array_equal(gpu[l][k][g_h], fresh[c_h, l, k][:, 0]), ("H2D", l, k)
 
 
+def test_duplex_zero_copy_transfers(dev):
+    """Zero-copy transfers of 32-128 MiB each way at once, from two threads on
+    streams with queues of their own, so that host-to-device calls start
+    alone and beside a device-to-host one (which gives them another grid).
+    Every byte matches."""
+    import threading
+    from gpu_util import DeviceCase, abi_transfer
+    from flexkv_amd import c_ext
+    case = KVCase(layers_total=8, num_layers=8, start_layer=0, kv=2, ng=600, nh=600, tokens=16,
+                  heads=8, dim=128).fill(seed=94)         # 32 KiB chunks
+    dc = DeviceCase(case)
+    g_all = inputs.distinct_ids(95, 512, 600)
+    c_all = inputs.distinct_ids(96, 512, 600)
+    fresh = case.host.copy()
+    fresh[c_all[256:]] ^= np.asarray(0x5A5A, dtype=case.dtype)
+    dc.set_host(fresh)
+    streams = [c_ext.transfer_stream() for _ in range(2)]
+    errors = []
+
+    def run(h2d):
+        try:
+            for n in (256, 64, 100, 256, 37):
+                ids = slice(256, 256 + n) if h2d else slice(0, n)
+                abi_transfer(dc, g_all[ids], c_all[ids], h2d=h2d, mode=0, stream=streams[h2d])
+        except Exception as e:   # surfaced below
+            errors.append(e)
+    try:
+        th = [threading.Thread(target=run, args=(h,)) for h in (False, True)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+    finally:
+        for st in streams:
+            c_ext.release_transfer_stream(st)
+    torch.cuda.synchronize()
+    assert not errors, errors
+    host, gpu = dc.host_np(), dc.gpu_np()
+    g_d, c_d, g_h, c_h = g_all[:256], c_all[:256], g_all[256:], c_all[256:]
+    for l in range(8):
+        for k in range(2):
+            assert np.array_equal(host[c_d, l, k][:, 0], case.gpu[l][k][g_d]), ("D2H", l, k)
+            assert np.array_equal(gpu[l][k][g_h], fresh[c_h, l, k][:, 0]), ("H2D", l, k)
+
+
 # Separate K and V allocations (fkv_transfer_kv_blocks_kv_ptrs): the same
 # bytes must move as with K and V halves of one allocation, so the oracle of
 # the combined layout is the expectation.  Geometry 7 (130 layers) needs three
