@@ -656,11 +656,13 @@ void launch_pack(PackArgs& pa, uint32_t num_cus, hipStream_t stream, hipEvent_t 
   pa.column_wgs = (grid + pa.columns.d - 1) / pa.columns.d;
   grid = pa.column_wgs * pa.columns.d;
   const unsigned lds = columns ? kPackColumnLds : 0;
+  // chunks of whole rows always fit groups of 8 rows or more
+  constexpr bool kWhole = kU > 1, kColumns = kH2D && kU == 32;
   const bool rows = pa.chunk.d % 64 == 0;
-  auto kernel = rows ? kv_pack_kernel<kH2D, kU, true, false> : kv_pack_kernel<kH2D, kU, false, false>;
+  auto kernel = rows ? kv_pack_kernel<kH2D, kU, kWhole, false> : kv_pack_kernel<kH2D, kU, false, false>;
   if (kH2D && columns)
-    kernel = rows ? kv_pack_kernel<kH2D, kU, true, kH2D && kU == 32>
-                  : kv_pack_kernel<kH2D, kU, false, kH2D && kU == 32>;
+    kernel = rows ? kv_pack_kernel<kH2D, kU, kWhole, kColumns>
+                  : kv_pack_kernel<kH2D, kU, false, kColumns>;
   hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, ea, eb, 0, pa);
 }
 
