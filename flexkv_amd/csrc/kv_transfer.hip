@@ -93,13 +93,14 @@ struct Divider {
 // launch's chunks in order, block -> layer -> K|V or layer -> K|V -> block.
 // Its 16-byte vectors are cut into groups of kU rows of 64 and wavefront w of
 // workgroup b moves group 4b + w (b in column order, launch_pack): no tile, no
-// LDS, no barrier, and every wavefront moves a full group.  Lane j first resolves the address of the
-// group's j-th chunk (a group touches at most 64, pack_fits), so ids and layer
-// pointers cost one round of loads a group whatever the chunk size; each row
-// then picks the chunk of each lane's vector out of those registers
-// (ds_bpermute), so rows that cross chunks (sizes that are not whole KiB, or
-// under one) leave no lane idle.  The scattered address is used in one of the
-// two walks only, so nothing but the loaded data is held between them.
+// LDS, no barrier, and every wavefront moves a full group.  Lane j first
+// resolves the address of the group's j-th chunk (a group touches at most 64,
+// pack_fits), so ids and layer pointers cost one round of loads a group
+// whatever the chunk size; each row then picks the chunk of each lane's vector
+// out of those registers (ds_bpermute), so rows that cross chunks (sizes that
+// are not whole KiB, or under one) leave no lane idle.  The scattered address
+// is used in one of the two walks only, so nothing but the loaded data is held
+// between them.
 //
 // HBM bounds the large launches and the launch the small ones.  Measured on
 // MI355X, us a gather / scatter call, against a kernel per chunk shape (tiled
@@ -254,14 +255,15 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
 // so 14 workgroups read (groups of 4 rows).  Writing (8 rows) 12 and 32 are as
 // fast alone, but beside a transfer the other way 12 starve: 2 GiB each way at
 // once moves 69 GB/s with 12 and 82-84 with 24-32, so 32 write; reading beside
-// them takes 28 (kZeroCopyReadersBeside).  A tiled kernel of 28-56 workgroups took 326 us for the 16 MiB and 36.0 us for a
-// 1 MiB host-to-device call of one layer (here 33.5).
+// them takes 28 (kZeroCopyReadersBeside).  A tiled kernel of 28-56 workgroups
+// took 326 us for the 16 MiB and 36.0 us for a 1 MiB host-to-device call of
+// one layer (here 33.5).
 //
 // kHost: the host cache lies in host memory.  One in device memory (!kHost) has
 // no link to wait for: loads in flight bound the launch, so it takes every
 // compute unit (zero_copy_workgroups), stores both ways with the non-temporal
 // hint alone, and finds a group's addresses once for the loads and again for
-// the stores, which leaves 44 registers and 8 wavefronts a SIMD (held through
+// the stores, which leaves 46 registers and 8 wavefronts a SIMD (held through
 // 8 rows: 80 and 6; the copy then takes a third longer within few compute
 // units).  Measured on MI355X, us a device-to-host / host-to-device call,
 // within the host cache's grid and stores -> now: 64 MiB of 32 KiB chunks
@@ -1546,28 +1548,46 @@ size_t layerwise_min_copy_bytes() {
 // kLayerwiseShortMinBlocks blocks (with fewer, a window's copies take no longer
 // than the host's round trip between windows).  A window takes one engine copy
 // per block, about 0.75 us each over eight engines however short, so windows
-// that grew from one layer group and shrank to one spent a layer-wise load of a
+// that grow from one layer group and shrink to one spend a layer-wise load of a
 // tensor-parallel shard (8 KiB a block and layer) on copies of 8-64 KiB.
-// Windows now hold at least this much of a block, or as many groups as gpw
-// allows, and the groups before the first of them move with the zero-copy
-// kernel, one event each.  Measured on MI355X, us with windows from one group /
-// 32 / 64 / 128 KiB a block (and on the link):
-//   Llama-3-8B, 256 blocks            11115  10819  10789  10527   (9419)
-//   Llama-3-70B TP-8, 3072 blocks     64381  50645  44956  41220  (35320)
-//     192 blocks                       4216   3381   3181   3224   (2208)
-//     80 blocks                        1904   1619   1611   1759    (920)
-//     8-bit, 1024 blocks              17677  10695   9123   8303   (5887)
-//   MLA, 16 tokens, 477 blocks        12874  11845  11059  10717   (9409)
-//   Llama-3-8B, 4 tokens, 1000        17232  14804  12952  11757   (9198)
+// Windows hold at least this much of a block, or as many groups as gpw allows
+// (the last window: the groups left), and the groups before the first of them
+// move with the zero-copy kernel, one event each.
+//
+// The last windows of short rows then hold many layers (16, 24, 16 and 9 of the
+// shard's 80, against 2, 1 and 1), whose compute starts only after the load.
+// That costs less than short copies do: measured on MI355X, us of the load
+// alone and of a prefill that overlaps it, its compute about as long as the
+// link's time (0.7-1.05 of it; 2.0 for 80 blocks), with windows from one group
+// / 64 / 128 KiB a block, 128 KiB shrinking to one group at the end, and 128
+// KiB with the last window's groups on the zero-copy kernel:
+//   load alone (on the link)           one     64    128  shrink  kernel
+//   Llama-3-8B, 256 blocks  (9419)   10750  10762  10463   10637   10299
+//   70B TP-8, 3072 blocks  (35320)   63214  44635  40550   53349   38935
+//     192 blocks            (2208)    4039   2982   2787    3597    2790
+//     80 blocks              (920)    1746   1336   1312    1595    1326
+//     8-bit, 1024 blocks    (5887)   17141   8598   7349   12924    6966
+//   MLA, 477 blocks         (9409)   12670  10961  10386   11770   10383
+//   Llama-3-8B, 4 tokens    (9198)   16811  12893  11577   14568   10586
+//   overlapped prefill
+//   Llama-3-8B, 256 blocks           12883  12941  12597   12563   12643
+//   70B TP-8, 3072 blocks            63663  50644  49583   54765   51071
+//     192 blocks                      4122   3251   3270    3672    3402
+//     80 blocks                       2370   2179   2209    2213    2252
+//     8-bit, 1024 blocks             17206   9359   9202   13017    9905
+//   MLA, 477 blocks                  13644  12823  12502   12573   12529
+//   Llama-3-8B, 4 tokens             17019  13179  12571   14954   12634
+// With compute of 0.4 of the link's time 128 KiB is within 3% of the best.
 constexpr size_t kLayerwiseShortCopyBytes = size_t(128) << 10;
 constexpr int kLayerwiseShortMinBlocks = 64;
 
 // Leading layer groups a copy-engine layer-wise handle moves with the
 // zero-copy kernel before its engines start (FLEXKV_LAYERWISE_CE_KERNEL_GROUPS,
 // default: the groups whose windows would be shorter than the shortest the
-// engines get, `window` groups; at most all groups but one).  A one-group window is bound by the engines' per-copy cost (one copy per block
-// of one group's rows), while a consumer waiting for the first group has
-// nothing else to run, so the kernel's compute units cost it little then.
+// engines get, `window` groups; at most all groups but one).  A one-group window
+// is bound by the engines' per-copy cost (one copy per block of one group's
+// rows), while a consumer waiting for the first group has nothing else to run, so
+// the kernel's compute units cost it little then.
 // Measured on MI355X at the Llama-3-8B shape with one layer per group, one
 // kernel group brings the first group in after 1.3 ms instead of 2.1 ms and
 // ends a prefill overlapped with 8 or 12 bf16 GEMMs per layer 1.1-1.7%
@@ -1626,12 +1646,12 @@ int layerwise_kernel_groups(fkv_transfer_handle_s* h, hipStream_t work, int firs
 }
 
 // The driver's work: the leading group(s) with the zero-copy kernel (see
-// layerwise_kernel_lead_groups), then the other layer groups in order, each
-// cut into pieces of whole blocks that fit a staging half; SDMA copies (one per block: the group's
-// rows are contiguous in block-wise host memory) on the wide engine set,
-// double-buffered; each piece's scatter on the pipeline stream after a
-// system-scope acquire; done[g] after the group's last piece.  The host
-// waits for a piece's scatter before reusing its half.
+// layerwise_kernel_lead_groups), then the other layer groups in order, in
+// windows cut into pieces of whole blocks that fit a staging half; SDMA copies
+// (one per block: the window's rows are contiguous in block-wise host memory) on
+// the wide engine set, double-buffered; each piece's scatter on the pipeline
+// stream after a system-scope acquire; done[g] after the last piece of its
+// window.  The host waits for a piece's scatter before reusing its half.
 int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
   DeviceState& d = g_dev[h->dev];
   const Geometry& g = h->geo;
@@ -1669,10 +1689,11 @@ int layerwise_ce_run(fkv_transfer_handle_s* h, CopyLane& ln, hipStream_t work) {
   // layerwise_min_copy_bytes() per block, which the engines move faster than
   // one-group copies.  Every group's event is recorded when the window
   // holding it has landed.  Windows grow from the shortest (1, 2, 4, ... groups
-  // where one group's rows are long enough), so the first group arrives early, and near the end hold at most half of the
-  // groups left, so the compute a window releases ends while the rest
-  // arrive: a consumer that keeps up waits for one group's compute after the
-  // last transfer, as with one group per window.
+  // where one group's rows are long enough), so the first group arrives early,
+  // and near the end hold at most half of the groups left, but no fewer than the
+  // shortest window: a consumer that keeps up has the last window's compute left
+  // after the last transfer, which is one group's where the shortest window is
+  // one group (see kLayerwiseShortCopyBytes for the others).
   const int lpl = g.layers_per_launch();
   const int ngroups = (g.num_layers + G - 1) / G;
   const size_t group_row = static_cast<size_t>(std::min(G, g.num_layers)) * g.kv * g.chunk;
@@ -1890,8 +1911,8 @@ Geometry make_geometry(int num_blocks, int start_layer_id, int num_layers,
 // (D2H / H2D) at the Llama-3-8B shape, 82% of the link, against 56.5 /
 // 57.2 GB/s for the zero-copy kernel.  Such transfers therefore move with
 // the zero-copy kernel, which holds compute units for the whole transfer
-// (bf16 GEMMs beside it take 1.05-2 times as long, by their order, and 1.02
-// times beside the rect copies); fkv_set_copy_engine_policy (or
+// (bf16 GEMMs beside it take 1.4 times as long in either order, and 1.02 times
+// beside the rect copies); fkv_set_copy_engine_policy (or
 // FLEXKV_CE_RECT_COPIES=1) keeps them on the engines.
 bool ce_pays_off(const Geometry& g, bool h2d) {
   // a "host" cache that is device memory has no PCIe copy to offload

@@ -91,11 +91,11 @@ enum {
  *
  * Arguments follow flexkv::transfer_kv_blocks (csrc/transfer.cu:63-70) one for
  * one; `transfer_cus` plays the role of `transfer_sms` (compute units the
- * zero-copy kernel may occupy; -1 = no bound).  Over host memory it runs at most
- * 14 workgroups host-to-device and 32 device-to-host, which fill the link, and
- * with more than 8 compute units named every workgroup those hold, a grid spread
- * over the chip.  When cpu_ptr is device memory it fills the compute units it may
- * occupy.
+ * zero-copy kernel may occupy; -1 = no bound).  Over host memory it runs at
+ * most 14 workgroups host-to-device (28 while a device-to-host one runs on the
+ * device) and 32 device-to-host, which fill the link, and with more than 8
+ * compute units named every workgroup those hold, a grid spread over the chip.
+ * When cpu_ptr is device memory it fills the compute units it may occupy.
  *
  * Host requirements (checked; violations return hipErrorInvalidValue):
  *   - gpu_block_ids, cpu_block_ids: host memory, num_blocks int64 each,
@@ -150,7 +150,7 @@ int fkv_transfer_kv_blocks_kv_ptrs(int num_blocks, int start_layer_id, int num_l
  * them (hipMemcpyAsync on `stream`) into a fixed 1 MiB device array compiled
  * into the library, one per GPU, held until the process ends.  At most 65536
  * blocks per call; more is refused with hipErrorInvalidValue.  Transfers of
- * up to 32 blocks carry their ids in the kernel arguments instead.  Calls on
+ * up to 96 blocks carry their ids in the kernel arguments instead.  Calls on
  * one GPU share that GPU's array: a call holds a per-GPU mutex from its copy
  * into the array until its kernels have finished, so concurrent calls from
  * several threads take turns.  Not for HIP graph capture: the call is
@@ -199,25 +199,30 @@ int fkv_scatter_kv_blocks(int num_blocks, int num_layers, const int64_t* gpu_blo
  * enqueued on `stream` before the call returns; fkv_handle_stream_wait makes
  * the other stream wait on the device, without a host round trip.
  * Small groups share launches of 1-4 MiB, and the event of the launch.
- * It runs at most 14 workgroups host-to-device and 32 device-to-host (enough
- * for the link; the rest of the chip stays with the compute the transfer
- * overlaps); transfer_cus bounds or raises that as in fkv_transfer_kv_blocks.
+ * It runs the workgroups of fkv_transfer_kv_blocks (few, but enough for the
+ * link; the rest of the chip stays with the compute the transfer overlaps), which
+ * transfer_cus bounds or raises as there.
  * use_ce_transfer = FKV_XFER_CE (host to device from block-wise host rows;
  * other transfers take the kernel): the copy engines, so the transfer holds
- * no compute unit while its bytes cross the link.  A library thread moves
- * windows of consecutive groups: one SDMA copy per block and window into
+ * no compute unit while the engines' bytes cross the link.  A library thread
+ * moves windows of consecutive groups: one SDMA copy per block and window into
  * double-buffered staging, then, once they have landed, the window's
  * scatter on a library stream with a hardware queue of its own, where the
  * events of the window's groups are recorded.  Windows grow 1, 2, 4, ...
- * groups up to FLEXKV_LAYERWISE_CE_MIN_COPY_BYTES per block (default
- * 256 KiB) and near the end hold at most half of the groups left, so the
- * first group arrives early and the compute a window releases ends while
- * the rest arrive.  Every window spreads its copies over the wide engine
- * set, FLEXKV_SDMA_ENGINES_WIDE engines (default 8, engines 0-7:
- * host-to-device copies on engines 8-15 slow compute kernels running beside
- * them about twofold).  FLEXKV_LAYERWISE_CE_KERNEL_GROUPS=n (default 0)
- * moves the first n groups with the zero-copy kernel before the engines
- * start, so the first group lands sooner.
+ * times the shortest, up to FLEXKV_LAYERWISE_CE_MIN_COPY_BYTES per block
+ * (default 256 KiB).  With fewer than 64 blocks, or where one group is 128 KiB
+ * of a block or more, the shortest window is one group; otherwise as many
+ * groups as make 128 KiB of a block (16 layers of a shard's 8 KiB), and the
+ * groups before the first window (15 of them) move with the zero-copy kernel,
+ * on its compute units, before the engines start.
+ * FLEXKV_LAYERWISE_CE_KERNEL_GROUPS=n sets another number of groups for it.
+ * Near the end a window holds at most half of the groups left but no fewer
+ * than the shortest window, so the first group arrives early and what a window
+ * releases is computed while the rest arrive; the last window's compute follows
+ * the load.  Every window spreads its copies over the wide engine set,
+ * FLEXKV_SDMA_ENGINES_WIDE engines (default 8, engines 0-7: host-to-device
+ * copies on engines 8-15 slow compute kernels running beside them about
+ * twofold).
  * fkv_handle_stream_wait and fkv_handle_wait first wait on the host until
  * the group's event exists (its copies have landed), fkv_handle_query
  * reports 0 until then.
