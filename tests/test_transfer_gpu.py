@@ -155,12 +155,10 @@ def test_geometries_match_oracle(dev, geo, mode):
                          ids=["kv-31.5MiB", "kv-32.5MiB", "mla-32.5MiB-odd", "mla-33MiB-odd",
                               "mla-65MiB-odd"])
 def test_zero_copy_variants_at_the_size_policy_edges(dev, kv, layers, n):
-    """Kernel-mode calls on either side of the sizes where the zero-copy
-    kernel changes variant: host-to-device calls take the whole-group kernel
-    from 32 MiB and the row-by-row one below, device-to-host calls the
-    whole-group kernel of two 4-row sub-groups (4 CUs from 64 MiB).  4 KiB
-    chunks; the MLA-shaped calls move an odd number of chunks (9 layers), so
-    a group's second sub-group can lie past the end of a launch."""
+    """Kernel-mode calls on either side of 32 MiB, from which copy-engine mode
+    hands transfers to the engines, and one of 65 MiB.  4 KiB chunks; the
+    MLA-shaped calls move an odd number of chunks (9 layers), so the last group
+    of rows is a part of one."""
     ng = max(1200, n + 200)
     case = KVCase(layers_total=layers, num_layers=layers, start_layer=0, kv=kv, ng=ng,
                   nh=ng + 100, tokens=16, heads=1, dim=128).fill(seed=kv * 1000 + n)
@@ -784,9 +782,8 @@ def test_zero_copy_cu_limits(dev, cus):
 @pytest.mark.parametrize("run", [1, 8, 64])
 def test_staged_runs_and_small_staging(dev, run, heads):
     """Copy-engine path with a tiny staging buffer: many pieces, run merging
-    across consecutive host ids, and a layer window split.  8 KiB chunks take
-    the general gather; 32 KiB chunks (8 heads, host layers 2..9 of 10) the
-    whole-group gather, with pieces that start past layer 0."""
+    across consecutive host ids, and a layer window split, with pieces that
+    start past layer 0 (host layers 2..9 of 10); 8 KiB and 32 KiB chunks."""
     from flexkv_amd import _lib
     _lib.set_staging_bytes(1 << 20)
     try:
@@ -918,12 +915,9 @@ def test_copy_engine_small_edge_cut_every_staging_order(dev, order, monkeypatch)
                                    (1, 1, 128, 8, 16), (1, 1, 256, 16, 16)],
                          ids=["65-rows-1x1", "65-rows-3x2", "32KiB-1x1", "128KiB-1x1"])
 def test_small_transfers_split_rows(dev, mode, shape):
-    """Transfers with fewer (block, layer) tiles than grid slots split each
-    tile's rows over several workgroups.  Chunks of 64 KiB + 16 B (65 rows,
-    the last a single vector) put range boundaries inside chunks and partial
-    rows at range ends; 32 KiB chunks split in the zero-copy kernels; 128 KiB
-    chunks (256 rows per tile) split in the staging kernels too, through the
-    whole-group gather in copy-engine mode."""
+    """Transfers of a few chunks split each chunk's rows over several
+    workgroups.  Chunks of 64 KiB + 16 B (65 rows, the last a single vector) put
+    the ends of groups inside chunks and partial rows at their ends."""
     n, nl, dim, heads, tokens = shape
     case = KVCase(layers_total=nl, num_layers=nl, start_layer=0, kv=2, ng=8, nh=12,
                   tokens=tokens, heads=heads, dim=dim).fill(seed=n * 10 + nl)
