@@ -259,17 +259,19 @@ __global__ __launch_bounds__(kThreads) void kv_pack_kernel(PackArgs a) {
 // took 326 us for the 16 MiB and 36.0 us for a 1 MiB host-to-device call of
 // one layer (here 33.5).
 //
+// Groups of 8 rows find their addresses once for the loads and again for the
+// stores, which leaves 46 registers and 8 wavefronts a SIMD.  Held through 8
+// rows they take 80-110 registers and leave 6 or 4: within one compute unit
+// 64 MiB device to host then take 1470 us instead of 1215.
+//
 // kHost: the host cache lies in host memory.  One in device memory (!kHost) has
 // no link to wait for: loads in flight bound the launch, so it takes every
-// compute unit (zero_copy_workgroups), stores both ways with the non-temporal
-// hint alone, and finds a group's addresses once for the loads and again for
-// the stores, which leaves 46 registers and 8 wavefronts a SIMD (held through
-// 8 rows: 80 and 6; the copy then takes a third longer within few compute
-// units).  Measured on MI355X, us a device-to-host / host-to-device call,
-// within the host cache's grid and stores -> now: 64 MiB of 32 KiB chunks
-// 152 / 341 -> 38.3 / 38.5, 1 GiB 2208 / 5238 -> 433 / 435, 47 MiB of 2 KiB
-// chunks 118 / 258 -> 33.5 / 33.8; within 8 compute units 64 MiB 73.3 / 72.2,
-// 1 GiB 976 / 950.  12 and 16 rows: 1 GiB 440 / 445 and 440 / 440.
+// compute unit (zero_copy_workgroups), and stores both ways with the
+// non-temporal hint alone.  Measured on MI355X, us a device-to-host /
+// host-to-device call, within the host cache's grid and stores -> now: 64 MiB of
+// 32 KiB chunks 152 / 341 -> 38.3 / 38.5, 1 GiB 2208 / 5238 -> 433 / 435, 47 MiB
+// of 2 KiB chunks 118 / 258 -> 33.5 / 33.8; within 8 compute units 64 MiB 73.3 /
+// 72.2, 1 GiB 976 / 950.  12 and 16 rows: 1 GiB 440 / 445 and 440 / 440.
 template <bool kH2D, bool kHost>
 constexpr int zero_copy_rows() { return kHost && kH2D ? 4 : 8; }
 constexpr int kMaxItems = 2 * kMaxLayersPerLaunch;   // (layer, K|V) pairs of a launch
@@ -355,22 +357,15 @@ __global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) 
       *cpu = a.cpu_base + s_item[2 * item + 1] + s_block[2 * (b - b0) + 1] + off;
     };
     u32x4 v[kU];
-    if constexpr (kHost) {
+    if constexpr (kHost && kH2D) {
       char *gpu[kU], *cpu[kU];
 #pragma unroll
       for (int u = 0; u < kU; ++u) locate(u, &gpu[u], &cpu[u]);
 #pragma unroll
-      for (int u = 0; u < kU; ++u)
-        v[u] = __builtin_nontemporal_load((const gvec*)(kH2D ? cpu[u] : gpu[u]));
+      for (int u = 0; u < kU; ++u) v[u] = __builtin_nontemporal_load((const gvec*)cpu[u]);
 #pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        if (v0 + u * 64 < a.num_vec) {
-          if (kH2D)
-            __builtin_nontemporal_store(v[u], (gvec*)gpu[u]);
-          else
-            store_system(cpu[u], v[u]);
-        }
-      }
+      for (int u = 0; u < kU; ++u)
+        if (v0 + u * 64 < a.num_vec) __builtin_nontemporal_store(v[u], (gvec*)gpu[u]);
     } else {
       char *gpu, *cpu;
 #pragma unroll
@@ -382,8 +377,12 @@ __global__ __launch_bounds__(kThreads) void kv_zero_copy_kernel(ZeroCopyArgs a) 
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
         locate(u, &gpu, &cpu);
-        if (v0 + u * 64 < a.num_vec)
-          __builtin_nontemporal_store(v[u], (gvec*)(kH2D ? gpu : cpu));
+        if (v0 + u * 64 < a.num_vec) {
+          if (kHost)
+            store_system(cpu, v[u]);
+          else
+            __builtin_nontemporal_store(v[u], (gvec*)(kH2D ? gpu : cpu));
+        }
       }
     }
   }
