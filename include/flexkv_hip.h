@@ -174,8 +174,9 @@ int fkv_transfer_kv_blocks_noalloc(int num_blocks, int start_layer_id, int num_l
  * the id list at byte offset i * num_layers * kv * chunk).  This is the
  * on-device half of FKV_XFER_CE exposed on its own, for callers that move the
  * packed blocks themselves (RDMA, file I/O, peer GPUs).  The buffer may be
- * device or pinned host memory; buffer_bytes must cover every block.  Same
- * checks and synchronous return as fkv_transfer_kv_blocks.  No counterpart in
+ * device memory (every compute unit takes part) or pinned host memory (the
+ * zero-copy kernel's few, which fill the link); buffer_bytes must cover every
+ * block.  Same checks and synchronous return as fkv_transfer_kv_blocks.  No counterpart in
  * the reference, which only ever copies between the two caches. */
 int fkv_gather_kv_blocks(int num_blocks, int num_layers, const int64_t* gpu_block_ids,
                          void* const* gpu_layer_ptrs, int64_t gpu_kv_stride_bytes,

@@ -1311,6 +1311,27 @@ def test_gather_scatter_match_oracle(dev, geo, buffer_on_host):
 from hypothesis import HealthCheck, given, settings, strategies as st  # noqa: E402
 
 
+@pytest.mark.parametrize("chunk,n,layers,kv", [
+    (16, 1, 1, 1), (496, 300, 4, 2), (1024, 40, 130, 2), (528, 97, 40, 2), (32768, 130, 8, 2),
+    (73728, 9, 61, 1)])
+def test_gather_scatter_host_buffers(dev, chunk, n, layers, kv):
+    """Gathers into and scatters from pinned host memory, over chunk sizes,
+    ids in the kernel arguments or not, and layers beyond one launch's."""
+    from flexkv_amd import c_ext
+    from flexkv_amd.storage.allocator import pinned_empty
+    cache = ResidentCache(dev, chunk, n, layers, kv)
+    buf = pinned_empty(n * layers * kv * chunk // 8, torch.int64).view(n, layers, kv, chunk // 8)
+    buf.zero_()
+    args = (cache.gids, cache.ptrs, cache.pool * chunk, chunk, chunk, buf, kv == 1)
+    c_ext.gather_kv_blocks(*args)
+    assert torch.equal(buf, cache.gpu[:, :, cache.gids].permute(2, 0, 1, 3).cpu())
+    buf.bitwise_xor_(0x0F0F)
+    want = cache.gpu.clone()
+    want[:, :, cache.gids] = buf.to(dev).permute(1, 2, 0, 3)
+    c_ext.scatter_kv_blocks(*args)
+    assert torch.equal(cache.gpu, want)
+
+
 def _run_ids(g, n, universe, run):
     """n distinct ids in runs of `run` consecutive ids (the last run may be
     shorter), runs at random non-overlapping starts."""
